@@ -148,6 +148,59 @@ def test_dlinoss_complex128_vs_fp64_oracle(K, variant, shape):
     no_device_errors()
 
 
+# chunk counts of the complex128 scans: sqrt(L) chunks, capped by 2048 waves of 64
+# channels: one chunk (L < 4; 1025 groups or more), two steps per chunk, a short
+# last chunk, channels ending inside a wave
+@pytest.mark.parametrize("shape", [(3, 1, 2), (4, 1, 1), (5, 2, 32), (17, 3, 43), (250, 1, 1),
+                                   (16, 1, 65600), (9, 5, 13200)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_complex128_scans_chunk_edges(K, shape):
+    """complex128 D-LinOSS and LinOSS at the edges of the chunk plan, against the
+    fp64 oracle (both sides sum in double, in other orders); a second call gives
+    the same bits (no sum depends on timing)."""
+    L, B, P = shape
+    rng = np.random.default_rng(L + P)
+    a, g, dt, bu, go = dlinoss_inputs(L, B, P, seed=L + B + P, variant="imex2")
+    a, g, dt = (x.astype(np.float64) for x in (a, g, dt))
+    bu, go = bu.astype(np.complex128) + 1e-3 * rng.normal(size=bu.shape), go.astype(np.complex128)
+    announce(f"complex128 chunk edges L={L} B={B} P={P}")
+    st = _fwd(K, "imex2", a, g, dt, bu)
+    grads = _bwd(K, "imex2", a, g, dt, bu, st, go)
+    ref = oracle.dlinoss_forward("imex2", a, g, dt, bu)
+    np.testing.assert_allclose(to_np(st), ref, rtol=1e-10, atol=1e-12)
+    for got, r in zip(grads, oracle.dlinoss_backward("imex2", a, g, dt, bu, ref, go)):
+        np.testing.assert_allclose(to_np(got), r, rtol=1e-10, atol=1e-12 * max(1.0, float(np.abs(r).max())))
+    again = _bwd(K, "imex2", a, g, dt, bu, st, go)
+    assert all(np.array_equal(to_np(x), to_np(y)) for x, y in zip(grads, again))
+    ms, b, go2 = _linoss_inputs(L, B, P, seed=L + P)
+    ms = [to_dev(m.astype(np.complex128)) for m in ms]
+    b, go2 = b.astype(np.complex128), go2.astype(np.complex128)
+    st = K.linoss_scan(*ms, to_dev(b))
+    ref = oracle.linoss_forward(*[to_np(m) for m in ms], b)
+    np.testing.assert_allclose(to_np(st), ref, rtol=1e-10, atol=1e-12 * max(1.0, float(np.abs(ref).max())))
+    for got, r in zip(K.linoss_scan_backward(*ms, st, to_dev(go2)),
+                      oracle.linoss_backward(*[to_np(m) for m in ms], ref, go2)):
+        np.testing.assert_allclose(to_np(got), r, rtol=1e-10, atol=1e-12 * max(1.0, float(np.abs(r).max())))
+
+
+def test_complex128_forward_captured_without_workspace(K):
+    """The complex128 forward allocated nothing before it was chunked, so a
+    capture on a fresh stream, whose workspace may not grow, still goes
+    through (as one chunk) and replays to the eager result."""
+    a, g, dt, bu, _ = dlinoss_inputs(300, 2, 40, seed=7)
+    args = [to_dev(x.astype(np.float64)) for x in (a, g, dt)] + [to_dev(bu.astype(np.complex128))]
+    eager = to_np(K.dlinoss_im_forward(*args))
+    torch.cuda.synchronize()
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    announce("complex128 capture without workspace")
+    with torch.cuda.graph(graph, stream=side):
+        st = K.dlinoss_im_forward(*args)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        np.testing.assert_allclose(to_np(st), eager, rtol=1e-10, atol=1e-12)
+
+
 def test_dlinoss_complex128_dtype_rules(K):
     """The reference's data_ptr<value_t> rules: complex128 bu needs float64
     coefficients and complex128 states / grad_output; other bu types are not

@@ -257,6 +257,24 @@ def test_sdlinoss_complex128_vs_oracle(K, variant, tag):
         assert_close(got, ref, RTOL64, ATOL64 * max(1.0, float(np.abs(ref).max())), f"c128 {name}")
 
 
+@pytest.mark.parametrize("tag", ["full", "bcast_t", "bcast_b", "m", "lm", "bm"])
+@pytest.mark.parametrize("shape", [(3, 2, 5), (4, 1, 1), (17, 3, 43), (90, 2, 65)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_sdlinoss_complex128_chunk_edges(K, shape, tag):
+    """One chunk, two steps per chunk, a short last chunk (sqrt(L) chunks), in
+    every parameter layout: time sums are added over the chunks."""
+    L, B, M = shape
+    A, G, S, bu, go = _to64(sdl_inputs("im", tag, L, B, M, seed=L + len(tag)))
+    announce(f"sdlinoss c128 chunk edges {tag} L={L} B={B} M={M}")
+    args = [to_dev(x) for x in (A, G, S, bu)]
+    st = K.sdlinoss_im_forward(*args)
+    ref_st = oracle.sdlinoss_forward("im", A, G, S, bu)
+    assert_close(to_np(st), ref_st, RTOL64, ATOL64 * max(1.0, float(np.abs(ref_st).max())), "states")
+    grads = K.sdlinoss_im_backward(*args, st, to_dev(go))
+    for got, ref, name in zip(grads, oracle.sdlinoss_backward("im", A, G, S, bu, ref_st, go), NAMES):
+        assert_close(to_np(got), ref, RTOL64, ATOL64 * max(1.0, float(np.abs(ref).max())), name)
+
+
 def test_sdlinoss_complex128_golden_and_edges(K):
     """The reference kernel vectors in fp64 (bound set by their fp32
     arithmetic), one-step and single-channel shapes, and empty inputs."""
