@@ -486,6 +486,22 @@ int ossm_mamba_conv_backward(const float* x, int64_t ld_x, const float* weight, 
                              float* grad_bias, int64_t batch, int64_t length, int64_t dim,
                              int64_t width, ossm_stream_t stream);
 
+/*
+ * The oscillator parameters of a layer from their stored form, out [3][ssm] =
+ * a, g, dt.  damped != 0: the D-LinOSS layer's stability projection
+ * (dlinoss.py:249-264: dt = sigmoid(steps), g = relu(G_diag), a clamped to its
+ * band); 0: the LinOSS layer's (linoss.py:209-215: a = relu(A_diag), g = 0; G_diag
+ * is not read).  Formed in double and rounded once.
+ */
+int ossm_layer_params_forward(int damped, const float* A_diag, const float* G_diag, const float* steps,
+                              float* out, int64_t ssm, ossm_stream_t stream);
+
+/* Gradients grad [3][ssm] of A_diag, G_diag (written only when damped) and steps
+ * from those of a, g and dt (each may be null: zero). */
+int ossm_layer_params_backward(int damped, const float* A_diag, const float* G_diag, const float* steps,
+                               const float* grad_a, const float* grad_g, const float* grad_dt,
+                               float* grad, int64_t ssm, ossm_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -35,7 +35,7 @@ from . import _lib
 from .bridge import run_dlinoss
 
 __all__ = ["DampedLinOSSLayer", "dlinoss_layer_forward", "dlinoss_layer_backward", "DlinossLayerFn",
-           "project_parameters", "unfused_layer_forward"]
+           "project_parameters", "unfused_layer_forward", "LayerParamsFn", "fused_layer_supported"]
 
 _VARIANTS = {"imex1": 0, "imex2": 1, "im": 2, "ex": 3}
 _LAYER_MAX = 256  # largest hidden_dim / ssm_size of the fused kernel
@@ -65,6 +65,58 @@ def project_parameters(A_diag: Tensor, G_diag: Tensor, steps: Tensor) -> Tuple[T
     hi = (2.0 + dg + 2.0 * root) / dt2
     a = lo + torch.relu(A_diag - lo) - torch.relu(A_diag - hi)
     return a, g, dt
+
+
+class LayerParamsFn(torch.autograd.Function):
+    """(a, g, dt) of a layer from its stored float32 GPU parameters, one launch
+    each way: ``project_parameters`` when ``damped``, else the LinOSS layer's
+    ``(relu(A), 0, sigmoid(steps))`` (G_diag is then None)."""
+
+    @staticmethod
+    def forward(ctx, damped: bool, A_diag: Tensor, G_diag: Optional[Tensor],
+                steps: Tensor) -> Tuple[Tensor, Tensor, Tensor]:  # type: ignore[override]
+        A, G, s = (None if t is None else t.contiguous() for t in (A_diag, G_diag, steps))
+        out = torch.empty((3, A.numel()), dtype=torch.float32, device=A.device)
+        with torch.cuda.device(A.device):
+            _lib.check(_lib.load().ossm_layer_params_forward(
+                int(damped), A.data_ptr(), _lib.ptr(G), s.data_ptr(), out.data_ptr(), A.numel(),
+                _lib.stream_of(A)))
+        ctx.damped = damped
+        ctx.set_materialize_grads(False)
+        ctx.save_for_backward(A_diag, G_diag, steps)
+        return out[0], out[1], out[2]
+
+    @staticmethod
+    def backward(ctx, *grads: Optional[Tensor]):  # type: ignore[override]
+        params = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            # create_graph: differentiable again, as torch operations
+            A, G, s = params
+            outs = project_parameters(A, G, s) if ctx.damped else \
+                (torch.relu(A), None, torch.sigmoid(s))
+            pairs = [(o, g) for o, g in zip(outs, grads) if o is not None and g is not None]
+            wanted = [t for t, n in zip(params, ctx.needs_input_grad[1:]) if n]
+            got = iter(torch.autograd.grad([o for o, _ in pairs], wanted, [g for _, g in pairs],
+                                           create_graph=True, allow_unused=True) if pairs else
+                       [None] * len(wanted))
+            return (None, *[next(got) if n else None for n in ctx.needs_input_grad[1:]])
+        A, G, s = (None if t is None else t.contiguous() for t in params)
+        up = [None if g is None else g.contiguous() for g in grads]
+        out = torch.empty((3, A.numel()), dtype=torch.float32, device=A.device)
+        with torch.cuda.device(A.device):
+            _lib.check(_lib.load().ossm_layer_params_backward(
+                int(ctx.damped), A.data_ptr(), _lib.ptr(G), s.data_ptr(), *[_lib.ptr(g) for g in up],
+                out.data_ptr(), A.numel(), _lib.stream_of(A)))
+        return (None, *[out[i] if n else None for i, n in enumerate(ctx.needs_input_grad[1:])])
+
+
+def fused_layer_supported(inputs: Tensor, params, hidden: int, ssm: int) -> bool:
+    """Whether a layer of this size runs as the fused kernel on ``inputs`` as it is:
+    float32 throughout on one GPU, no autocast, nothing empty."""
+    return (inputs.is_cuda and inputs.dtype == torch.float32 and inputs.numel() > 0
+            and 0 < hidden <= _LAYER_MAX and 0 < ssm <= _LAYER_MAX
+            and all(t.dtype == torch.float32 and t.device == inputs.device for t in params)
+            and not torch.is_autocast_enabled("cuda"))
 
 
 def _check_layer_args(inputs: Tensor, B: Tensor, C: Tensor, D: Tensor, a: Tensor, g: Tensor,
@@ -339,10 +391,11 @@ class DampedLinOSSLayer(nn.Module):
         u = inputs.to(compute)
         params = [t.to(device=u.device, dtype=compute) for t in
                   (self.A_diag, self.G_diag, self.steps, self.B, self.C, self.D)]
-        a, g, dt = project_parameters(*params[:3])
         Bw, Cw, Dw = params[3:]
         if u.is_cuda and self.hidden_dim <= _LAYER_MAX and self.ssm_size <= _LAYER_MAX:
+            a, g, dt = LayerParamsFn.apply(True, *params[:3])
             y = DlinossLayerFn.apply(self.variant, u, Bw, Cw, Dw, a, g, dt)
         else:
+            a, g, dt = project_parameters(*params[:3])
             y = unfused_layer_forward(self.variant, u, Bw, Cw, Dw, a, g, dt)
         return y if dtype == compute else y.to(dtype)

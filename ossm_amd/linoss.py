@@ -11,7 +11,10 @@ The recurrence ``s_t = M s_{t-1} + b_t`` runs through
 is the native ``linoss_scan_backward``, where the reference runs a Python
 loop of about twenty torch operations per time step (linoss.py:83-151).
 The layer glue around it (parameter maps, the B and C projections, the D
-skip) is the reference's arithmetic in torch operations.
+skip) is the reference's arithmetic in torch operations.  Float32 layers of
+up to 256 channels on a GPU run whole as the fused D-LinOSS layer kernels
+instead: with damping g = 0 the IM transition below is D-LinOSS im's and the
+IMEX one imex2's.
 
 Transition per discretisation (a = relu(A_diag), dt = sigmoid(steps)):
   IM   (linoss.py:244-251): schur = 1 / (1 + dt^2 a),
@@ -29,6 +32,7 @@ import torch
 from torch import Tensor, nn
 
 from .bridge import run_associative_scan
+from .layers import DlinossLayerFn, LayerParamsFn, fused_layer_supported
 
 __all__ = ["LinOSSLayer", "linoss_transition"]
 
@@ -80,6 +84,12 @@ class LinOSSLayer(nn.Module):
             raise ValueError(f"Expected hidden_dim={self.hidden_dim}, received {hidden}.")
         dtype, device = inputs.dtype, inputs.device
         cast = lambda t: t.to(device=device, dtype=dtype)  # noqa: E731
+        if fused_layer_supported(inputs, (self.A_diag, self.B, self.C, self.D, self.steps), hidden,
+                                 self.ssm_size):
+            # IM and IMEX are the undamped (g = 0) D-LinOSS im and imex2 recurrences
+            a, g, dt = LayerParamsFn.apply(False, self.A_diag, None, self.steps)
+            return DlinossLayerFn.apply("im" if self.discretization == "IM" else "imex2", inputs,
+                                        self.B, self.C, self.D, a, g, dt)
         a_diag = cast(torch.relu(self.A_diag))
         step = cast(torch.sigmoid(self.steps))
         flat = inputs.reshape(batch * length, hidden)
