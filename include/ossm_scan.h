@@ -487,11 +487,11 @@ int ossm_mamba_conv_backward(const float* x, int64_t ld_x, const float* weight, 
                              int64_t width, ossm_stream_t stream);
 
 /*
- * The oscillator parameters of a layer from their stored form, out [3][ssm] =
- * a, g, dt.  damped != 0: the D-LinOSS layer's stability projection
+ * The oscillator parameters of a layer from their stored form, out [6][ssm] =
+ * a, g, dt and (not damped) what the rounding of each to float32 left.  damped != 0: the D-LinOSS layer's stability projection
  * (dlinoss.py:249-264: dt = sigmoid(steps), g = relu(G_diag), a clamped to its
  * band); 0: the LinOSS layer's (linoss.py:209-215: a = relu(A_diag), g = 0; G_diag
- * is not read).  Formed in double and rounded once.
+ * is not read), formed in double.
  */
 int ossm_layer_params_forward(int damped, const float* A_diag, const float* G_diag, const float* steps,
                               float* out, int64_t ssm, ossm_stream_t stream);
@@ -501,6 +501,35 @@ int ossm_layer_params_forward(int damped, const float* A_diag, const float* G_di
 int ossm_layer_params_backward(int damped, const float* A_diag, const float* G_diag, const float* steps,
                                const float* grad_a, const float* grad_g, const float* grad_dt,
                                float* grad, int64_t ssm, ossm_stream_t stream);
+
+/*
+ * ossm_dlinoss_layer_forward / _backward with params_lo [3][ssm] (may be null): what
+ * a_diag, g_diag and step leave of their double values.  With it the oscillators'
+ * coefficients are formed from the sums in double and rounded once.
+ */
+int ossm_dlinoss_layer_forward_wide(int variant, const float* inputs, const float* B, const float* C,
+                                    const float* D, const float* a_diag, const float* g_diag,
+                                    const float* step, const float* params_lo, float* outputs,
+                                    void* carries, int64_t batch, int64_t length, int64_t hidden,
+                                    int64_t ssm, ossm_stream_t stream);
+int ossm_dlinoss_layer_backward_wide(int variant, const float* inputs, const float* grad_output,
+                                     const float* B, const float* C, const float* D,
+                                     const float* a_diag, const float* g_diag, const float* step,
+                                     const float* params_lo, const void* carries, float* grad_inputs,
+                                     void* grad_bu, void* x_conj, float* grad_a, float* grad_g,
+                                     float* grad_step, int64_t batch, int64_t length, int64_t hidden,
+                                     int64_t ssm, ossm_stream_t stream);
+
+/*
+ * out(i, j) = sum_r a[r, i] b[r, j] over row-major a [rows, m] (row stride ld_a) and
+ * b [rows, n] (ld_b): a layer's weight gradient from its upstream gradient and
+ * input.  Element (i, j) is written at out[(i / 2) out_pair_stride + (i % 2)
+ * out_odd_stride + j out_col_stride].  float32 precision on the bf16 matrix cores
+ * (each operand split into three terms); summed in a fixed order.  rows >= 16.
+ */
+int ossm_rows_product(const float* a, int64_t ld_a, const float* b, int64_t ld_b, float* out,
+                      int64_t out_pair_stride, int64_t out_odd_stride, int64_t out_col_stride,
+                      int64_t rows, int64_t m, int64_t n, ossm_stream_t stream);
 
 #ifdef __cplusplus
 }

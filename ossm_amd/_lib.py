@@ -105,6 +105,14 @@ _SIGNATURES = {
         ctypes.c_int,
         [ctypes.c_int, _fp, _fp, _fp, _fp, _fp, _fp, _fp, _fp, _vp, _fp, _vp, _vp, _fp, _fp, _fp,
          _c_int64, _c_int64, _c_int64, _c_int64, _vp]),
+    "ossm_dlinoss_layer_forward_wide": (
+        ctypes.c_int,
+        [ctypes.c_int, _fp, _fp, _fp, _fp, _fp, _fp, _fp, _fp, _fp, _vp, _c_int64, _c_int64, _c_int64,
+         _c_int64, _vp]),
+    "ossm_dlinoss_layer_backward_wide": (
+        ctypes.c_int,
+        [ctypes.c_int, _fp, _fp, _fp, _fp, _fp, _fp, _fp, _fp, _fp, _vp, _fp, _vp, _vp, _fp, _fp, _fp,
+         _c_int64, _c_int64, _c_int64, _c_int64, _vp]),
     "ossm_selective_mamba_forward": (
         ctypes.c_int,
         [_fp, _c_int64, _fp, _c_int64, _fp, _fp, _fp, _fp, _c_int64, _fp, _c_int64, _fp, _fp, _fp,
@@ -122,6 +130,9 @@ _SIGNATURES = {
         ctypes.c_int, [ctypes.c_int, _fp, _fp, _fp, _fp, _c_int64, _vp]),
     "ossm_layer_params_backward": (
         ctypes.c_int, [ctypes.c_int, _fp, _fp, _fp, _fp, _fp, _fp, _fp, _c_int64, _vp]),
+    "ossm_rows_product": (
+        ctypes.c_int,
+        [_fp, _c_int64, _fp, _c_int64, _fp, _c_int64, _c_int64, _c_int64, _c_int64, _c_int64, _c_int64, _vp]),
     "ossm_mamba_conv_forward": (
         ctypes.c_int, [_fp, _c_int64, _fp, _fp, _fp, _c_int64, _c_int64, _c_int64, _c_int64, _vp]),
     "ossm_mamba_conv_backward": (

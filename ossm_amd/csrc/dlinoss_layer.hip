@@ -87,10 +87,20 @@ struct LayerArgs {
   const float* a;
   const float* g;
   const float* dt;
+  const float* lo;  // [3, P]: what a, g, dt leave of their double values; may be null
   float* y;         // [B, L, H]
   float4* carries;  // [B, n_chunks, P]: state entering each chunk (for the backward); may be null
   int Bsz, L, H, P, n_chunks;
 };
+
+// Oscillator p's coefficients; with lo, from its parameters in double.
+template <int V, class Args>
+__device__ __forceinline__ DlCoef layer_coef(const Args& A, int p) {
+  const float a = A.a[p], g = A.g[p], dt = A.dt[p];
+  if (A.lo == nullptr) return Dlinoss<V>::coef_of({a, g, dt});
+  return Dlinoss<V>::coef_wide(static_cast<double>(a) + A.lo[p], static_cast<double>(g) + A.lo[A.P + p],
+                               static_cast<double>(dt) + A.lo[2 * A.P + p]);
+}
 
 // Row m of the accumulator register r (see the layout above).
 __device__ __forceinline__ int acc_row(int r, int lane) {
@@ -309,7 +319,7 @@ void dlinoss_layer_fwd_kernel(
   const int ch = b * A.P + p;
   const bool scan = A.n_chunks > 1;
   typename Model::Coef k{};
-  if (osc) k = Model::coef_of({A.a[p], A.g[p], A.dt[p]});
+  if (osc) k = layer_coef<V>(A, p);
   // All 32 steps run: rows past L hold zeros (zero u rows), which only the
   // last chunk has; its aggregate is never read and its rows past L never stored.
   const float2* bu_col = reinterpret_cast<const float2*>(sX) + p;
@@ -437,6 +447,7 @@ struct LayerBwdArgs {
   const float* a;
   const float* g;
   const float* dt;
+  const float* lo;       // as LayerArgs::lo
   const float4* carries; // [B, n_chunks, P] from the forward
   float* grad_u;         // [B, L, H]
   float2* grad_bu;       // [B, L, P] (re, im)
@@ -647,7 +658,7 @@ __global__ __launch_bounds__(kLayerThreads) void dlinoss_layer_bwd_kernel(
   float4 sp[kLc];  // state before step t of the chunk
   float4 e = f4zero();
   if (osc) {
-    k = Model::coef_of({A.a[p], A.g[p], A.dt[p]});
+    k = layer_coef<V>(A, p);
     float4 s = carry_in;
 #pragma unroll
     for (int t = 0; t < kLc; ++t) {
@@ -854,11 +865,11 @@ using namespace ossm;
 
 extern "C" {
 
-int ossm_dlinoss_layer_forward(int variant, const float* inputs, const float* B, const float* C,
-                               const float* D, const float* a_diag, const float* g_diag,
-                               const float* step, float* outputs, void* carries, int64_t batch,
-                               int64_t length, int64_t hidden, int64_t ssm,
-                               ossm_stream_t stream_v) {
+int ossm_dlinoss_layer_forward_wide(int variant, const float* inputs, const float* B, const float* C,
+                                    const float* D, const float* a_diag, const float* g_diag,
+                                    const float* step, const float* params_lo, float* outputs,
+                                    void* carries, int64_t batch, int64_t length, int64_t hidden,
+                                    int64_t ssm, ossm_stream_t stream_v) {
   clear_error();
   const char* what = "dlinoss_layer_forward";
   if (batch < 0 || length < 0 || hidden < 0 || ssm < 0)
@@ -876,7 +887,7 @@ int ossm_dlinoss_layer_forward(int variant, const float* inputs, const float* B,
     return set_error(OSSM_ERR_UNSUPPORTED, std::string(what) + ": size exceeds 32-bit indexing");
   if (!inputs || !D || !outputs || (ssm > 0 && (!B || !C || !a_diag || !g_diag || !step)))
     return set_error(OSSM_ERR_INVALID_ARGUMENT, std::string(what) + ": null pointer");
-  LayerArgs args{inputs, B, C, D, a_diag, g_diag, step, outputs, static_cast<float4*>(carries),
+  LayerArgs args{inputs, B, C, D, a_diag, g_diag, step, params_lo, outputs, static_cast<float4*>(carries),
                  static_cast<int>(batch), static_cast<int>(length), static_cast<int>(hidden),
                  static_cast<int>(ssm), static_cast<int>(n_chunks)};
   hipStream_t stream = static_cast<hipStream_t>(stream_v);
@@ -888,13 +899,21 @@ int ossm_dlinoss_layer_forward(int variant, const float* inputs, const float* B,
   }
 }
 
-int ossm_dlinoss_layer_backward(int variant, const float* inputs, const float* grad_output,
-                                const float* B, const float* C, const float* D,
-                                const float* a_diag, const float* g_diag, const float* step,
-                                const void* carries, float* grad_inputs, void* grad_bu,
-                                void* x_conj, float* grad_a, float* grad_g, float* grad_step,
-                                int64_t batch, int64_t length, int64_t hidden, int64_t ssm,
-                                ossm_stream_t stream_v) {
+int ossm_dlinoss_layer_forward(int variant, const float* inputs, const float* B, const float* C,
+                               const float* D, const float* a_diag, const float* g_diag,
+                               const float* step, float* outputs, void* carries, int64_t batch,
+                               int64_t length, int64_t hidden, int64_t ssm, ossm_stream_t stream) {
+  return ossm_dlinoss_layer_forward_wide(variant, inputs, B, C, D, a_diag, g_diag, step, nullptr, outputs,
+                                         carries, batch, length, hidden, ssm, stream);
+}
+
+int ossm_dlinoss_layer_backward_wide(int variant, const float* inputs, const float* grad_output,
+                                     const float* B, const float* C, const float* D,
+                                     const float* a_diag, const float* g_diag, const float* step,
+                                     const float* params_lo, const void* carries, float* grad_inputs,
+                                     void* grad_bu, void* x_conj, float* grad_a, float* grad_g,
+                                     float* grad_step, int64_t batch, int64_t length, int64_t hidden,
+                                     int64_t ssm, ossm_stream_t stream_v) {
   clear_error();
   const char* what = "dlinoss_layer_backward";
   if (batch < 0 || length < 0 || hidden < 0 || ssm < 0)
@@ -925,7 +944,7 @@ int ossm_dlinoss_layer_backward(int variant, const float* inputs, const float* g
   if (!inputs || !grad_output || !D || !grad_inputs ||
       (ssm > 0 && (!B || !C || !a_diag || !g_diag || !step || !carries || !grad_bu || !x_conj)))
     return set_error(OSSM_ERR_INVALID_ARGUMENT, std::string(what) + ": null pointer");
-  LayerBwdArgs args{inputs, grad_output, B, C, D, a_diag, g_diag, step,
+  LayerBwdArgs args{inputs, grad_output, B, C, D, a_diag, g_diag, step, params_lo,
                     static_cast<const float4*>(carries), grad_inputs,
                     static_cast<float2*>(grad_bu), static_cast<float2*>(x_conj), nullptr,
                     ZeroFill{}, static_cast<int>(batch), static_cast<int>(length),
@@ -936,6 +955,18 @@ int ossm_dlinoss_layer_backward(int variant, const float* inputs, const float* g
     case OSSM_DLINOSS_IM: return launch_layer_bwd<OSSM_DLINOSS_IM>(args, grad_a, grad_g, grad_step, stream);
     default: return launch_layer_bwd<OSSM_DLINOSS_EX>(args, grad_a, grad_g, grad_step, stream);
   }
+}
+
+int ossm_dlinoss_layer_backward(int variant, const float* inputs, const float* grad_output,
+                                const float* B, const float* C, const float* D,
+                                const float* a_diag, const float* g_diag, const float* step,
+                                const void* carries, float* grad_inputs, void* grad_bu,
+                                void* x_conj, float* grad_a, float* grad_g, float* grad_step,
+                                int64_t batch, int64_t length, int64_t hidden, int64_t ssm,
+                                ossm_stream_t stream) {
+  return ossm_dlinoss_layer_backward_wide(variant, inputs, grad_output, B, C, D, a_diag, g_diag, step,
+                                          nullptr, carries, grad_inputs, grad_bu, x_conj, grad_a, grad_g,
+                                          grad_step, batch, length, hidden, ssm, stream);
 }
 
 }  // extern "C"

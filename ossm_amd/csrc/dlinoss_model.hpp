@@ -72,6 +72,26 @@ struct Dlinoss {
     return k;
   }
 
+  // The same table formed in double and rounded once.  An oscillator that rings
+  // for n steps turns a relative error e of its transition into about n e of
+  // its phase, so the several float roundings of coef_of are most of a layer's
+  // error where damping is weak.
+  static __device__ __forceinline__ Coef coef_wide(double alpha, double gamma, double sigma) {
+    const double s2 = sigma * sigma;
+    double inv = 1.0;
+    if constexpr (V == OSSM_DLINOSS_IMEX1) inv = 1.0 / (1.0 + sigma * gamma);
+    if constexpr (V == OSSM_DLINOSS_IM) inv = 1.0 / (1.0 + sigma * gamma + s2 * alpha);
+    const auto f = [](double x) { return static_cast<float>(x); };
+    if constexpr (V == OSSM_DLINOSS_IMEX1)
+      return {f(inv), f(-alpha * s2 * inv), f(s2 * inv), 0.f, 0.f, 0.f};
+    else if constexpr (V == OSSM_DLINOSS_IMEX2)
+      return {f(1.0 - sigma * gamma), f(-sigma * alpha), f(sigma), f(sigma - s2 * gamma), f(1.0 - s2 * alpha), f(s2)};
+    else if constexpr (V == OSSM_DLINOSS_IM)
+      return {f(inv), f(-alpha * sigma * inv), f(sigma * inv), f(sigma * inv), f((1.0 + sigma * gamma) * inv), f(s2 * inv)};
+    else
+      return {f(1.0 - sigma * gamma), f(-sigma * alpha), f(sigma), f(sigma), 0.f, 0.f};
+  }
+
   static __device__ __forceinline__ float4 step(const Coef& k, float4 s, float2 bu) {
     const float n0r = s.x * k.c0 + s.z * k.c1 + bu.x * k.c2;
     const float n0i = s.y * k.c0 + s.w * k.c1 + bu.y * k.c2;

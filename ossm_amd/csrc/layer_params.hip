@@ -7,8 +7,11 @@
 // A few hundred values: the time is launches.  As torch operations the D-LinOSS
 // form takes 21 forward launches and about 40 backward, each a host call of about
 // 5 us: a [8, 1030, 100] layer forward 134 us against 39 here (28 of them the
-// layer's own kernel), a [32, 4096, 128] training step 935 against 825.  Each lane works in double and rounds once: lo is a
-// difference of nearly equal terms.
+// layer's own kernel), a [32, 4096, 128] training step 935 against 825.
+// The D-LinOSS values are the float operations' own, rounding by rounding (a is
+// a difference of nearly equal terms there, and the layer's unfused form, which
+// runs them, has to agree with the fused one).  The LinOSS values are formed in
+// double and come with what rounding them left, as do both gradients.
 
 #include <hip/hip_runtime.h>
 
@@ -23,29 +26,35 @@ namespace ossm {
 namespace {
 
 constexpr int kParamBlock = 128;
-constexpr double kClamp = 1e-6;  // the floor of dt^2 and 1 + dt g
+constexpr double kClamp = 1e-6;  // the floor of dt^2
 
-// relu and clamp that pass NaN, as torch's do
-__device__ __forceinline__ double relu_nan(double x) { return x < 0.0 ? 0.0 : x; }
-__device__ __forceinline__ double at_least(double x, double lo) { return x < lo ? lo : x; }
+// Comparisons are written so that NaN passes through relu and clamp, as in torch.
 __device__ __forceinline__ double sigmoid64(double x) { return 1.0 / (1.0 + exp(-x)); }
 
 struct Band {
-  double dt, g, dt2, dg, root, lo, hi;
+  float a, g, dt, dt2, dg, root, lo, hi;
 };
-__device__ __forceinline__ Band band_of(double G, double steps) {
+// project_parameters in its own float operations, none fused
+__device__ __forceinline__ Band band_of(float A, float G, float steps) {
+#pragma clang fp contract(off)
   Band b;
-  b.dt = sigmoid64(steps);
-  b.g = relu_nan(G);
-  b.dt2 = at_least(b.dt * b.dt, kClamp);
+  b.dt = 1.f / (1.f + expf(-steps));
+  b.g = G < 0.f ? 0.f : G;
+  const float sq = b.dt * b.dt;
+  b.dt2 = sq < 1e-6f ? 1e-6f : sq;
   b.dg = b.dt * b.g;
-  b.root = sqrt(at_least(1.0 + b.dg, kClamp));
-  b.lo = (2.0 + b.dg - 2.0 * b.root) / b.dt2;
-  b.hi = (2.0 + b.dg + 2.0 * b.root) / b.dt2;
+  const float one = 1.f + b.dg;
+  b.root = sqrtf(one < 1e-6f ? 1e-6f : one);
+  const float two = 2.f + b.dg, r2 = 2.f * b.root;
+  b.lo = (two - r2) / b.dt2;
+  b.hi = (two + r2) / b.dt2;
+  const float over = A - b.lo, above = A - b.hi;
+  b.a = b.lo + (over < 0.f ? 0.f : over) - (above < 0.f ? 0.f : above);
   return b;
 }
 
-// out [3][n]: a, g, dt
+// out [6][n]: a, g, dt, then (not DAMPED) what rounding each left, from which the
+// layer kernels form their coefficients
 template <bool DAMPED>
 __global__ __launch_bounds__(kParamBlock) void layer_params_fwd_kernel(const float* __restrict__ A,
                                                                        const float* __restrict__ G,
@@ -53,19 +62,22 @@ __global__ __launch_bounds__(kParamBlock) void layer_params_fwd_kernel(const flo
                                                                        float* __restrict__ out, int n) {
   const int p = static_cast<int>(blockIdx.x) * kParamBlock + static_cast<int>(threadIdx.x);
   if (p >= n) return;
-  double a = A[p], g = 0.0, dt;
   if constexpr (DAMPED) {
-    const Band b = band_of(G[p], steps[p]);
-    a = b.lo + relu_nan(a - b.lo) - relu_nan(a - b.hi);
-    g = b.g;
-    dt = b.dt;
+    const Band b = band_of(A[p], G[p], steps[p]);
+    out[p] = b.a;
+    out[n + p] = b.g;
+    out[2 * n + p] = b.dt;
   } else {
-    a = relu_nan(a);
-    dt = sigmoid64(steps[p]);
+    const float a = A[p];
+    const double dt = sigmoid64(steps[p]);
+    const float hi = static_cast<float>(dt);
+    out[p] = a < 0.f ? 0.f : a;
+    out[n + p] = 0.f;
+    out[2 * n + p] = hi;
+    out[3 * n + p] = 0.f;
+    out[4 * n + p] = 0.f;
+    out[5 * n + p] = static_cast<float>(dt - hi);
   }
-  out[p] = static_cast<float>(a);
-  out[n + p] = static_cast<float>(g);
-  out[2 * n + p] = static_cast<float>(dt);
 }
 
 // grad [3][n]: of A, G (DAMPED), steps; a null upstream gradient is zero
@@ -81,17 +93,19 @@ __global__ __launch_bounds__(kParamBlock) void layer_params_bwd_kernel(
   const double a = A[p];
   double gA, dt;
   if constexpr (DAMPED) {
-    const Band b = band_of(G[p], steps[p]);
-    dt = b.dt;
-    const bool above_lo = !(a - b.lo <= 0.0), above_hi = !(a - b.hi <= 0.0);
+    const Band b = band_of(A[p], G[p], steps[p]);  // which side of the band the forward took
+    const bool above_lo = !(A[p] - b.lo <= 0.f), above_hi = !(A[p] - b.hi <= 0.f);
+    dt = sigmoid64(steps[p]);
+    const double g = b.g, sq = dt * dt, dg = dt * g;
+    const double dt2 = sq < kClamp ? kClamp : sq, root = sqrt(1.0 + dg);
+    const double lo = (2.0 + dg - 2.0 * root) / dt2, hi = (2.0 + dg + 2.0 * root) / dt2;
     gA = (above_lo ? ga : 0.0) - (above_hi ? ga : 0.0);
     const double glo = above_lo ? 0.0 : ga, ghi = above_hi ? ga : 0.0;
-    const double groot = (ghi - glo) * 2.0 / b.dt2;
-    double gdg = (glo + ghi) / b.dt2;
-    if (!(1.0 + b.dg < kClamp)) gdg += groot * 0.5 / b.root;
-    if (!(b.dt * b.dt < kClamp)) gdt -= (glo * b.lo + ghi * b.hi) / b.dt2 * 2.0 * b.dt;
-    gdt += gdg * b.g;
-    const double gG = gg + gdg * b.dt;
+    // 1 + dg >= 1: its clamp never acts
+    const double gdg = (glo + ghi) / dt2 + (ghi - glo) * 2.0 / dt2 * 0.5 / root;
+    if (!(sq < kClamp)) gdt -= (glo * lo + ghi * hi) / dt2 * 2.0 * dt;
+    gdt += gdg * g;
+    const double gG = gg + gdg * dt;
     grad[n + p] = static_cast<float>(static_cast<double>(G[p]) <= 0.0 ? 0.0 : gG);
   } else {
     dt = sigmoid64(steps[p]);
@@ -103,7 +117,7 @@ __global__ __launch_bounds__(kParamBlock) void layer_params_bwd_kernel(
 
 int check_params(int damped, const float* A, const float* G, const float* steps, const float* out, int64_t n,
                  const char* what) {
-  if (n < 0 || n > INT_MAX / 4) return set_error(OSSM_ERR_INVALID_ARGUMENT, std::string(what) + ": bad size");
+  if (n < 0 || n > INT_MAX / 8) return set_error(OSSM_ERR_INVALID_ARGUMENT, std::string(what) + ": bad size");
   if (n > 0 && (!A || !steps || !out || (damped && !G)))
     return set_error(OSSM_ERR_INVALID_ARGUMENT, std::string(what) + ": null pointer");
   return OSSM_OK;

@@ -13,7 +13,7 @@ with bu and the states kept on chip; for training it also saves the state
 entering each 32-step chunk.  The backward is ``ossm_dlinoss_layer_backward``
 (the projections of the upstream gradient and of u on the matrix cores, the
 states re-run from those carries, the scan adjoint, grad_u), followed by the
-two weight-gradient GEMMs over the grad_bu and x it returns.  Shapes whose
+two weight-gradient products over the grad_bu and x it returns.  Shapes whose
 backward does not fit one workgroup's LDS recompute through the unfused
 composition (``unfused_layer_forward``) and differentiate that.
 
@@ -33,6 +33,7 @@ from torch import Tensor, nn
 
 from . import _lib
 from .bridge import run_dlinoss
+from .linear import MIN_ROWS, rows_product
 
 __all__ = ["DampedLinOSSLayer", "dlinoss_layer_forward", "dlinoss_layer_backward", "DlinossLayerFn",
            "project_parameters", "unfused_layer_forward", "LayerParamsFn", "fused_layer_supported"]
@@ -68,15 +69,16 @@ def project_parameters(A_diag: Tensor, G_diag: Tensor, steps: Tensor) -> Tuple[T
 
 
 class LayerParamsFn(torch.autograd.Function):
-    """(a, g, dt) of a layer from its stored float32 GPU parameters, one launch
-    each way: ``project_parameters`` when ``damped``, else the LinOSS layer's
-    ``(relu(A), 0, sigmoid(steps))`` (G_diag is then None)."""
+    """(a, g, dt, lo) of a layer from its stored float32 GPU parameters, one launch
+    each way: ``project_parameters`` when ``damped`` (the same float operations;
+    ``lo`` is None), else the LinOSS layer's ``(relu(A), 0, sigmoid(steps))``, with
+    G_diag None and ``lo`` [3, P] what rounding each to float32 left."""
 
     @staticmethod
     def forward(ctx, damped: bool, A_diag: Tensor, G_diag: Optional[Tensor],
-                steps: Tensor) -> Tuple[Tensor, Tensor, Tensor]:  # type: ignore[override]
+                steps: Tensor):  # type: ignore[override]
         A, G, s = (None if t is None else t.contiguous() for t in (A_diag, G_diag, steps))
-        out = torch.empty((3, A.numel()), dtype=torch.float32, device=A.device)
+        out = torch.empty((6, A.numel()), dtype=torch.float32, device=A.device)
         with torch.cuda.device(A.device):
             _lib.check(_lib.load().ossm_layer_params_forward(
                 int(damped), A.data_ptr(), _lib.ptr(G), s.data_ptr(), out.data_ptr(), A.numel(),
@@ -84,11 +86,15 @@ class LayerParamsFn(torch.autograd.Function):
         ctx.damped = damped
         ctx.set_materialize_grads(False)
         ctx.save_for_backward(A_diag, G_diag, steps)
-        return out[0], out[1], out[2]
+        lo = None
+        if not damped:
+            lo = out[3:]
+            ctx.mark_non_differentiable(lo)
+        return out[0], out[1], out[2], lo
 
     @staticmethod
     def backward(ctx, *grads: Optional[Tensor]):  # type: ignore[override]
-        params = ctx.saved_tensors
+        params, grads = ctx.saved_tensors, grads[:3]
         if torch.is_grad_enabled():
             # create_graph: differentiable again, as torch operations
             A, G, s = params
@@ -155,13 +161,22 @@ def _check_carries(carries: Tensor, batch: int, length: int, ssm: int, device) -
         raise RuntimeError(f"carries must be a contiguous float32 {want} tensor on {device}")
 
 
+def _check_lo(lo: Optional[Tensor], a: Tensor) -> Optional[Tensor]:
+    if lo is not None and (tuple(lo.shape) != (3, a.numel()) or lo.dtype != torch.float32
+                           or not lo.is_contiguous() or lo.device != a.device):
+        raise RuntimeError(f"lo must be a contiguous float32 (3, {a.numel()}) tensor on {a.device}")
+    return lo
+
+
 def dlinoss_layer_forward(variant: str, inputs: Tensor, B: Tensor, C: Tensor, D: Tensor,
                           a_diag: Tensor, g_diag: Tensor, step: Tensor,
-                          carries: Optional[Tensor] = None) -> Tensor:
+                          carries: Optional[Tensor] = None, lo: Optional[Tensor] = None) -> Tensor:
     """y = Re(x C^T) + D u with x the D-LinOSS states driven by bu = u B^T, in
     one kernel launch.  Every tensor float32 on one GPU; a, g, step projected.
     ``carries`` (float32 [batch, ceil(length / 32), ssm, 4]) receives the state
-    entering each chunk, for ``dlinoss_layer_backward``."""
+    entering each chunk, for ``dlinoss_layer_backward``.  ``lo`` ([3, ssm], from
+    ``LayerParamsFn``): what a, g, step leave of their double values; the
+    coefficients are formed in double from the sums."""
     variant = variant.lower()
     if variant not in _VARIANTS:
         raise ValueError(f"Unknown D-LinOSS variant '{variant}'.")
@@ -176,20 +191,21 @@ def dlinoss_layer_forward(variant: str, inputs: Tensor, B: Tensor, C: Tensor, D:
         _check_carries(carries, batch, length, ssm, u.device)
     lib = _lib.load()
     with torch.cuda.device(u.device):
-        _lib.check(lib.ossm_dlinoss_layer_forward(
+        _lib.check(lib.ossm_dlinoss_layer_forward_wide(
             _VARIANTS[variant], u.data_ptr(), Bc.data_ptr(), Cc.data_ptr(), Dc.data_ptr(),
-            a.data_ptr(), g.data_ptr(), s.data_ptr(), out.data_ptr(), _lib.ptr(carries), batch,
+            a.data_ptr(), g.data_ptr(), s.data_ptr(), _lib.ptr(_check_lo(lo, a)), out.data_ptr(), _lib.ptr(carries), batch,
             length, hidden, ssm, _lib.stream_of(u)))
     return out
 
 
 def dlinoss_layer_backward(variant: str, inputs: Tensor, grad_output: Tensor, B: Tensor,
                            C: Tensor, D: Tensor, a_diag: Tensor, g_diag: Tensor, step: Tensor,
-                           carries: Tensor):
+                           carries: Tensor, lo: Optional[Tensor] = None):
     """Gradients of the fused layer: ``(grad_inputs, grad_B, grad_C, grad_D, grad_a,
-    grad_g, grad_step)`` from the forward's ``carries``.  One kernel for
-    grad_inputs and the scan's parameter gradients; grad_B and grad_C are GEMMs
-    over the grad_bu and conj(x) it returns, grad_D a sum."""
+    grad_g, grad_step)`` from the forward's ``carries`` (and
+    ``lo``).  One kernel for
+    grad_inputs and the scan's parameter gradients; grad_B and grad_C are row
+    products over the grad_bu and conj(x) it returns, grad_D a sum."""
     variant = variant.lower()
     if variant not in _VARIANTS:
         raise ValueError(f"Unknown D-LinOSS variant '{variant}'.")
@@ -207,29 +223,30 @@ def dlinoss_layer_backward(variant: str, inputs: Tensor, grad_output: Tensor, B:
     xq = torch.empty_like(gbu)
     ga, gg, gs = (torch.empty(ssm, dtype=torch.float32, device=dev) for _ in range(3))
     with torch.cuda.device(dev):
-        _lib.check(_lib.load().ossm_dlinoss_layer_backward(
+        _lib.check(_lib.load().ossm_dlinoss_layer_backward_wide(
             _VARIANTS[variant], u.data_ptr(), go.data_ptr(), Bc.data_ptr(), Cc.data_ptr(),
-            Dc.data_ptr(), a.data_ptr(), g.data_ptr(), s.data_ptr(), carries.data_ptr(),
+            Dc.data_ptr(), a.data_ptr(), g.data_ptr(), s.data_ptr(), _lib.ptr(_check_lo(lo, a)),
+            carries.data_ptr(),
             gu.data_ptr(), gbu.data_ptr(), xq.data_ptr(), ga.data_ptr(), gg.data_ptr(),
             gs.data_ptr(), batch, length, hidden, ssm, _lib.stream_of(u)))
     rows = batch * length
     uf, gof = u.reshape(rows, hidden), go.reshape(rows, hidden)
     # grad_B[p, h, c] = sum_r grad_bu[r, p, c] u[r, h];  grad_C[h, p, c] = sum_r go[r, h] xq[r, p, c]
-    gB = _sum_rows_product(gbu.reshape(rows, 2 * ssm), uf)
-    gB = gB.reshape(ssm, 2, hidden).permute(0, 2, 1).contiguous()
-    gC = _sum_rows_product(gof, xq.reshape(rows, 2 * ssm)).reshape(hidden, ssm, 2)
+    gbu2, xq2 = gbu.reshape(rows, 2 * ssm), xq.reshape(rows, 2 * ssm)
+    if rows >= MIN_ROWS:
+        gB, gC = rows_product(gbu2, uf, pairs=True), rows_product(gof, xq2)
+    else:
+        gB = _sum_rows_product(gbu2, uf).reshape(ssm, 2, hidden).permute(0, 2, 1).contiguous()
+        gC = _sum_rows_product(gof, xq2)
+    gC = gC.reshape(hidden, ssm, 2)
     gD = (gof * uf).sum(0)
     return gu, gB, gC, gD, ga, gg, gs
 
 
 def _sum_rows_product(a: Tensor, b: Tensor, split: int = 32) -> Tensor:
-    """a^T b for row-major a [R, M], b [R, N] with R much larger than M, N (the
-    weight gradients sum over every (batch, step) row): the first
-    split * (R // split) rows are split into ``split`` slices multiplied as one
-    batched GEMM and the partials added, the remaining rows (fewer than
-    ``split``) by one small GEMM.  That is the shape the library GEMMs run
-    well: one GEMM with K = R ran at ~24 TFLOP/s here, 16–64 slices at ~110
-    (128 slices 104, 512 slices 80)."""
+    """a^T b for row-major a [R, M], b [R, N] of fewer rows than ``rows_product``
+    takes: the first split * (R // split) rows as ``split`` slices of one batched
+    GEMM, the partials added, the remaining rows by one small GEMM."""
     R = a.size(0)
     n = R // split
     if n < 4:
@@ -265,32 +282,34 @@ class DlinossLayerFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, variant: str, inputs: Tensor, B: Tensor, C: Tensor, D: Tensor,
-                a_diag: Tensor, g_diag: Tensor, step: Tensor) -> Tensor:  # type: ignore[override]
+                a_diag: Tensor, g_diag: Tensor, step: Tensor,
+                lo: Optional[Tensor] = None) -> Tensor:  # type: ignore[override]
         ctx.variant = variant
         batch, length, hidden = inputs.shape
         ssm = B.size(0)
         carries = None
-        if any(ctx.needs_input_grad[1:]) and _bwd_fits(hidden, ssm):
+        if any(ctx.needs_input_grad[1:8]) and _bwd_fits(hidden, ssm):
             carries = torch.empty((batch, -(-length // _CHUNK), ssm, 4), dtype=torch.float32,
                                   device=inputs.device)
         ctx.fused_bwd = carries is not None
-        ctx.save_for_backward(inputs, B, C, D, a_diag, g_diag, step, carries)
-        return dlinoss_layer_forward(variant, inputs, B, C, D, a_diag, g_diag, step, carries)
+        ctx.save_for_backward(inputs, B, C, D, a_diag, g_diag, step, carries, lo)
+        return dlinoss_layer_forward(variant, inputs, B, C, D, a_diag, g_diag, step, carries, lo)
 
     @staticmethod
     def backward(ctx, grad_out: Tensor):  # type: ignore[override]
-        *saved, carries = ctx.saved_tensors
-        needs = ctx.needs_input_grad[1:]
+        *saved, carries, lo = ctx.saved_tensors
+        needs = ctx.needs_input_grad[1:8]
+        tail = (None,) * (len(ctx.needs_input_grad) - 8)  # lo, where it was passed
         if ctx.fused_bwd:
-            grads = dlinoss_layer_backward(ctx.variant, *saved[:1], grad_out, *saved[1:], carries)
-            return (None, *[gr if n else None for gr, n in zip(grads, needs)])
+            grads = dlinoss_layer_backward(ctx.variant, *saved[:1], grad_out, *saved[1:], carries, lo)
+            return (None, *[gr if n else None for gr, n in zip(grads, needs)], *tail)
         with torch.enable_grad():
             leaves = [t.detach().requires_grad_(bool(n)) for t, n in zip(saved, needs)]
             y = unfused_layer_forward(ctx.variant, *leaves)
             wanted = [t for t in leaves if t.requires_grad]
             got = iter(torch.autograd.grad(y, wanted, grad_out)) if wanted else iter(())
         grads = [next(got) if t.requires_grad else None for t in leaves]
-        return (None, *grads)
+        return (None, *grads, *tail)
 
 
 class DampedLinOSSLayer(nn.Module):
@@ -393,8 +412,8 @@ class DampedLinOSSLayer(nn.Module):
                   (self.A_diag, self.G_diag, self.steps, self.B, self.C, self.D)]
         Bw, Cw, Dw = params[3:]
         if u.is_cuda and self.hidden_dim <= _LAYER_MAX and self.ssm_size <= _LAYER_MAX:
-            a, g, dt = LayerParamsFn.apply(True, *params[:3])
-            y = DlinossLayerFn.apply(self.variant, u, Bw, Cw, Dw, a, g, dt)
+            a, g, dt, lo = LayerParamsFn.apply(True, *params[:3])
+            y = DlinossLayerFn.apply(self.variant, u, Bw, Cw, Dw, a, g, dt, lo)
         else:
             a, g, dt = project_parameters(*params[:3])
             y = unfused_layer_forward(self.variant, u, Bw, Cw, Dw, a, g, dt)

@@ -87,9 +87,9 @@ class LinOSSLayer(nn.Module):
         if fused_layer_supported(inputs, (self.A_diag, self.B, self.C, self.D, self.steps), hidden,
                                  self.ssm_size):
             # IM and IMEX are the undamped (g = 0) D-LinOSS im and imex2 recurrences
-            a, g, dt = LayerParamsFn.apply(False, self.A_diag, None, self.steps)
+            a, g, dt, lo = LayerParamsFn.apply(False, self.A_diag, None, self.steps)
             return DlinossLayerFn.apply("im" if self.discretization == "IM" else "imex2", inputs,
-                                        self.B, self.C, self.D, a, g, dt)
+                                        self.B, self.C, self.D, a, g, dt, lo)
         a_diag = cast(torch.relu(self.A_diag))
         step = cast(torch.sigmoid(self.steps))
         flat = inputs.reshape(batch * length, hidden)

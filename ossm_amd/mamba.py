@@ -24,10 +24,10 @@ import math
 from typing import Optional, Tuple
 
 import torch
-import torch.nn.functional as F
 from torch import Tensor, nn
 
 from . import _lib
+from .linear import linear, linear_weight
 
 __all__ = ["MambaMixer", "mamba_conv_silu", "selective_scan_mamba", "ConvSiluFn", "MambaScanFn"]
 
@@ -270,14 +270,14 @@ class MambaMixer(nn.Module):
         if not inputs.is_cuda:
             raise RuntimeError("the fused Mamba mixer runs on the GPU only")
         Di, R, N = self.d_inner, self.dt_rank, self.d_state
-        xz = self.in_proj(inputs).float()
+        xz = linear(self.in_proj, inputs).float()
         x, z = _ColumnSplit.apply(xz, Di)                 # views, row stride 2 * d_inner
         x_conv = mamba_conv_silu(x, self.conv1d.weight.float(),
                                  None if self.conv1d.bias is None else self.conv1d.bias.float())
-        proj = self.x_proj(x_conv.to(self.x_proj.weight.dtype)).float()
+        proj = linear(self.x_proj, x_conv.to(self.x_proj.weight.dtype)).float()
         dt_raw, B_gen, C_gen = proj[..., :R], proj[..., R:R + N], proj[..., R + N:]
-        dt_pre = F.linear(dt_raw, self.dt_proj.weight.float())   # bias goes into the softplus
+        dt_pre = linear_weight(dt_raw, self.dt_proj.weight.float())  # bias goes into the softplus
         A = -torch.exp(self.A_log.float())
         y = selective_scan_mamba(x_conv, dt_pre, A, B_gen, C_gen, gate=z,
                                  dt_bias=self.dt_proj.bias.float())
-        return self.out_proj(y.to(self.out_proj.weight.dtype))
+        return linear(self.out_proj, y.to(self.out_proj.weight.dtype))
