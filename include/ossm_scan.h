@@ -487,6 +487,24 @@ int ossm_mamba_conv_backward(const float* x, int64_t ld_x, const float* weight, 
                              int64_t width, ossm_stream_t stream);
 
 /*
+ * The two backwards above with strided gradients, so that they can be written into
+ * parts of one tensor: grad_x with row stride ld_grad_x; dgate with ld_dgate, dB and
+ * dC with ld_dbc (then a gate is needed and nothing may be empty).
+ */
+int ossm_mamba_conv_backward_ld(const float* x, int64_t ld_x, const float* weight, const float* bias,
+                                const float* grad_out, float* grad_x, int64_t ld_grad_x,
+                                float* grad_weight, float* grad_bias, int64_t batch, int64_t length,
+                                int64_t dim, int64_t width, ossm_stream_t stream);
+int ossm_selective_mamba_backward_ld(const float* grad_out, const float* u, int64_t ld_u,
+                                     const float* dt, int64_t ld_dt, const float* dt_bias,
+                                     const float* A, const float* Bm, const float* Cm, int64_t ld_bc,
+                                     const float* gate, int64_t ld_z, const float* chunk_states,
+                                     const float* raw_out, float* du, float* ddt, float* dA,
+                                     float* dB, float* dC, int64_t ld_dbc, float* dgate,
+                                     int64_t ld_dgate, int64_t batch, int64_t dim, int64_t length,
+                                     int64_t dstate, ossm_stream_t stream);
+
+/*
  * The oscillator parameters of a layer from their stored form, out [6][ssm] =
  * a, g, dt and (not damped) what the rounding of each to float32 left.  damped != 0: the D-LinOSS layer's stability projection
  * (dlinoss.py:249-264: dt = sigmoid(steps), g = relu(G_diag), a clamped to its

@@ -130,6 +130,13 @@ _SIGNATURES = {
         ctypes.c_int, [ctypes.c_int, _fp, _fp, _fp, _fp, _c_int64, _vp]),
     "ossm_layer_params_backward": (
         ctypes.c_int, [ctypes.c_int, _fp, _fp, _fp, _fp, _fp, _fp, _fp, _c_int64, _vp]),
+    "ossm_mamba_conv_backward_ld": (
+        ctypes.c_int,
+        [_fp, _c_int64, _fp, _fp, _fp, _fp, _c_int64, _fp, _fp, _c_int64, _c_int64, _c_int64, _c_int64, _vp]),
+    "ossm_selective_mamba_backward_ld": (
+        ctypes.c_int,
+        [_fp, _fp, _c_int64, _fp, _c_int64, _fp, _fp, _fp, _fp, _c_int64, _fp, _c_int64, _fp, _fp, _fp,
+         _fp, _fp, _fp, _fp, _c_int64, _fp, _c_int64, _c_int64, _c_int64, _c_int64, _c_int64, _vp]),
     "ossm_rows_product": (
         ctypes.c_int,
         [_fp, _c_int64, _fp, _c_int64, _fp, _c_int64, _c_int64, _c_int64, _c_int64, _c_int64, _c_int64, _vp]),

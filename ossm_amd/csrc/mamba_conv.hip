@@ -47,11 +47,11 @@ struct ConvArgs {
   const float* w;     // [D, K]
   const float* bias;  // [D] or null
   const float* dout;  // backward: [B, L, D] dense
-  float* out;         // forward: [B, L, D] dense; backward: dx [B, L, D] dense
+  float* out;         // forward: [B, L, D] dense; backward: dx [B, L, D], row stride ld_out
   float* partials;    // backward: [B * n_spans][K + 1][D]
   float* grad_w;      // backward: zeroed by the first workgroup (the column sums add into it)
   float* grad_bias;
-  int B, L, D, ld_x;
+  int B, L, D, ld_x, ld_out;
   int n_spans;
 };
 
@@ -166,6 +166,7 @@ __global__ __launch_bounds__(kConvThreads) void conv_silu_bwd_kernel(ConvArgs a)
   if (!conv_pos<C>(a, b, span, d)) return;  // no barriers below
   const size_t xb = static_cast<size_t>(b) * a.L * a.ld_x;
   const size_t ob = static_cast<size_t>(b) * a.L * a.D;
+  const size_t gxb = static_cast<size_t>(b) * a.L * a.ld_out;
   float w[K][C], bias[C];
   load_weights<K, C>(a, d, w, bias);
   float gw[K][C], gb[C];
@@ -220,7 +221,7 @@ __global__ __launch_bounds__(kConvThreads) void conv_silu_bwd_kernel(ConvArgs a)
 #pragma unroll
         for (int k = 0; k < K; ++k) gw[k][e] = fmaf(dp[i].v[e], xs[i + k].v[e], gw[k][e]);
       }
-      store_vec<C>(a.out + ob + static_cast<size_t>(t) * a.D + d, gx);
+      store_vec<C>(a.out + gxb + static_cast<size_t>(t) * a.ld_out + d, gx);
     }
   }
   // partials row (b, span): [K + 1][D]
@@ -348,7 +349,7 @@ int ossm_mamba_conv_forward(const float* x, int64_t ld_x, const float* weight, c
     return set_error(OSSM_ERR_INVALID_ARGUMENT, "mamba_conv_forward: null pointer");
   ConvArgs a{x, weight, bias, nullptr, out, nullptr, nullptr, nullptr, static_cast<int>(batch),
              static_cast<int>(length), static_cast<int>(dim), static_cast<int>(ld_x),
-             static_cast<int>((length + kFwdSpan - 1) / kFwdSpan)};
+             static_cast<int>(dim), static_cast<int>((length + kFwdSpan - 1) / kFwdSpan)};
   const bool vec = dim % 4 == 0 && ld_x % 4 == 0 && aligned16(x) && aligned16(out);
   return by_width<FwdLaunch>(static_cast<int>(width), a, vec, static_cast<hipStream_t>(stream_v));
 }
@@ -356,9 +357,19 @@ int ossm_mamba_conv_forward(const float* x, int64_t ld_x, const float* weight, c
 int ossm_mamba_conv_backward(const float* x, int64_t ld_x, const float* weight, const float* bias,
                              const float* grad_out, float* grad_x, float* grad_weight,
                              float* grad_bias, int64_t batch, int64_t length, int64_t dim,
-                             int64_t width, ossm_stream_t stream_v) {
+                             int64_t width, ossm_stream_t stream) {
+  return ossm_mamba_conv_backward_ld(x, ld_x, weight, bias, grad_out, grad_x, dim, grad_weight, grad_bias,
+                                     batch, length, dim, width, stream);
+}
+
+int ossm_mamba_conv_backward_ld(const float* x, int64_t ld_x, const float* weight, const float* bias,
+                                const float* grad_out, float* grad_x, int64_t ld_grad_x,
+                                float* grad_weight, float* grad_bias, int64_t batch, int64_t length,
+                                int64_t dim, int64_t width, ossm_stream_t stream_v) {
   clear_error();
   if (int rc = check_conv(batch, length, dim, width, ld_x, "mamba_conv_backward")) return rc;
+  if (ld_grad_x < dim || ld_grad_x > INT_MAX)
+    return set_error(OSSM_ERR_INVALID_ARGUMENT, "mamba_conv_backward: ld_grad_x < D");
   hipStream_t stream = static_cast<hipStream_t>(stream_v);
   StreamCall call(stream);
   if (call.status()) return call.status();
@@ -377,7 +388,7 @@ int ossm_mamba_conv_backward(const float* x, int64_t ld_x, const float* weight, 
     return rc;
   ConvArgs a{x, weight, bias, grad_out, grad_x, static_cast<float*>(ws), grad_weight, grad_bias,
              static_cast<int>(batch), static_cast<int>(length), static_cast<int>(dim),
-             static_cast<int>(ld_x), n_spans};
+             static_cast<int>(ld_x), static_cast<int>(ld_grad_x), n_spans};
   return by_width<BwdLaunch>(static_cast<int>(width), a, stream);
 }
 

@@ -1008,9 +1008,9 @@ struct BwdArgs {
   int Bsz, D, L, N, n_base, n_chunks;
   int first, last, vec;
   int ld_bc;           // row stride of B and C
-  // [B, L, D] layout only: row strides of u, dt and z (gout, raw, du, ddt, dz:
+  // [B, L, D] layout only: row strides of u, dt, z and dz (gout, raw, du, ddt:
   // D); dt is given before its softplus and ddt is returned w.r.t. it
-  int ld_u, ld_dt, ld_z;
+  int ld_u, ld_dt, ld_z, ld_dz;
   const float* dt_bias;
   // SKIP kernels ([B, D, L] only): the skip D of the forward; the first pass
   // adds D gy to du and writes the (segment, batch row) partials of
@@ -1348,7 +1348,7 @@ __global__ __launch_bounds__(kThreads) void selective_bwd_kernel(BwdArgs<E> a) {
                                   go.y * y.y * (sg.y * (1.f + zz.y * (1.f - sg.y))),
                                   go.z * y.z * (sg.z * (1.f + zz.z * (1.f - sg.z))),
                                   go.w * y.w * (sg.w * (1.f + zz.w * (1.f - sg.w)))};
-            E* dst = a.dz + (row0 + t) * a.D + dd;
+            E* dst = a.dz + (row0 + t) * a.ld_dz + dd;
             if constexpr (VEC) {
               Elem<E>::store4(dst, make_float4(dzv[0], dzv[1], dzv[2], dzv[3]));
             } else {
@@ -2125,7 +2125,12 @@ __global__ __launch_bounds__(kFinThreads) void selective_finish_kernel(
     const float* __restrict__ part_dB, const float* __restrict__ part_dC,
     const float* __restrict__ part_dA, E* __restrict__ dB, E* __restrict__ dC,
     float* __restrict__ dA, int64_t n_bln, int n_dtiles, int64_t n_dn, int rows, int n_bc_blocks,
-    int vec, int n_dA_blocks, const float* __restrict__ part_dD, float* __restrict__ dD, int n_d) {
+    int vec, int n_dA_blocks, const float* __restrict__ part_dD, float* __restrict__ dD, int n_d, int N,
+    int ld_out) {
+  // element i of [B L, N] in dB / dC of row stride ld_out
+  const auto at = [&](int64_t i) -> int64_t {
+    return ld_out == N ? i : i / N * ld_out + i % N;
+  };
   if (static_cast<int>(blockIdx.x) < n_bc_blocks) {
     // tiles added in ascending order; the loads of 8 tiles are issued before
     // any of them is added (the sum stays the same, bit for bit)
@@ -2158,8 +2163,8 @@ __global__ __launch_bounds__(kFinThreads) void selective_finish_kernel(
         add(sb, *reinterpret_cast<const float4*>(part_dB + static_cast<size_t>(k) * n_bln + i));
         add(sc, *reinterpret_cast<const float4*>(part_dC + static_cast<size_t>(k) * n_bln + i));
       }
-      Elem<E>::store4(dB + i, sb);
-      Elem<E>::store4(dC + i, sc);
+      Elem<E>::store4(dB + at(i), sb);
+      Elem<E>::store4(dC + at(i), sc);
       return;
     }
     const int64_t i = static_cast<int64_t>(blockIdx.x) * kFinThreads + threadIdx.x;
@@ -2183,8 +2188,8 @@ __global__ __launch_bounds__(kFinThreads) void selective_finish_kernel(
       sb += part_dB[static_cast<size_t>(k) * n_bln + i];
       sc += part_dC[static_cast<size_t>(k) * n_bln + i];
     }
-    Elem<E>::store1(dB + i, sb);
-    Elem<E>::store1(dC + i, sc);
+    Elem<E>::store1(dB + at(i), sb);
+    Elem<E>::store1(dC + at(i), sc);
     return;
   }
   __shared__ float s_part[kFinGroups][kFinCols];
@@ -2259,6 +2264,8 @@ int zero_fill(E* p, int64_t n, hipStream_t stream) {
 struct MambaLayout {
   int64_t ld_u, ld_dt, ld_z, ld_bc;
   const float* dt_bias;
+  // backward: row strides of dz and of dB, dC (0: dense)
+  int64_t ld_dz = 0, ld_dbc = 0;
 };
 
 bool aligned_to(const void* p, size_t bytes) { return reinterpret_cast<uintptr_t>(p) % bytes == 0; }
@@ -2266,7 +2273,8 @@ bool aligned_to(const void* p, size_t bytes) { return reinterpret_cast<uintptr_t
 // 16-byte moves along the channels: D and every row stride a multiple of 4
 // and every tensor 16-byte aligned (null pointers pass).
 bool cols_vectorizable(int64_t D, const MambaLayout& ml, std::initializer_list<const void*> ptrs) {
-  if (D % 4 != 0 || ml.ld_u % 4 != 0 || ml.ld_dt % 4 != 0 || ml.ld_z % 4 != 0) return false;
+  if (D % 4 != 0 || ml.ld_u % 4 != 0 || ml.ld_dt % 4 != 0 || ml.ld_z % 4 != 0 || ml.ld_dz % 4 != 0)
+    return false;
   for (const void* p : ptrs)
     if (!aligned_to(p, 16)) return false;
   return true;
@@ -2526,6 +2534,7 @@ int selective_backward_impl(const E* grad_out, const E* u, const E* dt, const fl
     a.ld_u = static_cast<int>(ml->ld_u);
     a.ld_dt = static_cast<int>(ml->ld_dt);
     a.ld_z = static_cast<int>(ml->ld_z);
+    a.ld_dz = static_cast<int>(ml->ld_dz > 0 ? ml->ld_dz : dim);
     a.dt_bias = ml->dt_bias;
     a.vec = cols_vectorizable(dim, *ml, {grad_out, u, dt, gate, raw_out, du, ddt, dgate}) ? 1 : 0;
   } else {
@@ -2565,8 +2574,10 @@ int selective_backward_impl(const E* grad_out, const E* u, const E* dt, const fl
     hipLaunchKernelGGL(kern, grid, dim3(kThreads), 0, stream, a);
     if (int rc = launch_check("selective_bwd_kernel")) return rc;
   }
+  const int64_t ld_dbc = ml != nullptr && ml->ld_dbc > 0 ? ml->ld_dbc : dstate;
   const int fin_vec = n_bln % kFinVec == 0 && aligned_to(dB, kFinVec * sizeof(E)) &&
-                      aligned_to(dC, kFinVec * sizeof(E));
+                      aligned_to(dC, kFinVec * sizeof(E)) &&
+                      (ld_dbc == dstate || (ld_dbc % kFinVec == 0 && dstate % kFinVec == 0));
   const int64_t per_block = static_cast<int64_t>(kFinThreads) * (fin_vec ? kFinVec : 1);
   const int64_t n_bc_blocks = (n_bln + per_block - 1) / per_block;
   const int64_t n_dA_blocks = (n_dn + kFinCols - 1) / kFinCols;
@@ -2576,7 +2587,7 @@ int selective_backward_impl(const E* grad_out, const E* u, const E* dt, const fl
                      dim3(kFinThreads), 0, stream, part_dB, part_dC, part_dA, dB, dC, dA, n_bln,
                      static_cast<int>(n_dtiles), n_dn, static_cast<int>(dA_rows),
                      static_cast<int>(n_bc_blocks), fin_vec, static_cast<int>(n_dA_blocks), part_dD,
-                     dD, static_cast<int>(dim));
+                     dD, static_cast<int>(dim), static_cast<int>(dstate), static_cast<int>(ld_dbc));
   if (int rc = launch_check("selective_finish_kernel")) return rc;
   if (gate == nullptr && dgate != nullptr) return zero_fill(dgate, n_rows, stream);
   return OSSM_OK;
@@ -2643,12 +2654,31 @@ int ossm_selective_mamba_backward(const float* grad_out, const float* u, int64_t
                                   const float* raw_out, float* du, float* ddt, float* dA,
                                   float* dB, float* dC, float* dgate, int64_t batch, int64_t dim,
                                   int64_t length, int64_t dstate, ossm_stream_t stream) {
+  return ossm_selective_mamba_backward_ld(grad_out, u, ld_u, dt, ld_dt, dt_bias, A, Bm, Cm, ld_bc, gate,
+                                          ld_z, chunk_states, raw_out, du, ddt, dA, dB, dC, dstate, dgate,
+                                          dim, batch, dim, length, dstate, stream);
+}
+
+int ossm_selective_mamba_backward_ld(const float* grad_out, const float* u, int64_t ld_u,
+                                     const float* dt, int64_t ld_dt, const float* dt_bias,
+                                     const float* A, const float* Bm, const float* Cm, int64_t ld_bc,
+                                     const float* gate, int64_t ld_z, const float* chunk_states,
+                                     const float* raw_out, float* du, float* ddt, float* dA,
+                                     float* dB, float* dC, int64_t ld_dbc, float* dgate,
+                                     int64_t ld_dgate, int64_t batch, int64_t dim, int64_t length,
+                                     int64_t dstate, ossm_stream_t stream) {
   const char* what = "selective_mamba_backward";
   clear_error();
   if (dstate > 0)
     if (int rc = check_mamba_strides(dim, dstate, ld_u, ld_dt, ld_z, gate != nullptr, ld_bc, what))
       return rc;
-  const MambaLayout ml{ld_u, ld_dt, gate != nullptr ? ld_z : dim, ld_bc, dt_bias};
+  // empty problems and a missing gate clear their outputs as dense tensors
+  const bool dense = ld_dbc == dstate && ld_dgate == dim;
+  if (!dense && (ld_dbc < dstate || ld_dgate < dim || ld_dbc > INT_MAX || ld_dgate > INT_MAX || !gate ||
+                 batch <= 0 || dim <= 0 || length <= 0))
+    return set_error(OSSM_ERR_INVALID_ARGUMENT, std::string(what) + ": strided gradients need a gate, a "
+                                                                    "nonempty problem and row strides that hold a row");
+  const MambaLayout ml{ld_u, ld_dt, gate != nullptr ? ld_z : dim, ld_bc, dt_bias, ld_dgate, ld_dbc};
   return selective_backward_impl<float>(grad_out, u, dt, A, Bm, Cm, gate, chunk_states, raw_out,
                                         du, ddt, dA, dB, dC, dgate, batch, dim, length, dstate,
                                         static_cast<hipStream_t>(stream), what, &ml);

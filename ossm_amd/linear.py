@@ -16,7 +16,8 @@ from torch import Tensor, nn
 
 from . import _lib
 
-__all__ = ["rows_product", "linear", "linear_weight", "LinearFn", "MIN_ROWS"]
+__all__ = ["rows_product", "linear", "linear_weight", "LinearFn", "is_plain",
+           "MIN_ROWS"]
 
 # Fewer rows go to the library: 200 rows 9 us there against 12, 1000 rows 60
 # against 14 ([R, 80] x [R, 40] and [R, 256] x [R, 64]).
@@ -76,7 +77,7 @@ class LinearFn(torch.autograd.Function):
         return gx, gw, (g2.sum(0) if need_b and ctx.has_bias else None)
 
 
-def _plain(module: nn.Module) -> bool:
+def is_plain(module: nn.Module) -> bool:
     """Whether calling ``module`` is F.linear on its own weight and nothing else
     (no subclass, no hooks, its own or global, no replaced forward)."""
     glob = nn.modules.module
@@ -90,7 +91,7 @@ def _plain(module: nn.Module) -> bool:
 def linear(module: nn.Module, x: Tensor) -> Tensor:
     """``module(x)``; a plain float32 ``nn.Linear`` on the GPU that trains takes
     its weight gradient from ``rows_product``."""
-    if _plain(module):
+    if is_plain(module):
         return linear_weight(x, module.weight, module.bias, module)
     return module(x)
 

@@ -24,12 +24,14 @@ import math
 from typing import Optional, Tuple
 
 import torch
+import torch.nn.functional as F
 from torch import Tensor, nn
 
 from . import _lib
-from .linear import linear, linear_weight
+from .linear import is_plain, linear, linear_weight, rows_product
 
-__all__ = ["MambaMixer", "mamba_conv_silu", "selective_scan_mamba", "ConvSiluFn", "MambaScanFn"]
+__all__ = ["MambaMixer", "mamba_conv_silu", "selective_scan_mamba", "ConvSiluFn", "MambaScanFn",
+           "MixerCoreFn"]
 
 
 def _rows(t: Tensor, name: str) -> Tuple[Tensor, int]:
@@ -193,6 +195,13 @@ def selective_scan_mamba(inputs: Tensor, dt: Tensor, A: Tensor, B: Tensor, C: Te
     return MambaScanFn.apply(inputs, dt, A, B, C, gate, dt_bias)
 
 
+def _all_float(xz: Tensor, params) -> bool:
+    """xz and the parameters as they are: plain float32 tensors on one GPU, no autocast."""
+    return (not torch.is_autocast_enabled("cuda") and not torch.compiler.is_compiling()
+            and all(t is None or (type(t) in (Tensor, nn.Parameter) and t.dtype == torch.float32
+                                  and t.device == xz.device) for t in (xz, *params)))
+
+
 class _ColumnSplit(torch.autograd.Function):
     """``xz[..., :d], xz[..., d:]`` as views, whose backward writes the gradient
     of ``xz`` in one pass (torch.cat of the two); slicing the tensor directly
@@ -216,6 +225,78 @@ class _ColumnSplit(torch.autograd.Function):
         if gz is None:
             gz = torch.zeros(*shape[:-1], shape[-1] - d, dtype=ref.dtype, device=ref.device)
         return torch.cat([gx, gz], dim=-1), None
+
+
+class MixerCoreFn(torch.autograd.Function):
+    """The mixer between its in and out projections, ``xz`` [B, L, 2 Di] to
+    ``y`` [B, L, Di]: conv + SiLU, x_proj, dt_proj, the gated scan.  Its backward
+    writes the gradient of ``xz`` and that of x_proj's output in place, part by
+    part (the scan the gate's half, B and C; the conv the x half; a product the dt
+    part), and adds x_proj's into the scan's du in its own product, where separate
+    Functions zero-filled, copied, added and concatenated them: 9 launches and
+    about 90 us of a [256, 200, 64] training step's kernels, and as many host
+    calls."""
+
+    @staticmethod
+    def forward(ctx, xz: Tensor, conv_w: Tensor, conv_b: Optional[Tensor], xproj_w: Tensor,
+                dt_w: Tensor, dt_b: Tensor, A_log: Tensor) -> Tensor:  # type: ignore[override]
+        Di, R, N = dt_w.size(0), dt_w.size(1), A_log.size(1)
+        lib = _lib.load()
+        xz = xz.contiguous()
+        Bz, L, ld = xz.shape
+        w = conv_w.reshape(Di, -1).contiguous()
+        dev, st = xz.device, _lib.stream_of(xz)
+        bias, dtb = _param(conv_b, "conv bias"), dt_b.contiguous()
+        u = torch.empty((Bz, L, Di), dtype=torch.float32, device=dev)
+        with torch.cuda.device(dev):
+            _lib.check(lib.ossm_mamba_conv_forward(xz.data_ptr(), ld, w.data_ptr(), _lib.ptr(bias),
+                                                   u.data_ptr(), Bz, L, Di, w.size(1), st))
+            proj = F.linear(u, xproj_w)
+            dt = F.linear(proj[..., :R], dt_w)  # its bias goes into the softplus
+            A = -torch.exp(A_log)
+            y, raw = torch.empty_like(u), torch.empty_like(u)
+            ck = torch.empty((Bz, Di, int(lib.ossm_selective_num_chunks(L)), 2 * N), dtype=torch.float32,
+                             device=dev)
+            pp, z = proj.data_ptr() + 4 * R, xz.data_ptr() + 4 * Di
+            _lib.check(lib.ossm_selective_mamba_forward(
+                u.data_ptr(), Di, dt.data_ptr(), Di, dtb.data_ptr(), A.data_ptr(), pp, pp + 4 * N,
+                R + 2 * N, z, ld, y.data_ptr(), raw.data_ptr(), ck.data_ptr(), Bz, Di, L, N, st))
+        ctx.save_for_backward(xz, u, proj, dt, A, ck, raw, conv_w, conv_b, xproj_w, dt_w, dt_b)
+        return y
+
+    @staticmethod
+    def backward(ctx, gy: Tensor):  # type: ignore[override]
+        xz, u, proj, dt, A, ck, raw, conv_w, conv_b, xproj_w, dt_w, dt_b = ctx.saved_tensors
+        Di, R, N = dt_w.size(0), dt_w.size(1), A.size(1)
+        Bz, L, ld = xz.shape
+        rows, ldp = Bz * L, R + 2 * N
+        dev, st, lib = xz.device, _lib.stream_of(xz), _lib.load()
+        gy = gy.contiguous()
+        w = conv_w.reshape(Di, -1).contiguous()
+        bias, dtb = _param(conv_b, "conv bias"), dt_b.contiguous()
+        # of xproj_w, dt_w, dt_b, as the forward's arguments are numbered
+        need_xp, need_dtw, need_dtb = ctx.needs_input_grad[3:6]
+        with torch.no_grad(), torch.cuda.device(dev):
+            new = lambda *s: torch.empty(s, dtype=torch.float32, device=dev)  # noqa: E731
+            gxz, gproj, du, ddt = torch.empty_like(xz), torch.empty_like(proj), new(Bz, L, Di), new(Bz, L, Di)
+            dA, gw = new(Di, N), new(Di, w.size(1))
+            gb = new(Di) if bias is not None else None
+            pp, gp = proj.data_ptr() + 4 * R, gproj.data_ptr() + 4 * R
+            _lib.check(lib.ossm_selective_mamba_backward_ld(
+                gy.data_ptr(), u.data_ptr(), Di, dt.data_ptr(), Di, dtb.data_ptr(), A.data_ptr(), pp,
+                pp + 4 * N, ldp, xz.data_ptr() + 4 * Di, ld, ck.data_ptr(), raw.data_ptr(), du.data_ptr(),
+                ddt.data_ptr(), dA.data_ptr(), gp, gp + 4 * N, ldp, gxz.data_ptr() + 4 * Di, ld, Bz, Di, L,
+                N, st))
+            ddt2, gproj2, u2 = ddt.view(rows, Di), gproj.view(rows, ldp), u.view(rows, Di)
+            torch.mm(ddt2, dt_w, out=gproj2[:, :R])
+            du.view(rows, Di).addmm_(gproj2, xproj_w)
+            _lib.check(lib.ossm_mamba_conv_backward_ld(
+                xz.data_ptr(), ld, w.data_ptr(), _lib.ptr(bias), du.data_ptr(), gxz.data_ptr(), ld,
+                gw.data_ptr(), _lib.ptr(gb), Bz, L, Di, w.size(1), st))
+            g_dtw = rows_product(ddt2, proj.view(rows, ldp)[:, :R]) if need_dtw else None
+            g_xp = rows_product(gproj2, u2) if need_xp else None
+            g_dtb = ddt2.sum(0) if need_dtb else None
+            return gxz, gw.view(conv_w.shape), gb, g_xp, g_dtw, g_dtb, dA.mul_(A)
 
 
 # ------------------------------------------------------------------ the mixer
@@ -271,6 +352,10 @@ class MambaMixer(nn.Module):
             raise RuntimeError("the fused Mamba mixer runs on the GPU only")
         Di, R, N = self.d_inner, self.dt_rank, self.d_state
         xz = linear(self.in_proj, inputs).float()
+        params = (self.conv1d.weight, self.conv1d.bias, self.x_proj.weight, self.dt_proj.weight,
+                  self.dt_proj.bias, self.A_log)
+        if is_plain(self.x_proj) and self.x_proj.bias is None and xz.numel() > 0 and _all_float(xz, params):
+            return linear(self.out_proj, MixerCoreFn.apply(xz, *params))
         x, z = _ColumnSplit.apply(xz, Di)                 # views, row stride 2 * d_inner
         x_conv = mamba_conv_silu(x, self.conv1d.weight.float(),
                                  None if self.conv1d.bias is None else self.conv1d.bias.float())

@@ -254,3 +254,43 @@ def test_mamba_edge_cases_and_errors(M):
     e = torch.zeros(2, 0, 8, device="cuda")
     assert M.mamba_conv_silu(e, torch.randn(8, 1, 4, device="cuda")).shape == e.shape
     no_device_errors()
+
+
+# rows below and above the row-product rule, d_inner not a multiple of 4 and
+# R + 2N not either (element-wise stores), one state, more states than one pass
+@pytest.mark.parametrize("shape", [(1, 1, 4, 1, 4, True), (2, 37, 6, 5, 3, False), (3, 200, 16, 16, 4, True),
+                                   (2, 300, 33, 17, 2, True)], ids=lambda s: "x".join(map(str, s)))
+def test_mixer_core_matches_separate_functions(M, shape, monkeypatch):
+    """The mixer's fused middle (strided gradients) against the separate conv,
+    linear and scan Functions on the same inputs: the same kernels, with sums in
+    another order in the products (float32: 1e-5 of each result's scale); frozen
+    parameters get no gradient; a hooked x_proj is still called."""
+    nb, L, d_model, N, K, conv_bias = shape
+    torch.manual_seed(L + N)
+    mixer = M.MambaMixer(d_model, d_state=N, d_conv=K, expand=1 if d_model == 33 else 2, dt_rank=3,
+                         conv_bias=conv_bias).cuda()
+    x = torch.randn(nb, L, d_model, device="cuda", requires_grad=True)
+    go = torch.randn(nb, L, d_model, device="cuda")
+    announce(f"mixer core {shape}")
+
+    def run():
+        wrt = [x, *[p for p in mixer.parameters() if p.requires_grad]]
+        y = mixer(x)
+        return [y, *torch.autograd.grad(y, wrt, go)]
+
+    got = run()
+    with torch.no_grad():
+        assert torch.equal(mixer(x), got[0])
+    mixer.x_proj.weight.requires_grad_(False)
+    assert len(run()) == len(got) - 1
+    mixer.x_proj.weight.requires_grad_(True)
+    calls = []
+    handle = mixer.x_proj.register_forward_hook(lambda *a: calls.append(1))
+    mixer(x)
+    handle.remove()
+    assert calls == [1]
+    monkeypatch.setattr(M, "_all_float", lambda *a: False)
+    for g, r in zip(got, run()):
+        g, r = to_np(g), to_np(r)
+        np.testing.assert_allclose(g, r, rtol=1e-4, atol=1e-5 * max(1.0, float(np.abs(r).max())))
+    no_device_errors()
