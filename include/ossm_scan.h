@@ -523,7 +523,9 @@ int ossm_layer_params_backward(int damped, const float* A_diag, const float* G_d
 /*
  * ossm_dlinoss_layer_forward / _backward with params_lo [3][ssm] (may be null): what
  * a_diag, g_diag and step leave of their double values.  With it the oscillators'
- * coefficients are formed from the sums in double and rounded once.
+ * coefficients are formed from the sums in double and rounded once.  The backward
+ * also gives grad_d [hidden], the gradient of D (may be null), where hidden rounded
+ * up to 32 is a power of two.
  */
 int ossm_dlinoss_layer_forward_wide(int variant, const float* inputs, const float* B, const float* C,
                                     const float* D, const float* a_diag, const float* g_diag,
@@ -535,8 +537,8 @@ int ossm_dlinoss_layer_backward_wide(int variant, const float* inputs, const flo
                                      const float* a_diag, const float* g_diag, const float* step,
                                      const float* params_lo, const void* carries, float* grad_inputs,
                                      void* grad_bu, void* x_conj, float* grad_a, float* grad_g,
-                                     float* grad_step, int64_t batch, int64_t length, int64_t hidden,
-                                     int64_t ssm, ossm_stream_t stream);
+                                     float* grad_step, float* grad_d, int64_t batch, int64_t length,
+                                     int64_t hidden, int64_t ssm, ossm_stream_t stream);
 
 /*
  * out(i, j) = sum_r a[r, i] b[r, j] over row-major a [rows, m] (row stride ld_a) and

@@ -111,7 +111,7 @@ _SIGNATURES = {
          _c_int64, _vp]),
     "ossm_dlinoss_layer_backward_wide": (
         ctypes.c_int,
-        [ctypes.c_int, _fp, _fp, _fp, _fp, _fp, _fp, _fp, _fp, _fp, _vp, _fp, _vp, _vp, _fp, _fp, _fp,
+        [ctypes.c_int, _fp, _fp, _fp, _fp, _fp, _fp, _fp, _fp, _fp, _vp, _fp, _vp, _vp, _fp, _fp, _fp, _fp,
          _c_int64, _c_int64, _c_int64, _c_int64, _vp]),
     "ossm_selective_mamba_forward": (
         ctypes.c_int,

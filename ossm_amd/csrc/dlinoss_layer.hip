@@ -14,7 +14,8 @@
 // Decomposition: one workgroup (4 waves) per (batch row b, 32-step chunk).
 //   1. The chunk's u rows (contiguous in HBM) are staged in LDS.
 //   2. In-projection on the matrix cores, v_mfma_f32_32x32x2f32 (fp32 products
-//      and sums, no reduced precision): the 32 x 2P result (re and im planes)
+//      and sums) or, on larger problems, the same precision from six bf16
+//      products of split operands (SPLIT, split_mfma.hpp: 2.7 times the rate): the 32 x 2P result (re and im planes)
 //      waits in the accumulators until every wave has read u, then replaces
 //      u in LDS (one buffer: four workgroups share a CU at H, P <= 128).
 //      Wave w owns oscillator groups w, w+4, ... of 32; its lanes read the
@@ -51,11 +52,10 @@
 #include "runtime.hpp"
 #include "scan_device.hpp"
 #include "dlinoss_model.hpp"
+#include "split_mfma.hpp"
 
 namespace ossm {
 namespace {
-
-typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int kLc = 32;            // time steps per chunk = MFMA tile rows
 constexpr int kLayerWaves = 4;
@@ -88,6 +88,8 @@ struct LayerArgs {
   const float* g;
   const float* dt;
   const float* lo;  // [3, P]: what a, g, dt leave of their double values; may be null
+  const uint4* w_in;   // SPLIT: split weights of the in- and out-projection (SplitW)
+  const uint4* w_out;
   float* y;         // [B, L, H]
   float4* carries;  // [B, n_chunks, P]: state entering each chunk (for the backward); may be null
   int Bsz, L, H, P, n_chunks;
@@ -210,13 +212,114 @@ __device__ __forceinline__ void stage_store(const RowStage<SK>& r, float* __rest
   }
 }
 
+// ---- split-bf16 projections (SPLIT kernels) ---------------------------------
+// The projections on the bf16 matrix cores with float32 precision
+// (split_mfma.hpp).  The weights are split once per call by
+// split_weights_kernel into the order the lanes read them: for column group
+// cg of 32, k-step s of 16 and component c, term t (0, 1, 2) of lane l's eight
+// values k = 16 s + 8 (l / 32) + j, j = 0..7, at uint4 [((cg S + s) NC + c) 3 + t]
+// [l]; columns and k outside the tensor hold zeros, so the loops need no masks.
+// "in" form: column p, k = h, components re and im (NC = 2); "out" form: column
+// h, k = 2 p + component (NC = 1).
+struct SplitW {
+  const float* w;
+  uint4* out;
+  int w_is_c;  // C [H, P, 2], else B [P, H, 2]
+  int in_form;
+};
+
+__device__ __forceinline__ float weight_at(const SplitW& g, int H, int P, int h, int p, int c) {
+  if (h >= H || p >= P) return 0.f;
+  return g.w[(g.w_is_c ? static_cast<size_t>(h) * P + p : static_cast<size_t>(p) * H + h) * 2 + c];
+}
+
+constexpr int kSplitThreads = 256;
+
+// uint4 of one split matrix (either form)
+__host__ __device__ __forceinline__ size_t split_w_uint4(int H, int P) {
+  const size_t Hp = (H + 31) / 32 * 32, Pp = (P + 31) / 32 * 32;
+  return Hp * Pp * 2 / 8 * 3;
+}
+
+__global__ __launch_bounds__(kSplitThreads) void split_weights_kernel(SplitW g0, SplitW g1, SplitW g2,
+                                                                      int H, int P) {
+  const SplitW g = blockIdx.y == 0 ? g0 : (blockIdx.y == 1 ? g1 : g2);
+  const int Hp = round32(H), Pp = round32(P);
+  const int i = static_cast<int>(blockIdx.x) * kSplitThreads + static_cast<int>(threadIdx.x);
+  if (i >= Hp * Pp / 4) return;  // 8 values each
+  const int l = i % kWave, b = i / kWave;
+  const int col = l & 31, k0 = 8 * (l >> 5);
+  float v[8];
+  if (g.in_form) {
+    const int c = b & 1, s = (b >> 1) % (Hp / 16), cg = (b >> 1) / (Hp / 16);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = weight_at(g, H, P, 16 * s + k0 + j, cg * 32 + col, c);
+  } else {
+    const int s = b % (Pp / 8), cg = b / (Pp / 8);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = weight_at(g, H, P, cg * 32 + col, 8 * s + (k0 + j) / 2, j & 1);
+  }
+  const SplitFrag f = split8(v);
+  uint4* dst = g.out + static_cast<size_t>(b) * 3 * kWave + l;
+  dst[0] = __builtin_bit_cast(uint4, f.t0);
+  dst[kWave] = __builtin_bit_cast(uint4, f.t1);
+  dst[2 * kWave] = __builtin_bit_cast(uint4, f.t2);
+}
+
+// acc[c] += A (32 rows, fp32 in LDS; arow: the lane's row from its first k) times
+// the split weights of one column group over S k-steps.  Weights AH steps ahead.
+template <int NC, int AH>
+__device__ __forceinline__ void split_project(const float* arow, const uint4* __restrict__ w, int S,
+                                              floatx16 (&acc)[NC]) {
+  constexpr int kStep = NC * 3 * kWave;
+  w += threadIdx.x & (kWave - 1);
+  uint4 wb[AH][NC][3];
+#pragma unroll
+  for (int a = 0; a < AH; ++a)
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int t = 0; t < 3; ++t) wb[a][c][t] = w[a * kStep + (c * 3 + t) * kWave];
+  float4 n0 = *reinterpret_cast<const float4*>(arow), n1 = *reinterpret_cast<const float4*>(arow + 4);
+  for (int s0 = 0; s0 < S; s0 += AH) {
+#pragma unroll
+    for (int a = 0; a < AH; ++a) {
+      const int s = s0 + a;
+      const float x[8] = {n0.x, n0.y, n0.z, n0.w, n1.x, n1.y, n1.z, n1.w};
+      const float* nx = arow + 16 * min(s + 1, S - 1);
+      n0 = *reinterpret_cast<const float4*>(nx);
+      n1 = *reinterpret_cast<const float4*>(nx + 4);
+      const SplitFrag fa = split8(x);
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const SplitFrag fw{__builtin_bit_cast(bf16x8, wb[a][c][0]), __builtin_bit_cast(bf16x8, wb[a][c][1]),
+                           __builtin_bit_cast(bf16x8, wb[a][c][2])};
+        acc[c] = mfma_split(fa, fw, acc[c]);
+      }
+      const uint4* nw = w + static_cast<size_t>(min(s + AH, S - 1)) * kStep;
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int t = 0; t < 3; ++t) wb[a][c][t] = nw[(c * 3 + t) * kWave];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+}
+
 // SMALL: Hp, Pp <= 128 (one oscillator group per wave, four row groups per
 // thread): the registers are sized for that, so that four workgroups share a CU.
+// SPLIT: split-bf16 projections (use_split).  A operands are split as they are read
+// from LDS, 44 VALU per step and wave next to 12 (in) or 6 (out) matrix
+// instructions of 32 cycles; weights come split, one step ahead where SMALL caps
+// the registers (two steps ahead spill 25 there: 176 against 162 us at
+// [32, 4096, 128, 128]; three waves per SIMD instead of the cap 166).  What is left
+// besides the 41 us of matrix instructions: splitting, the weights' L2 latency
+// and the serial scan and look-back of each workgroup.
 // PAD: H or P is not a multiple of 32, so the projections' padded rows and
 // columns read clamped weights that mask_* zeroes; without padding every weight
 // is in range and the loops consume the loads as they are (a select on a loaded
 // value is where the compiler puts the wait for it).
-template <int V, bool VEC, bool SMALL, bool PAD>
+template <int V, bool VEC, bool SMALL, bool PAD, bool SPLIT>
 __global__ __launch_bounds__(kLayerThreads) __attribute__((amdgpu_waves_per_eu(SMALL ? 4 : 1)))
 void dlinoss_layer_fwd_kernel(
     LayerArgs A, unsigned long long* __restrict__ rec, LaunchSync sync) {
@@ -267,6 +370,14 @@ void dlinoss_layer_fwd_kernel(
       const int p = pg * 32 + m;
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc_re[i][r] = acc_im[i][r] = 0.f;
+      if constexpr (SPLIT) {
+        floatx16 acc[2] = {acc_re[i], acc_im[i]};
+        const int S = Hp / 16;
+        split_project<2, SMALL ? 1 : 2>(sU + m * HS + 8 * half, A.w_in + static_cast<size_t>(pg) * S * 6 * kWave, S, acc);
+        acc_re[i] = acc[0];
+        acc_im[i] = acc[1];
+        continue;
+      }
       float4 wb[AH][2];
 #pragma unroll
       for (int j = 0; j < AH; ++j) load_bw<VEC>(A.Bw, A.H, A.P, p, half * hh + 4 * j, wb[j]);
@@ -383,6 +494,12 @@ void dlinoss_layer_fwd_kernel(
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         uv[r] = A.u[row0 + static_cast<size_t>(min(acc_row(r, lane), nt - 1)) * A.H + min(h, A.H - 1)];
+      if constexpr (SPLIT) {
+        floatx16 one[1] = {acc};
+        const int S = Pp / 8;
+        split_project<1, SMALL ? 1 : 2>(sX + m * XS + 8 * kk, A.w_out + static_cast<size_t>(hg) * S * 3 * kWave, S, one);
+        acc = one[0];
+      } else {
       float4 cb[AH];
 #pragma unroll
       for (int j = 0; j < AH; ++j) cb[j] = load_cw<VEC>(A.Cw, A.H, A.P, h, 4 * j + 2 * kk);
@@ -405,6 +522,7 @@ void dlinoss_layer_fwd_kernel(
           acc = mfma32(av.w, cv.w, acc);
           __builtin_amdgcn_sched_barrier(0);  // groups stay in program order (prefetch distance)
         }
+      }
       }
       if (h < A.H) {
         const float dh = A.Dw[h];
@@ -448,11 +566,15 @@ struct LayerBwdArgs {
   const float* g;
   const float* dt;
   const float* lo;       // as LayerArgs::lo
+  const uint4* w_gx;     // SPLIT: split weights of the g_x, bu and grad_u projections
+  const uint4* w_bu;
+  const uint4* w_gu;
   const float4* carries; // [B, n_chunks, P] from the forward
   float* grad_u;         // [B, L, H]
   float2* grad_bu;       // [B, L, P] (re, im)
   float2* xq;            // [B, L, P] (x.re, -x.im)
   float* partials;       // [n_chunks][NS][B * P]
+  float* part_d;         // [workgroup][H]: sums of gy u over the chunk's steps, or null
   ZeroFill zero;         // grad a, g, dt, cleared by the first workgroup
   int Bsz, L, H, P, n_chunks;
 };
@@ -501,13 +623,14 @@ __device__ __forceinline__ float4 mask_bw_pair(int H, int P, int h, int p0, floa
 }
 
 // PAD: as for the forward (H or P not a multiple of 32: weights masked where used).
-template <int V, bool VEC, bool PAD>
+template <int V, bool VEC, bool PAD, bool SPLIT>
 __global__ __launch_bounds__(kLayerThreads) void dlinoss_layer_bwd_kernel(
     LayerBwdArgs A, unsigned long long* __restrict__ rec, LaunchSync sync) {
   using Model = Dlinoss<V>;
   constexpr int NS = Model::kSums;
   extern __shared__ __align__(16) float smem[];
   __shared__ int s_ticket;
+  __shared__ __align__(16) float s_d[kLayerWaves][kLayerMax];
 
   const int Hp = round32(A.H), Pp = round32(A.P);
   const int HS = Hp + 4, XS = 2 * Pp + 4;
@@ -550,6 +673,13 @@ __global__ __launch_bounds__(kLayerThreads) void dlinoss_layer_bwd_kernel(
       floatx16 acc_re, acc_im;
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc_re[r] = acc_im[r] = 0.f;
+      if constexpr (SPLIT) {
+        floatx16 acc[2] = {acc_re, acc_im};
+        const int S = Hp / 16;
+        split_project<2, 2>(sA + m * HS + 8 * half, A.w_gx + static_cast<size_t>(pg) * S * 6 * kWave, S, acc);
+        acc_re = acc[0];
+        acc_im = acc[1];
+      } else {
       float4 wb[kAhead][2];
 #pragma unroll
       for (int j = 0; j < kAhead; ++j) load_cw_pair<VEC>(A.Cw, A.H, A.P, half * hh + 4 * j, p, wb[j]);
@@ -579,6 +709,7 @@ __global__ __launch_bounds__(kLayerThreads) void dlinoss_layer_bwd_kernel(
           __builtin_amdgcn_sched_barrier(0);  // groups stay in program order (prefetch distance)
         }
       }
+      }
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int t = acc_row(r, lane);
@@ -589,9 +720,30 @@ __global__ __launch_bounds__(kLayerThreads) void dlinoss_layer_bwd_kernel(
   __syncthreads();
 
   // 2. u -> LDS (over gy); bu on the matrix cores, held in the accumulators
-  //    until every wave has read u, then written to sX over it
+  //    until every wave has read u, then written to sX over it.  Where u
+  //    replaces gy the thread holds both: its share of grad_D = sum gy u.
+  if (A.part_d != nullptr) {
+    const int q4 = Hp / 4;  // a power of two: the thread's columns are the same in every group
+    float4 d = f4zero();
+#pragma unroll
+    for (int k = 0; k < kLayerMax / 32; ++k) {
+      if (k >= Hp / 32) break;  // uniform
+      const int e = threadIdx.x + k * kLayerThreads, t = e / q4;
+      const float4 gv = *reinterpret_cast<const float4*>(sA + t * HS + (e - t * q4) * 4);
+      const float4 uv = st_u.v[k];
+      if (t < nt) d = make_float4(d.x + gv.x * uv.x, d.y + gv.y * uv.y, d.z + gv.z * uv.z, d.w + gv.w * uv.w);
+    }
+    for (int o = q4; o < kWave; o *= 2)
+      d = make_float4(d.x + __shfl_xor(d.x, o), d.y + __shfl_xor(d.y, o), d.z + __shfl_xor(d.z, o),
+                      d.w + __shfl_xor(d.w, o));
+    if (lane < q4) *reinterpret_cast<float4*>(s_d[w] + 4 * lane) = d;
+  }
   stage_store(st_u, sA, nt, A.H, Hp, HS);
   __syncthreads();
+  if (A.part_d != nullptr && static_cast<int>(threadIdx.x) < A.H) {
+    const int h = threadIdx.x;
+    A.part_d[static_cast<size_t>(ticket) * A.H + h] = s_d[0][h] + s_d[1][h] + s_d[2][h] + s_d[3][h];
+  }
   {
     const float* arow = sA + m * HS + half * hh;
     floatx16 acc_re[kBwdGroups], acc_im[kBwdGroups];
@@ -602,6 +754,14 @@ __global__ __launch_bounds__(kLayerThreads) void dlinoss_layer_bwd_kernel(
       const int p = pg * 32 + m;
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc_re[i][r] = acc_im[i][r] = 0.f;
+      if constexpr (SPLIT) {
+        floatx16 acc[2] = {acc_re[i], acc_im[i]};
+        const int S = Hp / 16;
+        split_project<2, 2>(sA + m * HS + 8 * half, A.w_bu + static_cast<size_t>(pg) * S * 6 * kWave, S, acc);
+        acc_re[i] = acc[0];
+        acc_im[i] = acc[1];
+        continue;
+      }
       float4 wb[kAhead][2];
 #pragma unroll
       for (int j = 0; j < kAhead; ++j) load_bw<VEC>(A.Bw, A.H, A.P, p, half * hh + 4 * j, wb[j]);
@@ -732,6 +892,12 @@ __global__ __launch_bounds__(kLayerThreads) void dlinoss_layer_bwd_kernel(
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         gyv[r] = A.gy[row0 + static_cast<size_t>(min(acc_row(r, lane), nt - 1)) * A.H + min(h, A.H - 1)];
+      if constexpr (SPLIT) {
+        floatx16 one[1] = {acc};
+        const int S = Pp / 8;
+        split_project<1, 2>(sG + m * XS + 8 * kk, A.w_gu + static_cast<size_t>(hg) * S * 3 * kWave, S, one);
+        acc = one[0];
+      } else {
       float4 cb[kAhead];
 #pragma unroll
       for (int j = 0; j < kAhead; ++j) cb[j] = load_bw_pair(A.Bw, A.H, A.P, h, 4 * j + 2 * kk);
@@ -755,6 +921,7 @@ __global__ __launch_bounds__(kLayerThreads) void dlinoss_layer_bwd_kernel(
           __builtin_amdgcn_sched_barrier(0);  // groups stay in program order (prefetch distance)
         }
       }
+      }
       if (h < A.H) {
         const float dh = A.Dw[h];
 #pragma unroll
@@ -765,6 +932,47 @@ __global__ __launch_bounds__(kLayerThreads) void dlinoss_layer_bwd_kernel(
       }
     }
   }
+}
+
+// grad_D[h] = the workgroups' sums: 16 columns by 16 row lanes, in order, in double.
+__global__ __launch_bounds__(256) void layer_grad_d_kernel(const float* __restrict__ part, float* __restrict__ out,
+                                                           int rows, int H) {
+  __shared__ double s_p[16][16];
+  const int cl = threadIdx.x & 15, rl = threadIdx.x >> 4, h = blockIdx.x * 16 + cl;
+  double s = 0.0;
+  if (h < H) {
+#pragma unroll 8
+    for (int r = rl; r < rows; r += 16) s += part[static_cast<size_t>(r) * H + h];
+  }
+  s_p[rl][cl] = s;
+  __syncthreads();
+  if (rl != 0 || h >= H) return;
+#pragma unroll
+  for (int v = 1; v < 16; ++v) s += s_p[v][cl];
+  out[h] = static_cast<float>(s);
+}
+
+int launch_split_weights(const SplitW& g0, const SplitW& g1, const SplitW& g2, int n, int H, int P,
+                         hipStream_t stream) {
+  const int items = (H + 31) / 32 * 32 * ((P + 31) / 32 * 32) / 4;
+  hipLaunchKernelGGL(split_weights_kernel,
+                     dim3(static_cast<unsigned>((items + kSplitThreads - 1) / kSplitThreads),
+                          static_cast<unsigned>(n)),
+                     dim3(kSplitThreads), 0, stream, g0, g1, g2, H, P);
+  return launch_check("split_weights_kernel");
+}
+
+// Whether the projections run split: from `floor` of rows x padded H x padded P on,
+// where their matrix-core time pays for the extra launch that splits the weights.
+// Kernels, fp32 -> split, us, at [B, L, H, P] (rows Hp Pp in millions):
+//   forward   [2, 500, 64, 64] (4) 16.0 -> 18.1; [8, 1024, 64, 64] (34) 20.0 -> 21.7;
+//             [8, 1030, 100, 64] (68) 26.5 -> 25.3, a launch more on the host;
+//             [16, 2048, 200, 100] (940) 118 -> 83; [8, 4096, 256, 256] (2147)
+//             218 -> 142; [32, 4096, 128, 128] (2147) 240 -> 162
+//   backward  26.2 -> 25.7; 32.2 -> 31.5; 46.8 -> 36.9; 181 -> 120; 385 -> 277; 418 -> 295
+constexpr int64_t kSplitFwd = int64_t(1) << 27, kSplitBwd = int64_t(1) << 25;
+bool use_split(int64_t rows, int64_t H, int64_t P, int64_t floor) {
+  return P > 0 && rows * ((H + 31) / 32 * 32) * ((P + 31) / 32 * 32) >= floor;
 }
 
 template <class Model>
@@ -783,7 +991,7 @@ size_t layer_bwd_lds_bytes(int64_t H, int64_t P) {
 constexpr size_t kMaxLds = 160 * 1024;
 
 template <int V>
-int launch_layer_bwd(LayerBwdArgs args, float* ga, float* gg, float* gs, hipStream_t stream) {
+int launch_layer_bwd(LayerBwdArgs args, float* ga, float* gg, float* gs, float* grad_d, hipStream_t stream) {
   StreamCall call(stream);
   if (call.status()) return call.status();
   using Model = Dlinoss<V>;
@@ -794,15 +1002,41 @@ int launch_layer_bwd(LayerBwdArgs args, float* ga, float* gg, float* gs, hipStre
   void* payload = nullptr;
   LaunchSync sync{};
   void* ws = nullptr;
-  if (int rc = acquire_workspace(call, static_cast<size_t>(args.n_chunks) * NS * nc * sizeof(float), &ws))
-    return rc;
+  // partial sums (parameters, then grad_D), then (split) the three weight matrices
+  const size_t n_part = static_cast<size_t>(args.n_chunks) * NS * nc;
+  const size_t n_part_d = grad_d != nullptr ? static_cast<size_t>(n_wg) * args.H : 0;
+  const size_t part_bytes = ((n_part + n_part_d) * sizeof(float) + 15) & ~size_t(15);
+  const size_t w_uint4 = split_w_uint4(args.H, args.P);
+  bool split = use_split(static_cast<int64_t>(args.Bsz) * args.L, args.H, args.P, kSplitBwd);
+  if (split) {
+    if (acquire_workspace(call, part_bytes + 3 * w_uint4 * sizeof(uint4), &ws)) {
+      // e.g. under capture, where it may not grow: the fp32 projections need none
+      (void)hipGetLastError();
+      clear_error();
+      split = false;
+    }
+  }
+  if (!split)
+    if (int rc = acquire_workspace(call, part_bytes, &ws)) return rc;
   args.partials = static_cast<float*>(ws);
+  args.part_d = grad_d != nullptr ? args.partials + n_part : nullptr;
+  if (split) {
+    auto* w = reinterpret_cast<uint4*>(static_cast<char*>(ws) + part_bytes);
+    args.w_gx = w;
+    args.w_bu = w + w_uint4;
+    args.w_gu = w + 2 * w_uint4;
+    if (int rc = launch_split_weights({args.Cw, w, 1, 1}, {args.Bw, w + w_uint4, 0, 1},
+                                      {args.Bw, w + 2 * w_uint4, 0, 0}, 3, args.H, args.P, stream))
+      return rc;
+  }
   args.zero = ZeroFill{{ga, gg, gs}, {args.P, args.P, args.P}};
   const bool vec = args.H % 4 == 0 && args.P % 4 == 0 && aligned16(args.u) && aligned16(args.gy) &&
                    aligned16(args.Bw) && aligned16(args.Cw);
   const bool pad = args.H % 32 != 0 || args.P % 32 != 0;
-  auto kern = vec ? (pad ? dlinoss_layer_bwd_kernel<V, true, true> : dlinoss_layer_bwd_kernel<V, true, false>)
-                  : (pad ? dlinoss_layer_bwd_kernel<V, false, true> : dlinoss_layer_bwd_kernel<V, false, false>);
+  auto kern = vec ? (pad ? dlinoss_layer_bwd_kernel<V, true, true, false> : dlinoss_layer_bwd_kernel<V, true, false, false>)
+                  : (pad ? dlinoss_layer_bwd_kernel<V, false, true, false> : dlinoss_layer_bwd_kernel<V, false, false, false>);
+  if (split)
+    kern = vec ? dlinoss_layer_bwd_kernel<V, true, false, true> : dlinoss_layer_bwd_kernel<V, false, false, true>;
   const size_t lds = layer_bwd_lds_bytes(args.H, args.P);
   // before the ticket reservation: a failure here leaves nothing reserved
   if (int rc = hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -814,6 +1048,11 @@ int launch_layer_bwd(LayerBwdArgs args, float* ga, float* gg, float* gs, hipStre
   hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(n_wg)), dim3(kLayerThreads), lds, stream, args,
                      static_cast<unsigned long long*>(payload), sync);
   if (int rc = launch_check("dlinoss_layer_bwd_kernel")) return rc;
+  if (grad_d != nullptr) {
+    hipLaunchKernelGGL(layer_grad_d_kernel, dim3(static_cast<unsigned>((args.H + 15) / 16)), dim3(256), 0, stream,
+                       args.part_d, grad_d, static_cast<int>(n_wg), args.H);
+    if (int rc = launch_check("layer_grad_d_kernel")) return rc;
+  }
   if (args.P == 0) return OSSM_OK;
   const typename Model::Params prm{args.a, args.g, args.dt, args.P};
   return launch_column_sums<NS>(static_cast<const float*>(ws), args.P, args.Bsz, args.n_chunks,
@@ -827,7 +1066,7 @@ size_t layer_lds_bytes(int64_t H, int64_t P) {
 
 
 template <int V>
-int launch_layer(const LayerArgs& args, hipStream_t stream) {
+int launch_layer(LayerArgs args, hipStream_t stream) {
   StreamCall call(stream);
   if (call.status()) return call.status();
   const int64_t n_wg = static_cast<int64_t>(args.Bsz) * args.n_chunks;
@@ -838,13 +1077,32 @@ int launch_layer(const LayerArgs& args, hipStream_t stream) {
   const bool vec = args.H % 4 == 0 && args.P % 4 == 0 && aligned16(args.u) && aligned16(args.Bw) &&
                    aligned16(args.Cw);
   const bool small = args.H <= 128 && args.P <= 128;
+  bool split = use_split(static_cast<int64_t>(args.Bsz) * args.L, args.H, args.P, kSplitFwd);
+  if (split) {
+    const size_t n = split_w_uint4(args.H, args.P);
+    void* ws = nullptr;
+    if (acquire_workspace(call, 2 * n * sizeof(uint4), &ws)) {
+      // e.g. under capture, where it may not grow: the fp32 projections need none
+      (void)hipGetLastError();
+      clear_error();
+      split = false;
+    } else {
+      auto* w = static_cast<uint4*>(ws);
+      args.w_in = w;
+      args.w_out = w + n;
+      if (int rc = launch_split_weights({args.Bw, w, 0, 1}, {args.Cw, w + n, 1, 0}, {}, 2, args.H, args.P, stream))
+        return rc;
+    }
+  }
   const bool pad = args.H % 32 != 0 || args.P % 32 != 0;
   using K = void (*)(LayerArgs, unsigned long long*, LaunchSync);
   const K kern =
-      vec ? (small ? (pad ? dlinoss_layer_fwd_kernel<V, true, true, true> : dlinoss_layer_fwd_kernel<V, true, true, false>)
-                   : (pad ? dlinoss_layer_fwd_kernel<V, true, false, true> : dlinoss_layer_fwd_kernel<V, true, false, false>))
-          : (small ? (pad ? dlinoss_layer_fwd_kernel<V, false, true, true> : dlinoss_layer_fwd_kernel<V, false, true, false>)
-                   : (pad ? dlinoss_layer_fwd_kernel<V, false, false, true> : dlinoss_layer_fwd_kernel<V, false, false, false>));
+      split ? (vec ? (small ? dlinoss_layer_fwd_kernel<V, true, true, false, true> : dlinoss_layer_fwd_kernel<V, true, false, false, true>)
+                   : (small ? dlinoss_layer_fwd_kernel<V, false, true, false, true> : dlinoss_layer_fwd_kernel<V, false, false, false, true>))
+      : vec ? (small ? (pad ? dlinoss_layer_fwd_kernel<V, true, true, true, false> : dlinoss_layer_fwd_kernel<V, true, true, false, false>)
+                     : (pad ? dlinoss_layer_fwd_kernel<V, true, false, true, false> : dlinoss_layer_fwd_kernel<V, true, false, false, false>))
+            : (small ? (pad ? dlinoss_layer_fwd_kernel<V, false, true, true, false> : dlinoss_layer_fwd_kernel<V, false, true, false, false>)
+                     : (pad ? dlinoss_layer_fwd_kernel<V, false, false, true, false> : dlinoss_layer_fwd_kernel<V, false, false, false, false>));
   const size_t lds = layer_lds_bytes(args.H, args.P);
   // before the ticket reservation: a failure here leaves nothing reserved
   if (int rc = hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -887,7 +1145,7 @@ int ossm_dlinoss_layer_forward_wide(int variant, const float* inputs, const floa
     return set_error(OSSM_ERR_UNSUPPORTED, std::string(what) + ": size exceeds 32-bit indexing");
   if (!inputs || !D || !outputs || (ssm > 0 && (!B || !C || !a_diag || !g_diag || !step)))
     return set_error(OSSM_ERR_INVALID_ARGUMENT, std::string(what) + ": null pointer");
-  LayerArgs args{inputs, B, C, D, a_diag, g_diag, step, params_lo, outputs, static_cast<float4*>(carries),
+  LayerArgs args{inputs, B, C, D, a_diag, g_diag, step, params_lo, nullptr, nullptr, outputs, static_cast<float4*>(carries),
                  static_cast<int>(batch), static_cast<int>(length), static_cast<int>(hidden),
                  static_cast<int>(ssm), static_cast<int>(n_chunks)};
   hipStream_t stream = static_cast<hipStream_t>(stream_v);
@@ -912,8 +1170,8 @@ int ossm_dlinoss_layer_backward_wide(int variant, const float* inputs, const flo
                                      const float* a_diag, const float* g_diag, const float* step,
                                      const float* params_lo, const void* carries, float* grad_inputs,
                                      void* grad_bu, void* x_conj, float* grad_a, float* grad_g,
-                                     float* grad_step, int64_t batch, int64_t length, int64_t hidden,
-                                     int64_t ssm, ossm_stream_t stream_v) {
+                                     float* grad_step, float* grad_d, int64_t batch, int64_t length,
+                                     int64_t hidden, int64_t ssm, ossm_stream_t stream_v) {
   clear_error();
   const char* what = "dlinoss_layer_backward";
   if (batch < 0 || length < 0 || hidden < 0 || ssm < 0)
@@ -927,6 +1185,11 @@ int ossm_dlinoss_layer_backward_wide(int variant, const float* inputs, const flo
   hipStream_t stream = static_cast<hipStream_t>(stream_v);
   if (ssm > 0 && (!grad_a || !grad_g || !grad_step))
     return set_error(OSSM_ERR_INVALID_ARGUMENT, std::string(what) + ": null pointer");
+  const int64_t hp = (hidden + 31) / 32 * 32;
+  if (grad_d != nullptr && (hidden == 0 || (hp & (hp - 1)) != 0))
+    return set_error(OSSM_ERR_UNSUPPORTED, std::string(what) + ": grad_D needs a hidden_dim that pads to a power of two");
+  if (grad_d != nullptr && (batch == 0 || length == 0))
+    if (int rc = fill_zero(grad_d, hidden, stream)) return rc;
   if (batch == 0 || length == 0 || hidden == 0) {
     // no terms: zero parameter gradients (grad_inputs, grad_bu, x_conj are empty
     // or, with hidden == 0, hold no dependence on the scan)
@@ -944,16 +1207,16 @@ int ossm_dlinoss_layer_backward_wide(int variant, const float* inputs, const flo
   if (!inputs || !grad_output || !D || !grad_inputs ||
       (ssm > 0 && (!B || !C || !a_diag || !g_diag || !step || !carries || !grad_bu || !x_conj)))
     return set_error(OSSM_ERR_INVALID_ARGUMENT, std::string(what) + ": null pointer");
-  LayerBwdArgs args{inputs, grad_output, B, C, D, a_diag, g_diag, step, params_lo,
+  LayerBwdArgs args{inputs, grad_output, B, C, D, a_diag, g_diag, step, params_lo, nullptr, nullptr, nullptr,
                     static_cast<const float4*>(carries), grad_inputs,
-                    static_cast<float2*>(grad_bu), static_cast<float2*>(x_conj), nullptr,
+                    static_cast<float2*>(grad_bu), static_cast<float2*>(x_conj), nullptr, nullptr,
                     ZeroFill{}, static_cast<int>(batch), static_cast<int>(length),
                     static_cast<int>(hidden), static_cast<int>(ssm), static_cast<int>(n_chunks)};
   switch (variant) {
-    case OSSM_DLINOSS_IMEX1: return launch_layer_bwd<OSSM_DLINOSS_IMEX1>(args, grad_a, grad_g, grad_step, stream);
-    case OSSM_DLINOSS_IMEX2: return launch_layer_bwd<OSSM_DLINOSS_IMEX2>(args, grad_a, grad_g, grad_step, stream);
-    case OSSM_DLINOSS_IM: return launch_layer_bwd<OSSM_DLINOSS_IM>(args, grad_a, grad_g, grad_step, stream);
-    default: return launch_layer_bwd<OSSM_DLINOSS_EX>(args, grad_a, grad_g, grad_step, stream);
+    case OSSM_DLINOSS_IMEX1: return launch_layer_bwd<OSSM_DLINOSS_IMEX1>(args, grad_a, grad_g, grad_step, grad_d, stream);
+    case OSSM_DLINOSS_IMEX2: return launch_layer_bwd<OSSM_DLINOSS_IMEX2>(args, grad_a, grad_g, grad_step, grad_d, stream);
+    case OSSM_DLINOSS_IM: return launch_layer_bwd<OSSM_DLINOSS_IM>(args, grad_a, grad_g, grad_step, grad_d, stream);
+    default: return launch_layer_bwd<OSSM_DLINOSS_EX>(args, grad_a, grad_g, grad_step, grad_d, stream);
   }
 }
 
@@ -966,7 +1229,7 @@ int ossm_dlinoss_layer_backward(int variant, const float* inputs, const float* g
                                 ossm_stream_t stream) {
   return ossm_dlinoss_layer_backward_wide(variant, inputs, grad_output, B, C, D, a_diag, g_diag, step,
                                           nullptr, carries, grad_inputs, grad_bu, x_conj, grad_a, grad_g,
-                                          grad_step, batch, length, hidden, ssm, stream);
+                                          grad_step, nullptr, batch, length, hidden, ssm, stream);
 }
 
 }  // extern "C"

@@ -205,7 +205,7 @@ def dlinoss_layer_backward(variant: str, inputs: Tensor, grad_output: Tensor, B:
     grad_g, grad_step)`` from the forward's ``carries`` (and
     ``lo``).  One kernel for
     grad_inputs and the scan's parameter gradients; grad_B and grad_C are row
-    products over the grad_bu and conj(x) it returns, grad_D a sum."""
+    products over the grad_bu and conj(x) it returns."""
     variant = variant.lower()
     if variant not in _VARIANTS:
         raise ValueError(f"Unknown D-LinOSS variant '{variant}'.")
@@ -222,13 +222,16 @@ def dlinoss_layer_backward(variant: str, inputs: Tensor, grad_output: Tensor, B:
     gbu = torch.empty((batch, length, ssm, 2), dtype=torch.float32, device=dev)
     xq = torch.empty_like(gbu)
     ga, gg, gs = (torch.empty(ssm, dtype=torch.float32, device=dev) for _ in range(3))
+    padded = -(-hidden // 32) * 32
+    # the kernel sums grad_D where the padded width is a power of two
+    gD = torch.empty(hidden, dtype=torch.float32, device=dev) if hidden and padded & (padded - 1) == 0 else None
     with torch.cuda.device(dev):
         _lib.check(_lib.load().ossm_dlinoss_layer_backward_wide(
             _VARIANTS[variant], u.data_ptr(), go.data_ptr(), Bc.data_ptr(), Cc.data_ptr(),
             Dc.data_ptr(), a.data_ptr(), g.data_ptr(), s.data_ptr(), _lib.ptr(_check_lo(lo, a)),
             carries.data_ptr(),
             gu.data_ptr(), gbu.data_ptr(), xq.data_ptr(), ga.data_ptr(), gg.data_ptr(),
-            gs.data_ptr(), batch, length, hidden, ssm, _lib.stream_of(u)))
+            gs.data_ptr(), _lib.ptr(gD), batch, length, hidden, ssm, _lib.stream_of(u)))
     rows = batch * length
     uf, gof = u.reshape(rows, hidden), go.reshape(rows, hidden)
     # grad_B[p, h, c] = sum_r grad_bu[r, p, c] u[r, h];  grad_C[h, p, c] = sum_r go[r, h] xq[r, p, c]
@@ -239,7 +242,8 @@ def dlinoss_layer_backward(variant: str, inputs: Tensor, grad_output: Tensor, B:
         gB = _sum_rows_product(gbu2, uf).reshape(ssm, 2, hidden).permute(0, 2, 1).contiguous()
         gC = _sum_rows_product(gof, xq2)
     gC = gC.reshape(hidden, ssm, 2)
-    gD = (gof * uf).sum(0)
+    if gD is None:
+        gD = (gof * uf).sum(0)
     return gu, gB, gC, gD, ga, gg, gs
 
 

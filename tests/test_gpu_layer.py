@@ -307,3 +307,38 @@ def test_layer_backward_recompute_path(layers, monkeypatch):
     layers.DlinossLayerFn.apply("imex1", *leaves).backward(to_dev(gy))
     _check_grads([t.grad for t in leaves], args, gy, "imex1", "recompute path")
     no_device_errors()
+
+
+# at and above the sizes where the projections run as split bf16 products:
+# exact tiles, ragged H and P (weights zero-padded by the split), unaligned rows
+# (P or H not a multiple of 4), a short last chunk, grad_D in the kernel (padded H a
+# power of two) and outside it
+SPLIT_SHAPES = [(16, 513, 128, 128), (9, 927, 100, 97), (5, 411, 250, 256), (3, 700, 256, 255),
+                (64, 2050, 20, 30), (40, 1100, 65, 33)]
+
+
+@pytest.mark.parametrize("variant", VARIANTS)
+@pytest.mark.parametrize("shape", SPLIT_SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_layer_split_projections_vs_float64(layers, variant, shape):
+    """Forward and every gradient against the float64 composition (torch products
+    and the complex128 scan).  Damped oscillators: the float32 scan is then within
+    a few 2^-24 per remembered step, 2e-6 of each result's norm."""
+    nb, L, H, P = shape
+    announce(f"layer split {variant} {shape}")
+    g = torch.Generator().manual_seed(L + H)
+    rand = lambda *s: torch.rand(*s, generator=g, dtype=torch.float64)  # noqa: E731
+    args = [torch.randn(nb, L, H, generator=g).double(), (rand(P, H, 2) * 2 - 1) / H ** 0.5,
+            (rand(H, P, 2) * 2 - 1) / P ** 0.5, torch.randn(H, generator=g).double(),
+            0.1 + 0.5 * rand(P), 0.5 + 0.5 * rand(P), 0.2 + 0.3 * rand(P)]
+    args = [t.float() for t in args]
+    go = torch.randn(nb, L, H, generator=g).cuda()
+    f32 = [t.cuda().requires_grad_() for t in args]
+    y = layers.DlinossLayerFn.apply(variant, *f32)
+    got = [y, *torch.autograd.grad(y, f32, go)]
+    f64 = [t.double().cuda().requires_grad_() for t in args]
+    y64 = layers.unfused_layer_forward(variant, *f64)
+    want = [y64, *torch.autograd.grad(y64, f64, go.double())]
+    for x, r, name in zip(got, want, ("y", "u", "B", "C", "D", "a", "g", "step")):
+        err = float((x.detach().double() - r.detach()).norm() / r.detach().norm())
+        assert err < (2e-5 if name in ("a", "g", "step") else 2e-6), f"{name}: {err:.2g}"
+    no_device_errors()
