@@ -487,7 +487,17 @@ int ossm_mamba_conv_backward(const float* x, int64_t ld_x, const float* weight, 
                              int64_t width, ossm_stream_t stream);
 
 /*
- * The two backwards above with strided gradients, so that they can be written into
+ * ossm_diag_scan_forward / _backward (f64 == 0: float32, else float64) with the
+ * eigenvalues as one complex array [state].
+ */
+int ossm_diag_scan_forward_cx(int f64, const void* lambda, const void* b_seq, void* out, int64_t length,
+                              int64_t batch, int64_t state, ossm_stream_t stream);
+int ossm_diag_scan_backward_cx(int f64, const void* lambda, const void* states, const void* grad_output,
+                               void* grad_lambda, void* grad_b, int64_t length, int64_t batch, int64_t state,
+                               ossm_stream_t stream);
+
+/*
+ * The two mixer backwards above with strided gradients, so that they can be written into
  * parts of one tensor: grad_x with row stride ld_grad_x; dgate with ld_dgate, dB and
  * dC with ld_dbc (then a gate is needed and nothing may be empty).
  */

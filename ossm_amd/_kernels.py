@@ -78,10 +78,11 @@ def _on_device(*tensors: Optional[torch.Tensor]) -> None:
     for t in tensors:
         if t is None:
             continue
-        _check(t.is_cuda, "All tensors must be on the same device")
+        index = t.get_device() if t.is_cuda else -1
         if dev is None:
-            dev = t.device
-        _check(t.device == dev, "All tensors must be on the same device")
+            dev = index
+        if index < 0 or index != dev:
+            raise RuntimeError("All tensors must be on the same device")
 
 
 # ------------------------------------------------------------------- D-LinOSS
@@ -99,9 +100,11 @@ def _dlinoss_entry(variant: str, direction: str, bu, coeffs, same_as_bu) -> str:
         raise RuntimeError(f'"dlinoss_{variant}_{direction}_cuda" not implemented for '
                            f"'{_TYPE_NAMES.get(bu.dtype, str(bu.dtype))}'")
     real, suffix = _DLINOSS_ENTRIES[bu.dtype]
-    for t, want in [(c, real) for c in coeffs] + [(c, bu.dtype) for c in same_as_bu]:
-        _check(t.dtype == want, f"expected scalar type {_TYPE_NAMES[want]} but found "
-                                f"{_TYPE_NAMES.get(t.dtype, str(t.dtype))}")
+    for group, want in ((coeffs, real), (same_as_bu, bu.dtype)):
+        for t in group:
+            if t.dtype != want:
+                raise RuntimeError(f"expected scalar type {_TYPE_NAMES[want]} but found "
+                                   f"{_TYPE_NAMES.get(t.dtype, str(t.dtype))}")
     return f"ossm_dlinoss_{direction}{suffix}"
 
 
@@ -123,10 +126,8 @@ def _dlinoss_forward(variant: str, a_diag, g_diag, step, bu):
         return _delegate(f"dlinoss_{variant}_forward", a_diag, g_diag, step, bu)
     _on_device(a_diag, g_diag, step, bu)
     entry = _dlinoss_entry(variant, "forward", bu, (a_diag, g_diag, step), ())
-    with torch.cuda.device(bu.device):
-        _lib.check(getattr(_lib.load(), entry)(
-            _VARIANT_CODE[variant], a_diag.data_ptr(), g_diag.data_ptr(), step.data_ptr(),
-            bu.data_ptr(), output.data_ptr(), length, batch, ssm, _lib.stream_of(bu)))
+    _lib.run(getattr(_lib.load(), entry), bu, _VARIANT_CODE[variant], a_diag.data_ptr(),
+             g_diag.data_ptr(), step.data_ptr(), bu.data_ptr(), output.data_ptr(), length, batch, ssm)
     return output
 
 
@@ -160,12 +161,10 @@ def _dlinoss_backward(variant: str, a_diag, g_diag, step, bu, states, grad_outpu
                          grad_output)
     _on_device(a_diag, g_diag, step, bu, states, grad_output)
     entry = _dlinoss_entry(variant, "backward", bu, (a_diag, g_diag, step), (states, grad_output))
-    with torch.cuda.device(bu.device):
-        _lib.check(getattr(_lib.load(), entry)(
-            _VARIANT_CODE[variant], a_diag.data_ptr(), g_diag.data_ptr(), step.data_ptr(),
-            bu.data_ptr(), states.data_ptr(), grad_output.data_ptr(), grad_a.data_ptr(),
-            grad_g.data_ptr(), grad_step.data_ptr(), grad_bu.data_ptr(), length, batch, ssm,
-            _lib.stream_of(bu)))
+    _lib.run(getattr(_lib.load(), entry), bu, _VARIANT_CODE[variant], a_diag.data_ptr(),
+             g_diag.data_ptr(), step.data_ptr(), bu.data_ptr(), states.data_ptr(),
+             grad_output.data_ptr(), grad_a.data_ptr(), grad_g.data_ptr(), grad_step.data_ptr(),
+             grad_bu.data_ptr(), length, batch, ssm)
     return [grad_a, grad_g, grad_step, grad_bu]
 
 
@@ -213,8 +212,8 @@ def linoss_scan(m11, m12, m21, m22, b_seq):
     output = torch.empty_like(b_seq)
     if b_seq.size(0) == 0:
         return output
-    _check(b_seq.dim() == 4,
-           f"b_seq must have shape (length, batch, ssm_size, 2), got {list(b_seq.shape)}")
+    if b_seq.dim() != 4:
+        raise RuntimeError(f"b_seq must have shape (length, batch, ssm_size, 2), got {list(b_seq.shape)}")
     _check(m11.is_contiguous() and m12.is_contiguous() and m21.is_contiguous()
            and m22.is_contiguous(), "Coefficient tensors must be contiguous")
     _check(b_seq.is_contiguous(), "b_seq must be contiguous")
@@ -225,15 +224,14 @@ def linoss_scan(m11, m12, m21, m22, b_seq):
     _on_device(m11, m12, m21, m22, b_seq)
     # complex64 and complex128, as the reference's device kernel dispatches
     # (AT_DISPATCH_COMPLEX_TYPES, linoss_scan_cuda.cu:139)
-    _check(b_seq.dtype in _LINOSS_ENTRIES,
-           f"linoss_scan: b_seq must be complex64 or complex128, got {b_seq.dtype}")
+    if b_seq.dtype not in _LINOSS_ENTRIES:
+        raise RuntimeError(f"linoss_scan: b_seq must be complex64 or complex128, got {b_seq.dtype}")
     for m in (m11, m12, m21, m22):
         _check(m.dim() == 1 and m.size(0) == ssm, "Coefficient tensors must have shape (ssm_size,)")
         _check(m.dtype == b_seq.dtype, "Coefficient tensors must have b_seq's dtype")
-    with torch.cuda.device(b_seq.device):
-        _lib.check(getattr(_lib.load(), _LINOSS_ENTRIES[b_seq.dtype][0])(
-            m11.data_ptr(), m12.data_ptr(), m21.data_ptr(), m22.data_ptr(), b_seq.data_ptr(),
-            output.data_ptr(), length, batch, ssm, _lib.stream_of(b_seq)))
+    _lib.run(getattr(_lib.load(), _LINOSS_ENTRIES[b_seq.dtype][0]), b_seq, m11.data_ptr(),
+             m12.data_ptr(), m21.data_ptr(), m22.data_ptr(), b_seq.data_ptr(), output.data_ptr(), length,
+             batch, ssm)
     return output
 
 
@@ -257,11 +255,9 @@ def linoss_scan_backward(m11, m12, m21, m22, states, grad_output):
                "Coefficient tensors must be contiguous (ssm_size,) of the states' dtype")
     _check(states.is_contiguous() and grad_output.is_contiguous(),
            "states and grad_output must be contiguous")
-    with torch.cuda.device(states.device):
-        _lib.check(getattr(_lib.load(), _LINOSS_ENTRIES[states.dtype][1])(
-            m11.data_ptr(), m12.data_ptr(), m21.data_ptr(), m22.data_ptr(), states.data_ptr(),
-            grad_output.data_ptr(), grad_m.data_ptr(), grad_b.data_ptr(), length, batch, ssm,
-            _lib.stream_of(states)))
+    _lib.run(getattr(_lib.load(), _LINOSS_ENTRIES[states.dtype][1]), states, m11.data_ptr(),
+             m12.data_ptr(), m21.data_ptr(), m22.data_ptr(), states.data_ptr(), grad_output.data_ptr(),
+             grad_m.data_ptr(), grad_b.data_ptr(), length, batch, ssm)
     return [grad_m, grad_b]
 
 
@@ -353,19 +349,15 @@ def _selective_forward(inputs, dt, A, B, C, gate, dtype, name, skip=None):
     out = torch.empty_like(u) if z is not None else raw
     chunks = torch.empty((batch, dim, _num_chunks(length), dstate * 2), dtype=torch.float32,
                          device=u.device)
-    with torch.cuda.device(u.device):
-        if skip is not None:
-            _lib.check(_lib.load().ossm_selective_forward_skip(
-                _ELEM[dtype], u.data_ptr(), d.data_ptr(), a.data_ptr(), b.data_ptr(), c.data_ptr(),
-                skip.contiguous().data_ptr(), _lib.ptr(z), out.data_ptr(), raw.data_ptr(),
-                chunks.data_ptr(), batch, dim, length, dstate, _lib.stream_of(u)))
-            return [out, chunks, raw]
-        fn = _lib.load().ossm_selective_forward if dtype == torch.float32 else \
-            _lib.load().ossm_selective_forward_bf16
-        _lib.check(fn(
-            u.data_ptr(), d.data_ptr(), a.data_ptr(), b.data_ptr(), c.data_ptr(), _lib.ptr(z),
-            out.data_ptr(), raw.data_ptr(), chunks.data_ptr(), batch, dim, length, dstate,
-            _lib.stream_of(u)))
+    if skip is not None:
+        _lib.run(_lib.load().ossm_selective_forward_skip, u, _ELEM[dtype], u.data_ptr(), d.data_ptr(),
+                 a.data_ptr(), b.data_ptr(), c.data_ptr(), skip.contiguous().data_ptr(), _lib.ptr(z),
+                 out.data_ptr(), raw.data_ptr(), chunks.data_ptr(), batch, dim, length, dstate)
+        return [out, chunks, raw]
+    fn = _lib.load().ossm_selective_forward if dtype == torch.float32 else \
+        _lib.load().ossm_selective_forward_bf16
+    _lib.run(fn, u, u.data_ptr(), d.data_ptr(), a.data_ptr(), b.data_ptr(), c.data_ptr(), _lib.ptr(z),
+             out.data_ptr(), raw.data_ptr(), chunks.data_ptr(), batch, dim, length, dstate)
     return [out, chunks, raw]
 
 
@@ -441,22 +433,17 @@ def _selective_backward(grad_output, inputs, dt, A, B, C, gate, chunk_states, ra
     if z is not None:
         raw = raw_outputs.contiguous() if raw_outputs is not None else \
             _selective_forward(inputs, dt, A, B, C, gate, dtype, name, skip=skip)[2]
-    with torch.cuda.device(u.device):
-        if skip is not None:
-            _lib.check(_lib.load().ossm_selective_backward_skip(
-                _ELEM[dtype], gout.data_ptr(), u.data_ptr(), d.data_ptr(), a.data_ptr(),
-                b.data_ptr(), c.data_ptr(), skip.contiguous().data_ptr(), _lib.ptr(z),
-                cs.data_ptr(), _lib.ptr(raw), du.data_ptr(), ddt.data_ptr(), dA.data_ptr(),
-                dB.data_ptr(), dC.data_ptr(), dD.data_ptr(), dz.data_ptr(), batch, dim, length,
-                dstate, _lib.stream_of(u)))
-            return [du, ddt, dA, dB, dC, dD, dz]
-        fn = _lib.load().ossm_selective_backward if dtype == torch.float32 else \
-            _lib.load().ossm_selective_backward_bf16
-        _lib.check(fn(
-            gout.data_ptr(), u.data_ptr(), d.data_ptr(), a.data_ptr(), b.data_ptr(), c.data_ptr(),
-            _lib.ptr(z), cs.data_ptr(), _lib.ptr(raw), du.data_ptr(), ddt.data_ptr(),
-            dA.data_ptr(), dB.data_ptr(), dC.data_ptr(), dz.data_ptr(), batch, dim, length,
-            dstate, _lib.stream_of(u)))
+    if skip is not None:
+        _lib.run(_lib.load().ossm_selective_backward_skip, u, _ELEM[dtype], gout.data_ptr(), u.data_ptr(),
+                 d.data_ptr(), a.data_ptr(), b.data_ptr(), c.data_ptr(), skip.contiguous().data_ptr(),
+                 _lib.ptr(z), cs.data_ptr(), _lib.ptr(raw), du.data_ptr(), ddt.data_ptr(), dA.data_ptr(),
+                 dB.data_ptr(), dC.data_ptr(), dD.data_ptr(), dz.data_ptr(), batch, dim, length, dstate)
+        return [du, ddt, dA, dB, dC, dD, dz]
+    fn = _lib.load().ossm_selective_backward if dtype == torch.float32 else \
+        _lib.load().ossm_selective_backward_bf16
+    _lib.run(fn, u, gout.data_ptr(), u.data_ptr(), d.data_ptr(), a.data_ptr(), b.data_ptr(), c.data_ptr(),
+             _lib.ptr(z), cs.data_ptr(), _lib.ptr(raw), du.data_ptr(), ddt.data_ptr(), dA.data_ptr(),
+             dB.data_ptr(), dC.data_ptr(), dz.data_ptr(), batch, dim, length, dstate)
     return [du, ddt, dA, dB, dC, dz]
 
 
@@ -481,24 +468,26 @@ def _sdl_param(param: torch.Tensor, name: str, length: int, batch: int, ssm: int
     """normalize_param_view_cpu (sdlinoss_cpu_utils.h:11-72): the (La, Ba, M)
     view of a parameter given as (M,), (L,M), (B,M) or (L|1, B|1, M);
     returns the contiguous float32 view and (La, Ba)."""
-    shape = list(param.shape)
-    _check(1 <= param.dim() <= 3,
-           f"{name} must be shaped as (M,), (L,M), (B,M), or (L,B,M); got {shape}")
-    _check(param.size(-1) == ssm,
-           f"{name} must have size {ssm} along the last dimension; got {shape}")
-    if param.dim() == 1:
+    shape = param.shape
+    dims = len(shape)
+    if not 1 <= dims <= 3:
+        raise RuntimeError(f"{name} must be shaped as (M,), (L,M), (B,M), or (L,B,M); got {list(shape)}")
+    if shape[-1] != ssm:
+        raise RuntimeError(f"{name} must have size {ssm} along the last dimension; got {list(shape)}")
+    if dims == 1:
         la, ba = 1, 1
-    elif param.dim() == 2:
-        if param.size(0) == length:
+    elif dims == 2:
+        if shape[0] == length:
             la, ba = length, 1
-        elif param.size(0) == batch:
+        elif shape[0] == batch:
             la, ba = 1, batch
         else:
-            raise RuntimeError(f"{name} must be shaped as (M,), (L,M), (B,M), or (L,B,M); got {shape}")
+            raise RuntimeError(f"{name} must be shaped as (M,), (L,M), (B,M), or (L,B,M); got {list(shape)}")
     else:
-        _check(param.size(0) in (length, 1) and param.size(1) in (batch, 1),
-               f"{name} must have shape (L,B,M) with optional singleton L/B axes; got {shape}")
-        la, ba = param.size(0), param.size(1)
+        la, ba = shape[0], shape[1]
+        if la not in (length, 1) or ba not in (batch, 1):
+            raise RuntimeError(f"{name} must have shape (L,B,M) with optional singleton L/B axes; "
+                               f"got {list(shape)}")
     return param.contiguous(), la, ba
 
 
@@ -513,11 +502,12 @@ def _sdl_entries(variant: str, direction: str, bu: torch.Tensor, params):
     """The reference's device kernels dispatch complex64 and complex128
     (AT_DISPATCH_COMPLEX_TYPES, sdlinoss_imex1_cuda.cu:232, 271); parameters
     must be the matching real dtype."""
-    _check(bu.dtype in _SDL_ENTRIES,
-           f"sdlinoss_{variant}_{direction}: bu must be complex64 or complex128, got {bu.dtype}")
+    if bu.dtype not in _SDL_ENTRIES:
+        raise RuntimeError(f"sdlinoss_{variant}_{direction}: bu must be complex64 or complex128, got {bu.dtype}")
     real, fwd, bwd = _SDL_ENTRIES[bu.dtype]
     for p, name in params:
-        _check(p.dtype == real, f"{name} must be {real} to match bu ({bu.dtype}); got {p.dtype}")
+        if p.dtype != real:
+            raise RuntimeError(f"{name} must be {real} to match bu ({bu.dtype}); got {p.dtype}")
     return fwd if direction == "forward" else bwd
 
 
@@ -539,10 +529,8 @@ def _sdl_forward(variant: str, A, G, step, bu):
     args = []
     for v, la, ba in views:
         args += [v.data_ptr(), la, ba]
-    with torch.cuda.device(bu.device):
-        _lib.check(getattr(_lib.load(), entry)(
-            _VARIANT_CODE[variant], *args, b.data_ptr(), out.data_ptr(), length, batch, ssm,
-            _lib.stream_of(b)))
+    _lib.run(getattr(_lib.load(), entry), bu, _VARIANT_CODE[variant], *args, b.data_ptr(),
+             out.data_ptr(), length, batch, ssm)
     return out
 
 
@@ -573,11 +561,9 @@ def _sdl_backward(variant: str, A, G, step, bu, states, grad_output):
     args = []
     for v, la, ba in views:
         args += [v.data_ptr(), la, ba]
-    with torch.cuda.device(bu.device):
-        _lib.check(getattr(_lib.load(), entry)(
-            _VARIANT_CODE[variant], *args, b.data_ptr(), states.data_ptr(), grad_output.data_ptr(),
-            grads[0].data_ptr(), grads[1].data_ptr(), grads[2].data_ptr(), grad_bu.data_ptr(),
-            length, batch, ssm, _lib.stream_of(b)))
+    _lib.run(getattr(_lib.load(), entry), bu, _VARIANT_CODE[variant], *args, b.data_ptr(),
+             states.data_ptr(), grad_output.data_ptr(), grads[0].data_ptr(), grads[1].data_ptr(),
+             grads[2].data_ptr(), grad_bu.data_ptr(), length, batch, ssm)
     return grads + [grad_bu]
 
 
@@ -641,8 +627,8 @@ def _diag_lambda(lambda_real, lambda_imag, state: int, dtype):
 
 
 def _diag_entry(dtype, direction: str):
-    _check(dtype in (torch.float32, torch.float64),
-           f"diagonal scan HIP kernel supports float32 and float64, got {dtype}")
+    if dtype not in (torch.float32, torch.float64):
+        raise RuntimeError(f"diagonal scan HIP kernel supports float32 and float64, got {dtype}")
     suffix = "" if dtype == torch.float32 else "_f64"
     return getattr(_lib.load(), f"ossm_diag_scan_{direction}{suffix}")
 
@@ -652,8 +638,8 @@ def _diag_forward(name: str, lambda_real, lambda_imag, b_seq):
     CPU path (:68-92); the GPU result is the same recurrence on the device."""
     if b_seq.size(0) == 0:
         return torch.empty_like(b_seq)
-    _check(b_seq.dim() == 4,
-           f"b_seq must have shape (length, batch, state, 2), got {list(b_seq.shape)}")
+    if b_seq.dim() != 4:
+        raise RuntimeError(f"b_seq must have shape (length, batch, state, 2), got {list(b_seq.shape)}")
     if not b_seq.is_cuda:
         return _delegate(name, lambda_real, lambda_imag, b_seq)
     _check(b_seq.size(-1) == 2, "b_seq must have shape (length, batch, state, 2)")
@@ -663,9 +649,8 @@ def _diag_forward(name: str, lambda_real, lambda_imag, b_seq):
     fn = _diag_entry(b_seq.dtype, "forward")
     b_seq = b_seq.contiguous()
     result = torch.empty_like(b_seq)
-    with torch.cuda.device(b_seq.device):
-        _lib.check(fn(lre.data_ptr(), lim.data_ptr(), b_seq.data_ptr(), result.data_ptr(),
-                      length, batch, state, _lib.stream_of(b_seq)))
+    _lib.run(fn, b_seq, lre.data_ptr(), lim.data_ptr(), b_seq.data_ptr(), result.data_ptr(),
+             length, batch, state)
     return result
 
 
@@ -686,11 +671,46 @@ def _diag_backward(lambda_real, lambda_imag, states, grad_output):
     grad_output = grad_output.contiguous()
     grad_lambda = torch.empty((state, 2), dtype=states.dtype, device=states.device)
     grad_b = torch.empty_like(grad_output)
-    with torch.cuda.device(states.device):
-        _lib.check(fn(lre.data_ptr(), lim.data_ptr(), states.data_ptr(), grad_output.data_ptr(),
-                      grad_lambda.data_ptr(), grad_b.data_ptr(), length, batch, state,
-                      _lib.stream_of(states)))
+    _lib.run(fn, states, lre.data_ptr(), lim.data_ptr(), states.data_ptr(),
+             grad_output.data_ptr(), grad_lambda.data_ptr(), grad_b.data_ptr(), length, batch, state)
     return [grad_lambda, grad_b]
+
+
+def _diag_complex_ok(lam, *tensors) -> bool:
+    """Whether the complex scans below take ``lam`` [P] and ``tensors`` [L, B, P] as
+    they are; anything else goes through the real-view entry points and their checks."""
+    dtype, device = lam.dtype, lam.device
+    if dtype not in (torch.complex64, torch.complex128) or not lam.is_cuda or lam.dim() != 1:
+        return False
+    first = tensors[0]
+    if first.dim() != 3 or first.size(2) != lam.size(0) or first.numel() == 0:
+        return False
+    for t in tensors:
+        if t.dtype != dtype or t.device != device or t.shape != first.shape or t.is_conj() or t.is_neg():
+            return False
+    return not (lam.is_conj() or lam.is_neg())
+
+
+def _diag_complex_forward(lam, b_seq):
+    """The diagonal scan on complex tensors as they lie in memory (see
+    ``_diag_complex_ok``): states [L, B, P]."""
+    lam, b_seq = lam.contiguous(), b_seq.contiguous()
+    length, batch, state = b_seq.shape
+    states = torch.empty_like(b_seq)
+    _lib.run(_lib.load().ossm_diag_scan_forward_cx, b_seq, int(b_seq.dtype == torch.complex128),
+             lam.data_ptr(), b_seq.data_ptr(), states.data_ptr(), length, batch, state)
+    return states
+
+
+def _diag_complex_backward(lam, states, grad_output):
+    """``(grad_lambda [P], grad_b [L, B, P])`` of the above."""
+    lam, states, grad_output = lam.contiguous(), states.contiguous(), grad_output.contiguous()
+    length, batch, state = states.shape
+    grad_lambda, grad_b = torch.empty_like(lam), torch.empty_like(grad_output)
+    _lib.run(_lib.load().ossm_diag_scan_backward_cx, states, int(states.dtype == torch.complex128),
+             lam.data_ptr(), states.data_ptr(), grad_output.data_ptr(), grad_lambda.data_ptr(),
+             grad_b.data_ptr(), length, batch, state)
+    return grad_lambda, grad_b
 
 
 def lru_scan(lambda_real, lambda_imag, b_seq):

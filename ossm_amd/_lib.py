@@ -97,6 +97,10 @@ _SIGNATURES = {
         ctypes.c_int, [_fp, _fp, _vp, _vp, _c_int64, _c_int64, _c_int64, _vp]),
     "ossm_diag_scan_backward_f64": (
         ctypes.c_int, [_fp, _fp, _vp, _vp, _vp, _vp, _c_int64, _c_int64, _c_int64, _vp]),
+    "ossm_diag_scan_forward_cx": (
+        ctypes.c_int, [ctypes.c_int, _vp, _vp, _vp, _c_int64, _c_int64, _c_int64, _vp]),
+    "ossm_diag_scan_backward_cx": (
+        ctypes.c_int, [ctypes.c_int, _vp, _vp, _vp, _vp, _vp, _c_int64, _c_int64, _c_int64, _vp]),
     "ossm_dlinoss_layer_forward": (
         ctypes.c_int,
         [ctypes.c_int, _fp, _fp, _fp, _fp, _fp, _fp, _fp, _fp, _vp, _c_int64, _c_int64, _c_int64,
@@ -194,12 +198,24 @@ def check(rc: int) -> None:
                                "its outputs are not valid")
 
 
+def run(fn, t: torch.Tensor, *args) -> None:
+    """``fn(*args, stream)`` on ``t``'s device and its current stream, checked.  The
+    raw stream handle and the device-index test cost ~0.3 us of a small call's
+    ~15; torch.cuda.device and current_stream, which this replaces, ~4.5."""
+    dev = t.get_device()
+    if dev == torch._C._cuda_getDevice():
+        check(fn(*args, torch._C._cuda_getCurrentRawStream(dev)))
+    else:
+        with torch.cuda.device(dev):
+            check(fn(*args, torch._C._cuda_getCurrentRawStream(dev)))
+
+
 def ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def device_error_bits(device: Optional[torch.device] = None) -> int:

@@ -124,10 +124,10 @@ def _register_ops() -> bool:
 CUSTOM_OPS = _register_ops()
 
 
-def _dlinoss_op(variant: str, direction: str):
-    if CUSTOM_OPS:
-        return getattr(torch.ops.ossm, f"dlinoss_{variant}_{direction}")
-    return getattr(_kernels, f"dlinoss_{variant}_{direction}")
+# the overloads, looked up once: calling the packet resolves them per call
+_DLINOSS_OPS = {(v, d): getattr(torch.ops.ossm, f"dlinoss_{v}_{d}").default if CUSTOM_OPS
+                else getattr(_kernels, f"dlinoss_{v}_{d}")
+                for v in SUPPORTED_VARIANTS for d in ("forward", "backward")}
 
 
 class DlinossFn(torch.autograd.Function):
@@ -138,7 +138,7 @@ class DlinossFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, variant: str, a_diag: Tensor, g_diag: Tensor, step: Tensor,
                 bu: Tensor) -> Tensor:  # type: ignore[override]
-        states = _dlinoss_op(variant, "forward")(a_diag, g_diag, step, bu)
+        states = _DLINOSS_OPS[variant, "forward"](a_diag, g_diag, step, bu)
         ctx.variant = variant
         ctx.save_for_backward(a_diag, g_diag, step, bu, states)
         return states[..., 1]
@@ -146,7 +146,7 @@ class DlinossFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output: Tensor):  # type: ignore[override]
         a_diag, g_diag, step, bu, states = ctx.saved_tensors
-        grad_a, grad_g, grad_step, grad_bu = _dlinoss_op(ctx.variant, "backward")(
+        grad_a, grad_g, grad_step, grad_bu = _DLINOSS_OPS[ctx.variant, "backward"](
             a_diag, g_diag, step, bu, states, grad_output.contiguous())
         return None, grad_a, grad_g, grad_step, grad_bu
 
@@ -347,8 +347,12 @@ class DiagScanFn(torch.autograd.Function):
         if b_seq.size(0) == 0:
             ctx.save_for_backward(lambda_bar, b_seq)
             return b_seq
-        fwd = _kernels.lru_scan if name == "lru" else _kernels.s5_scan
         lam = lambda_bar.resolve_conj()
+        if _kernels._diag_complex_ok(lam, b_seq):
+            states = _kernels._diag_complex_forward(lam, b_seq)
+            ctx.save_for_backward(lambda_bar, states)
+            return states
+        fwd = _kernels.lru_scan if name == "lru" else _kernels.s5_scan
         result = fwd(lam.real.contiguous(), lam.imag.contiguous(),
                      torch.view_as_real(b_seq.contiguous()))
         states = torch.view_as_complex(result)
@@ -361,9 +365,12 @@ class DiagScanFn(torch.autograd.Function):
         if grad_output.size(0) == 0:
             return None, torch.zeros_like(lambda_bar), grad_output
         lam = lambda_bar.resolve_conj()
+        grad_output = grad_output.resolve_conj()
+        if _kernels._diag_complex_ok(lam, states, grad_output):
+            return (None, *_kernels._diag_complex_backward(lam, states, grad_output))
         grad_lambda, grad_b = _kernels.lru_scan_backward(
             lam.real.contiguous(), lam.imag.contiguous(), torch.view_as_real(states),
-            torch.view_as_real(grad_output.resolve_conj().contiguous()))
+            torch.view_as_real(grad_output.contiguous()))
         return None, torch.view_as_complex(grad_lambda), torch.view_as_complex(grad_b)
 
 

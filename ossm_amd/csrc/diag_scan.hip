@@ -248,12 +248,21 @@ __device__ V diag_lookback(unsigned long long* rec, int c, int dir, int n_chunks
   return acc;
 }
 
+// Eigenvalues as two real arrays (stride 1) or one complex array (stride 2, im
+// one element behind re): read in place, where copies of the two parts were two
+// launches per scan and direction, 6 us of its kernels and 20 of its host time.
+template <class R>
+struct Lambda {
+  const R* re;
+  const R* im;
+  int stride;
+};
+
 // The channel's eigenvalue (lanes past the last channel read the last one).
 template <class R>
-__device__ __forceinline__ Cx<R> lane_lambda(const R* lam_re, const R* lam_im, int g, unsigned lc,
-                                             int P) {
-  const unsigned p = (static_cast<unsigned>(g) * kWave + lc) % static_cast<unsigned>(P);
-  return cx(lam_re[p], lam_im[p]);
+__device__ __forceinline__ Cx<R> lane_lambda(const Lambda<R>& lam, int g, unsigned lc, int P) {
+  const size_t p = (static_cast<unsigned>(g) * kWave + lc) % static_cast<unsigned>(P);
+  return cx(lam.re[p * lam.stride], lam.im[p * lam.stride]);
 }
 
 // ============================================================================
@@ -261,8 +270,7 @@ __device__ __forceinline__ Cx<R> lane_lambda(const R* lam_re, const R* lam_im, i
 // ============================================================================
 template <class R, int T, int W>
 __global__ __launch_bounds__(W * kWave) void diag_forward_kernel(
-    const R* __restrict__ lam_re, const R* __restrict__ lam_im, int P,
-    const Cx<R>* __restrict__ in, Cx<R>* __restrict__ out, int L, int nc, int n_groups,
+    Lambda<R> lambda, int P, const Cx<R>* __restrict__ in, Cx<R>* __restrict__ out, int L, int nc, int n_groups,
     int n_chunks, unsigned long long* __restrict__ rec, LaunchSync sync) {
   using V = Cx<R>;
   __shared__ V s_agg[W][kWave];
@@ -277,7 +285,7 @@ __global__ __launch_bounds__(W * kWave) void diag_forward_kernel(
   const int ch = g * kWave + lane;
   const bool active = ch < nc;
   const unsigned lc = clamped_lane(g, nc);
-  const V lam = lane_lambda(lam_re, lam_im, g, lc, P);
+  const V lam = lane_lambda(lambda, g, lc, P);
   const long long t0 = static_cast<long long>(c) * (T * W) + static_cast<long long>(w) * T;
 
   // clamped in-range loads (steps past L and inactive lanes are never stored)
@@ -355,7 +363,7 @@ __global__ __launch_bounds__(W * kWave) void diag_forward_kernel(
 // g_t conj(x_{t-1}) into it.
 template <class R, int T, int W>
 __global__ __launch_bounds__(W * kWave) void diag_backward_kernel(
-    const R* __restrict__ lam_re, const R* __restrict__ lam_im, int P, const Cx<R>* states,
+    Lambda<R> lambda, int P, const Cx<R>* states,
     const Cx<R>* __restrict__ gout, Cx<R>* __restrict__ gin, R* __restrict__ grad_lambda,
     ZeroFill zero, int L, int nc, int n_groups, int n_chunks, unsigned long long* __restrict__ rec,
     LaunchSync sync) {
@@ -375,7 +383,7 @@ __global__ __launch_bounds__(W * kWave) void diag_backward_kernel(
   const int ch = g * kWave + lane;
   const bool active = ch < nc;
   const unsigned lc = clamped_lane(g, nc);
-  const V lamc = cx_conj(lane_lambda(lam_re, lam_im, g, lc, P));
+  const V lamc = cx_conj(lane_lambda(lambda, g, lc, P));
   const long long t0 = static_cast<long long>(c) * (T * W) + static_cast<long long>(w) * T;
 
   // Issue order = order of use: the saved states x_{t-1} first, then the
@@ -536,7 +544,7 @@ int check_diag_sizes(int64_t L, int64_t B, int64_t P, const char* what) {
 }
 
 template <class R>
-int diag_forward_impl(const R* lam_re, const R* lam_im, const void* b_seq, void* out, int64_t L,
+int diag_forward_impl(const Lambda<R>& lambda, const void* b_seq, void* out, int64_t L,
                       int64_t B, int64_t P, hipStream_t stream) {
   StreamCall call(stream);
   if (call.status()) return call.status();
@@ -555,7 +563,7 @@ int diag_forward_impl(const R* lam_re, const R* lam_im, const void* b_seq, void*
 #define OSSM_LAUNCH_DIAG_FWD(TT, WW)                                                              \
   if (!launched && tile.T == TT && tile.W == WW) {                                                \
     hipLaunchKernelGGL((diag_forward_kernel<R, TT, WW>), dim3(static_cast<unsigned>(total)),      \
-                       dim3(WW * kWave), 0, stream, lam_re, lam_im, static_cast<int>(P),          \
+                       dim3(WW * kWave), 0, stream, lambda, static_cast<int>(P),                  \
                        static_cast<const Cx<R>*>(b_seq), static_cast<Cx<R>*>(out),                \
                        static_cast<int>(L), static_cast<int>(nc), static_cast<int>(n_groups),     \
                        static_cast<int>(n_chunks), static_cast<unsigned long long*>(payload), sync); \
@@ -573,7 +581,7 @@ int diag_forward_impl(const R* lam_re, const R* lam_im, const void* b_seq, void*
 }
 
 template <class R>
-int diag_backward_impl(const R* lam_re, const R* lam_im, const void* states, const void* gout,
+int diag_backward_impl(const Lambda<R>& lambda, const void* states, const void* gout,
                        R* grad_lambda, void* grad_b, int64_t L, int64_t B, int64_t P,
                        hipStream_t stream) {
   StreamCall call(stream);
@@ -595,7 +603,7 @@ int diag_backward_impl(const R* lam_re, const R* lam_im, const void* states, con
 #define OSSM_LAUNCH_DIAG_BWD(TT, WW)                                                              \
   if (!launched && tile.T == TT && tile.W == WW) {                                                \
     hipLaunchKernelGGL((diag_backward_kernel<R, TT, WW>), dim3(static_cast<unsigned>(total)),     \
-                       dim3(WW * kWave), 0, stream, lam_re, lam_im, static_cast<int>(P),          \
+                       dim3(WW * kWave), 0, stream, lambda, static_cast<int>(P),                  \
                        static_cast<const Cx<R>*>(states), static_cast<const Cx<R>*>(gout),        \
                        static_cast<Cx<R>*>(grad_b), grad_lambda, zero, static_cast<int>(L),       \
                        static_cast<int>(nc), static_cast<int>(n_groups),                          \
@@ -613,18 +621,18 @@ int diag_backward_impl(const R* lam_re, const R* lam_im, const void* states, con
 }
 
 template <class R>
-int diag_forward_entry(const R* lam_re, const R* lam_im, const void* b_seq, void* out, int64_t L,
+int diag_forward_entry(const Lambda<R>& lambda, const void* b_seq, void* out, int64_t L,
                        int64_t B, int64_t P, ossm_stream_t stream, const char* what) {
   clear_error();
   if (int rc = check_diag_sizes(L, B, P, what)) return rc;
   if (L == 0 || B == 0 || P == 0) return OSSM_OK;
-  if (!lam_re || !lam_im || !b_seq || !out)
+  if (!lambda.re || !lambda.im || !b_seq || !out)
     return set_error(OSSM_ERR_INVALID_ARGUMENT, std::string(what) + ": null pointer");
-  return diag_forward_impl<R>(lam_re, lam_im, b_seq, out, L, B, P, static_cast<hipStream_t>(stream));
+  return diag_forward_impl<R>(lambda, b_seq, out, L, B, P, static_cast<hipStream_t>(stream));
 }
 
 template <class R>
-int diag_backward_entry(const R* lam_re, const R* lam_im, const void* states, const void* gout,
+int diag_backward_entry(const Lambda<R>& lambda, const void* states, const void* gout,
                         void* grad_lambda, void* grad_b, int64_t L, int64_t B, int64_t P,
                         ossm_stream_t stream_v, const char* what) {
   clear_error();
@@ -636,9 +644,9 @@ int diag_backward_entry(const R* lam_re, const R* lam_im, const void* states, co
     return fill_zero(static_cast<float*>(grad_lambda), 2 * P * int64_t(sizeof(R) / sizeof(float)), stream);
   }
   if (L == 0 || B == 0 || P == 0) return OSSM_OK;
-  if (!lam_re || !lam_im || !states || !gout || !grad_lambda || !grad_b)
+  if (!lambda.re || !lambda.im || !states || !gout || !grad_lambda || !grad_b)
     return set_error(OSSM_ERR_INVALID_ARGUMENT, std::string(what) + ": null pointer");
-  return diag_backward_impl<R>(lam_re, lam_im, states, gout, static_cast<R*>(grad_lambda), grad_b,
+  return diag_backward_impl<R>(lambda, states, gout, static_cast<R*>(grad_lambda), grad_b,
                                L, B, P, stream);
 }
 
@@ -652,21 +660,21 @@ extern "C" {
 int ossm_diag_scan_forward(const float* lambda_real, const float* lambda_imag, const void* b_seq,
                            void* out, int64_t length, int64_t batch, int64_t state,
                            ossm_stream_t stream) {
-  return diag_forward_entry<float>(lambda_real, lambda_imag, b_seq, out, length, batch, state,
+  return diag_forward_entry<float>({lambda_real, lambda_imag, 1}, b_seq, out, length, batch, state,
                                    stream, "diag_scan_forward");
 }
 
 int ossm_diag_scan_backward(const float* lambda_real, const float* lambda_imag, const void* states,
                             const void* grad_output, void* grad_lambda, void* grad_b,
                             int64_t length, int64_t batch, int64_t state, ossm_stream_t stream) {
-  return diag_backward_entry<float>(lambda_real, lambda_imag, states, grad_output, grad_lambda,
+  return diag_backward_entry<float>({lambda_real, lambda_imag, 1}, states, grad_output, grad_lambda,
                                     grad_b, length, batch, state, stream, "diag_scan_backward");
 }
 
 int ossm_diag_scan_forward_f64(const double* lambda_real, const double* lambda_imag,
                                const void* b_seq, void* out, int64_t length, int64_t batch,
                                int64_t state, ossm_stream_t stream) {
-  return diag_forward_entry<double>(lambda_real, lambda_imag, b_seq, out, length, batch, state,
+  return diag_forward_entry<double>({lambda_real, lambda_imag, 1}, b_seq, out, length, batch, state,
                                     stream, "diag_scan_forward_f64");
 }
 
@@ -674,8 +682,33 @@ int ossm_diag_scan_backward_f64(const double* lambda_real, const double* lambda_
                                 const void* states, const void* grad_output, void* grad_lambda,
                                 void* grad_b, int64_t length, int64_t batch, int64_t state,
                                 ossm_stream_t stream) {
-  return diag_backward_entry<double>(lambda_real, lambda_imag, states, grad_output, grad_lambda,
+  return diag_backward_entry<double>({lambda_real, lambda_imag, 1}, states, grad_output, grad_lambda,
                                      grad_b, length, batch, state, stream, "diag_scan_backward_f64");
+}
+
+int ossm_diag_scan_forward_cx(int f64, const void* lambda, const void* b_seq, void* out, int64_t length,
+                              int64_t batch, int64_t state, ossm_stream_t stream) {
+  if (f64) {
+    const auto* l = static_cast<const double*>(lambda);
+    return diag_forward_entry<double>({l, l ? l + 1 : nullptr, 2}, b_seq, out, length, batch, state, stream,
+                                      "diag_scan_forward_cx");
+  }
+  const auto* l = static_cast<const float*>(lambda);
+  return diag_forward_entry<float>({l, l ? l + 1 : nullptr, 2}, b_seq, out, length, batch, state, stream,
+                                   "diag_scan_forward_cx");
+}
+
+int ossm_diag_scan_backward_cx(int f64, const void* lambda, const void* states, const void* grad_output,
+                               void* grad_lambda, void* grad_b, int64_t length, int64_t batch, int64_t state,
+                               ossm_stream_t stream) {
+  if (f64) {
+    const auto* l = static_cast<const double*>(lambda);
+    return diag_backward_entry<double>({l, l ? l + 1 : nullptr, 2}, states, grad_output, grad_lambda, grad_b,
+                                       length, batch, state, stream, "diag_scan_backward_cx");
+  }
+  const auto* l = static_cast<const float*>(lambda);
+  return diag_backward_entry<float>({l, l ? l + 1 : nullptr, 2}, states, grad_output, grad_lambda, grad_b,
+                                    length, batch, state, stream, "diag_scan_backward_cx");
 }
 
 }  // extern "C"

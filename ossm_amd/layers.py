@@ -79,10 +79,8 @@ class LayerParamsFn(torch.autograd.Function):
                 steps: Tensor):  # type: ignore[override]
         A, G, s = (None if t is None else t.contiguous() for t in (A_diag, G_diag, steps))
         out = torch.empty((6, A.numel()), dtype=torch.float32, device=A.device)
-        with torch.cuda.device(A.device):
-            _lib.check(_lib.load().ossm_layer_params_forward(
-                int(damped), A.data_ptr(), _lib.ptr(G), s.data_ptr(), out.data_ptr(), A.numel(),
-                _lib.stream_of(A)))
+        _lib.run(_lib.load().ossm_layer_params_forward, A, int(damped), A.data_ptr(), _lib.ptr(G),
+                 s.data_ptr(), out.data_ptr(), A.numel())
         ctx.damped = damped
         ctx.set_materialize_grads(False)
         ctx.save_for_backward(A_diag, G_diag, steps)
@@ -109,10 +107,8 @@ class LayerParamsFn(torch.autograd.Function):
         A, G, s = (None if t is None else t.contiguous() for t in params)
         up = [None if g is None else g.contiguous() for g in grads]
         out = torch.empty((3, A.numel()), dtype=torch.float32, device=A.device)
-        with torch.cuda.device(A.device):
-            _lib.check(_lib.load().ossm_layer_params_backward(
-                int(ctx.damped), A.data_ptr(), _lib.ptr(G), s.data_ptr(), *[_lib.ptr(g) for g in up],
-                out.data_ptr(), A.numel(), _lib.stream_of(A)))
+        _lib.run(_lib.load().ossm_layer_params_backward, A, int(ctx.damped), A.data_ptr(), _lib.ptr(G),
+                 s.data_ptr(), *[_lib.ptr(g) for g in up], out.data_ptr(), A.numel())
         return (None, *[out[i] if n else None for i, n in enumerate(ctx.needs_input_grad[1:])])
 
 
@@ -189,12 +185,9 @@ def dlinoss_layer_forward(variant: str, inputs: Tensor, B: Tensor, C: Tensor, D:
         return out
     if carries is not None:
         _check_carries(carries, batch, length, ssm, u.device)
-    lib = _lib.load()
-    with torch.cuda.device(u.device):
-        _lib.check(lib.ossm_dlinoss_layer_forward_wide(
-            _VARIANTS[variant], u.data_ptr(), Bc.data_ptr(), Cc.data_ptr(), Dc.data_ptr(),
-            a.data_ptr(), g.data_ptr(), s.data_ptr(), _lib.ptr(_check_lo(lo, a)), out.data_ptr(), _lib.ptr(carries), batch,
-            length, hidden, ssm, _lib.stream_of(u)))
+    _lib.run(_lib.load().ossm_dlinoss_layer_forward_wide, u, _VARIANTS[variant], u.data_ptr(),
+             Bc.data_ptr(), Cc.data_ptr(), Dc.data_ptr(), a.data_ptr(), g.data_ptr(), s.data_ptr(),
+             _lib.ptr(_check_lo(lo, a)), out.data_ptr(), _lib.ptr(carries), batch, length, hidden, ssm)
     return out
 
 
@@ -225,13 +218,11 @@ def dlinoss_layer_backward(variant: str, inputs: Tensor, grad_output: Tensor, B:
     padded = -(-hidden // 32) * 32
     # the kernel sums grad_D where the padded width is a power of two
     gD = torch.empty(hidden, dtype=torch.float32, device=dev) if hidden and padded & (padded - 1) == 0 else None
-    with torch.cuda.device(dev):
-        _lib.check(_lib.load().ossm_dlinoss_layer_backward_wide(
-            _VARIANTS[variant], u.data_ptr(), go.data_ptr(), Bc.data_ptr(), Cc.data_ptr(),
-            Dc.data_ptr(), a.data_ptr(), g.data_ptr(), s.data_ptr(), _lib.ptr(_check_lo(lo, a)),
-            carries.data_ptr(),
-            gu.data_ptr(), gbu.data_ptr(), xq.data_ptr(), ga.data_ptr(), gg.data_ptr(),
-            gs.data_ptr(), _lib.ptr(gD), batch, length, hidden, ssm, _lib.stream_of(u)))
+    _lib.run(_lib.load().ossm_dlinoss_layer_backward_wide, u, _VARIANTS[variant], u.data_ptr(),
+             go.data_ptr(), Bc.data_ptr(), Cc.data_ptr(), Dc.data_ptr(), a.data_ptr(), g.data_ptr(),
+             s.data_ptr(), _lib.ptr(_check_lo(lo, a)), carries.data_ptr(), gu.data_ptr(), gbu.data_ptr(),
+             xq.data_ptr(), ga.data_ptr(), gg.data_ptr(), gs.data_ptr(), _lib.ptr(gD), batch, length,
+             hidden, ssm)
     rows = batch * length
     uf, gof = u.reshape(rows, hidden), go.reshape(rows, hidden)
     # grad_B[p, h, c] = sum_r grad_bu[r, p, c] u[r, h];  grad_C[h, p, c] = sum_r go[r, h] xq[r, p, c]

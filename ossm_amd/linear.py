@@ -48,10 +48,8 @@ def rows_product(a: Tensor, b: Tensor, pairs: bool = False) -> Tensor:
     strides = (2 * N, 1, 2) if pairs else (2 * N, N, 1)
     if not pairs and _tiles(N, M) < _tiles(M, N):  # the wider side of the tile along N
         a, b, M, N, strides = b, a, N, M, (2, 1, N)
-    with torch.cuda.device(a.device):
-        _lib.check(_lib.load().ossm_rows_product(
-            a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), out.data_ptr(), *strides, R, M, N,
-            _lib.stream_of(a)))
+    _lib.run(_lib.load().ossm_rows_product, a, a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0),
+             out.data_ptr(), *strides, R, M, N)
     return out
 
 
