@@ -534,8 +534,7 @@ int ossm_layer_params_backward(int damped, const float* A_diag, const float* G_d
  * ossm_dlinoss_layer_forward / _backward with params_lo [3][ssm] (may be null): what
  * a_diag, g_diag and step leave of their double values.  With it the oscillators'
  * coefficients are formed from the sums in double and rounded once.  The backward
- * also gives grad_d [hidden], the gradient of D (may be null), where hidden rounded
- * up to 32 is a power of two.
+ * also gives grad_d [hidden], the gradient of D (may be null).
  */
 int ossm_dlinoss_layer_forward_wide(int variant, const float* inputs, const float* B, const float* C,
                                     const float* D, const float* a_diag, const float* g_diag,

@@ -722,8 +722,9 @@ __global__ __launch_bounds__(kLayerThreads) void dlinoss_layer_bwd_kernel(
   // 2. u -> LDS (over gy); bu on the matrix cores, held in the accumulators
   //    until every wave has read u, then written to sX over it.  Where u
   //    replaces gy the thread holds both: its share of grad_D = sum gy u.
-  if (A.part_d != nullptr) {
-    const int q4 = Hp / 4;  // a power of two: the thread's columns are the same in every group
+  const bool pow2 = (Hp & (Hp - 1)) == 0;
+  if (A.part_d != nullptr && pow2) {
+    const int q4 = Hp / 4;  // the thread's columns are the same in every group
     float4 d = f4zero();
 #pragma unroll
     for (int k = 0; k < kLayerMax / 32; ++k) {
@@ -742,7 +743,18 @@ __global__ __launch_bounds__(kLayerThreads) void dlinoss_layer_bwd_kernel(
   __syncthreads();
   if (A.part_d != nullptr && static_cast<int>(threadIdx.x) < A.H) {
     const int h = threadIdx.x;
-    A.part_d[static_cast<size_t>(ticket) * A.H + h] = s_d[0][h] + s_d[1][h] + s_d[2][h] + s_d[3][h];
+    float d = 0.f;
+    if (pow2) {
+      d = s_d[0][h] + s_d[1][h] + s_d[2][h] + s_d[3][h];
+    } else {  // column h of gy again (from L2) against u's in LDS
+      float gv[kLc];
+#pragma unroll
+      for (int t = 0; t < kLc; ++t) gv[t] = A.gy[row0 + static_cast<size_t>(min(t, nt - 1)) * A.H + h];
+#pragma unroll
+      for (int t = 0; t < kLc; ++t)
+        if (t < nt) d += gv[t] * sA[t * HS + h];
+    }
+    A.part_d[static_cast<size_t>(ticket) * A.H + h] = d;
   }
   {
     const float* arow = sA + m * HS + half * hh;
@@ -970,9 +982,20 @@ int launch_split_weights(const SplitW& g0, const SplitW& g1, const SplitW& g2, i
 //             [16, 2048, 200, 100] (940) 118 -> 83; [8, 4096, 256, 256] (2147)
 //             218 -> 142; [32, 4096, 128, 128] (2147) 240 -> 162
 //   backward  26.2 -> 25.7; 32.2 -> 31.5; 46.8 -> 36.9; 181 -> 120; 385 -> 277; 418 -> 295
+// Where H or P is not a multiple of 4 the fp32 projections load their weights
+// one by one and the split ones still read theirs whole: wide layers then run
+// split at any length and the forward's floor is the backward's.  [26, 100, 139, 116]
+// 34.6 -> 28.6 / 51.6 -> 43.1; [2, 100, 255, 255] 60.6 -> 46.6 / 95.9 -> 72.7;
+// [7, 3252, 57, 34] 39.0 -> 35.6 / 72.2 -> 58.5; [30, 125, 55, 98] 20.6 -> 20.8 / 33.2 -> 29.9.
 constexpr int64_t kSplitFwd = int64_t(1) << 27, kSplitBwd = int64_t(1) << 25;
-bool use_split(int64_t rows, int64_t H, int64_t P, int64_t floor) {
-  return P > 0 && rows * ((H + 31) / 32 * 32) * ((P + 31) / 32 * 32) >= floor;
+constexpr int64_t kSplitWide = int64_t(1) << 14;  // padded H x padded P
+bool use_split(int64_t rows, int64_t H, int64_t P, int64_t floor, bool vec) {
+  const int64_t hp = (H + 31) / 32 * 32 * ((P + 31) / 32 * 32);
+  if (!vec) {
+    if (hp >= kSplitWide) return true;
+    floor = std::min(floor, kSplitBwd);
+  }
+  return P > 0 && rows * hp >= floor;
 }
 
 template <class Model>
@@ -1002,12 +1025,14 @@ int launch_layer_bwd(LayerBwdArgs args, float* ga, float* gg, float* gs, float* 
   void* payload = nullptr;
   LaunchSync sync{};
   void* ws = nullptr;
+  const bool vec = args.H % 4 == 0 && args.P % 4 == 0 && aligned16(args.u) && aligned16(args.gy) &&
+                   aligned16(args.Bw) && aligned16(args.Cw);
   // partial sums (parameters, then grad_D), then (split) the three weight matrices
   const size_t n_part = static_cast<size_t>(args.n_chunks) * NS * nc;
   const size_t n_part_d = grad_d != nullptr ? static_cast<size_t>(n_wg) * args.H : 0;
   const size_t part_bytes = ((n_part + n_part_d) * sizeof(float) + 15) & ~size_t(15);
   const size_t w_uint4 = split_w_uint4(args.H, args.P);
-  bool split = use_split(static_cast<int64_t>(args.Bsz) * args.L, args.H, args.P, kSplitBwd);
+  bool split = use_split(static_cast<int64_t>(args.Bsz) * args.L, args.H, args.P, kSplitBwd, vec);
   if (split) {
     if (acquire_workspace(call, part_bytes + 3 * w_uint4 * sizeof(uint4), &ws)) {
       // e.g. under capture, where it may not grow: the fp32 projections need none
@@ -1030,8 +1055,6 @@ int launch_layer_bwd(LayerBwdArgs args, float* ga, float* gg, float* gs, float* 
       return rc;
   }
   args.zero = ZeroFill{{ga, gg, gs}, {args.P, args.P, args.P}};
-  const bool vec = args.H % 4 == 0 && args.P % 4 == 0 && aligned16(args.u) && aligned16(args.gy) &&
-                   aligned16(args.Bw) && aligned16(args.Cw);
   const bool pad = args.H % 32 != 0 || args.P % 32 != 0;
   auto kern = vec ? (pad ? dlinoss_layer_bwd_kernel<V, true, true, false> : dlinoss_layer_bwd_kernel<V, true, false, false>)
                   : (pad ? dlinoss_layer_bwd_kernel<V, false, true, false> : dlinoss_layer_bwd_kernel<V, false, false, false>);
@@ -1077,7 +1100,7 @@ int launch_layer(LayerArgs args, hipStream_t stream) {
   const bool vec = args.H % 4 == 0 && args.P % 4 == 0 && aligned16(args.u) && aligned16(args.Bw) &&
                    aligned16(args.Cw);
   const bool small = args.H <= 128 && args.P <= 128;
-  bool split = use_split(static_cast<int64_t>(args.Bsz) * args.L, args.H, args.P, kSplitFwd);
+  bool split = use_split(static_cast<int64_t>(args.Bsz) * args.L, args.H, args.P, kSplitFwd, vec);
   if (split) {
     const size_t n = split_w_uint4(args.H, args.P);
     void* ws = nullptr;
@@ -1185,9 +1208,6 @@ int ossm_dlinoss_layer_backward_wide(int variant, const float* inputs, const flo
   hipStream_t stream = static_cast<hipStream_t>(stream_v);
   if (ssm > 0 && (!grad_a || !grad_g || !grad_step))
     return set_error(OSSM_ERR_INVALID_ARGUMENT, std::string(what) + ": null pointer");
-  const int64_t hp = (hidden + 31) / 32 * 32;
-  if (grad_d != nullptr && (hidden == 0 || (hp & (hp - 1)) != 0))
-    return set_error(OSSM_ERR_UNSUPPORTED, std::string(what) + ": grad_D needs a hidden_dim that pads to a power of two");
   if (grad_d != nullptr && (batch == 0 || length == 0))
     if (int rc = fill_zero(grad_d, hidden, stream)) return rc;
   if (batch == 0 || length == 0 || hidden == 0) {

@@ -49,22 +49,33 @@ struct RowsProduct {
   int M, N, tiles_m, tiles_n, slices;
 };
 
-// W columns of a row from the lane's offset(s); VEC: one aligned vector load.
-template <bool VEC, int W>
+// W columns of a row from the lane's offsets, V at a time (V = W: one aligned vector
+// load; 2: pairs, for even widths that are no multiple of 4).
+template <int V, int W>
 __device__ __forceinline__ void load_cols(const float* __restrict__ row, const unsigned (&off)[W],
                                           float (&v)[W]) {
-  if constexpr (VEC) {
-    typedef float V __attribute__((ext_vector_type(W)));
-    const V x = *reinterpret_cast<const V*>(row + off[0]);
-#pragma unroll
-    for (int j = 0; j < W; ++j) v[j] = x[j];
-  } else {
+  if constexpr (V == 1) {
 #pragma unroll
     for (int j = 0; j < W; ++j) v[j] = row[off[j]];
+  } else {
+    typedef float X __attribute__((ext_vector_type(V)));
+#pragma unroll
+    for (int q = 0; q < W; q += V) {
+      const X x = *reinterpret_cast<const X*>(row + off[q]);
+#pragma unroll
+      for (int j = 0; j < V; ++j) v[q + j] = x[j];
+    }
   }
 }
 
-template <bool VEC>
+// The lane's column j of W from c0, clamped in range V columns at a time.
+template <int V>
+__device__ __forceinline__ unsigned clamp_col(int c0, int j, int n) {
+  return static_cast<unsigned>(min(c0 + j / V * V, n - V) + j % V);
+}
+
+// VA, VB: columns of a and b loaded at once.
+template <int VA, int VB>
 __global__ __launch_bounds__(kRpThreads, 1) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void rows_product_kernel(RowsProduct g) {
   extern __shared__ __align__(16) float s_tile[];  // [kRpWaves / 2][kTm * kTn]
@@ -80,17 +91,14 @@ void rows_product_kernel(RowsProduct g) {
   const int slice = id / tiles, tile = id - slice * tiles;
   const int m0 = (tile / g.tiles_n) * kTm, n0 = (tile % g.tiles_n) * kTn;
   // lane offsets from the block's first row; columns out of range read clamped
-  // ones (VEC: whole vectors, M % 4 == 0 and N % 2 == 0), which only reach
-  // outputs that are not stored
+  // ones, which only reach outputs that are not stored
   unsigned oa[4], ob[2];
 #pragma unroll
   for (int j = 0; j < 4; ++j)
-    oa[j] = static_cast<unsigned>(8 * half * g.lda) +
-            static_cast<unsigned>(VEC ? min(m0 + 4 * l32, g.M - 4) + j : min(m0 + 4 * l32 + j, g.M - 1));
+    oa[j] = static_cast<unsigned>(8 * half * g.lda) + clamp_col<VA>(m0 + 4 * l32, j, g.M);
 #pragma unroll
   for (int j = 0; j < 2; ++j)
-    ob[j] = static_cast<unsigned>(8 * half * g.ldb) +
-            static_cast<unsigned>(VEC ? min(n0 + 2 * l32, g.N - 2) + j : min(n0 + 2 * l32 + j, g.N - 1));
+    ob[j] = static_cast<unsigned>(8 * half * g.ldb) + clamp_col<VB>(n0 + 2 * l32, j, g.N);
 
   floatx16 acc[4][2];
 #pragma unroll
@@ -110,8 +118,8 @@ void rows_product_kernel(RowsProduct g) {
     const long long r0 = min(k * kBlockRows, g.R - kBlockRows);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      load_cols<VEC, 4>(g.a + (r0 + i) * g.lda, oa, ra[i]);
-      load_cols<VEC, 2>(g.b + (r0 + i) * g.ldb, ob, rb[i]);
+      load_cols<VA, 4>(g.a + (r0 + i) * g.lda, oa, ra[i]);
+      load_cols<VB, 2>(g.b + (r0 + i) * g.ldb, ob, rb[i]);
     }
   };
   if (blk < n_blocks) load(blk);
@@ -279,9 +287,12 @@ int ossm_rows_product(const float* a, int64_t ld_a, const float* b, int64_t ld_b
   const RowsProduct g{a, b, static_cast<float*>(ws), rows, ld_a, ld_b, static_cast<int>(m),
                       static_cast<int>(n), static_cast<int>(tm), static_cast<int>(tn),
                       static_cast<int>(slices)};
-  const bool vec = m % 4 == 0 && ld_a % 4 == 0 && aligned_to(a, 16) && n % 2 == 0 && ld_b % 2 == 0 &&
-                   aligned_to(b, 8);
-  auto kern = vec ? rows_product_kernel<true> : rows_product_kernel<false>;
+  const int va = m % 4 == 0 && ld_a % 4 == 0 && aligned_to(a, 16)  ? 4
+                 : m % 2 == 0 && ld_a % 2 == 0 && aligned_to(a, 8) ? 2
+                                                                   : 1;
+  const bool vb = n % 2 == 0 && ld_b % 2 == 0 && aligned_to(b, 8);
+  auto kern = vb ? (va == 4 ? rows_product_kernel<4, 2> : va == 2 ? rows_product_kernel<2, 2> : rows_product_kernel<1, 2>)
+                 : (va == 4 ? rows_product_kernel<4, 1> : va == 2 ? rows_product_kernel<2, 1> : rows_product_kernel<1, 1>);
   constexpr int lds = kRpWaves / 2 * kTm * kTn * static_cast<int>(sizeof(float));
   if (int rc = hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, lds),

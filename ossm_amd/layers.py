@@ -33,7 +33,7 @@ from torch import Tensor, nn
 
 from . import _lib
 from .bridge import run_dlinoss
-from .linear import MIN_ROWS, rows_product
+from .linear import BLOCK_ROWS, rows_product
 
 __all__ = ["DampedLinOSSLayer", "dlinoss_layer_forward", "dlinoss_layer_backward", "DlinossLayerFn",
            "project_parameters", "unfused_layer_forward", "LayerParamsFn", "fused_layer_supported"]
@@ -215,26 +215,22 @@ def dlinoss_layer_backward(variant: str, inputs: Tensor, grad_output: Tensor, B:
     gbu = torch.empty((batch, length, ssm, 2), dtype=torch.float32, device=dev)
     xq = torch.empty_like(gbu)
     ga, gg, gs = (torch.empty(ssm, dtype=torch.float32, device=dev) for _ in range(3))
-    padded = -(-hidden // 32) * 32
-    # the kernel sums grad_D where the padded width is a power of two
-    gD = torch.empty(hidden, dtype=torch.float32, device=dev) if hidden and padded & (padded - 1) == 0 else None
+    gD = torch.empty(hidden, dtype=torch.float32, device=dev)
     _lib.run(_lib.load().ossm_dlinoss_layer_backward_wide, u, _VARIANTS[variant], u.data_ptr(),
              go.data_ptr(), Bc.data_ptr(), Cc.data_ptr(), Dc.data_ptr(), a.data_ptr(), g.data_ptr(),
              s.data_ptr(), _lib.ptr(_check_lo(lo, a)), carries.data_ptr(), gu.data_ptr(), gbu.data_ptr(),
-             xq.data_ptr(), ga.data_ptr(), gg.data_ptr(), gs.data_ptr(), _lib.ptr(gD), batch, length,
+             xq.data_ptr(), ga.data_ptr(), gg.data_ptr(), gs.data_ptr(), gD.data_ptr(), batch, length,
              hidden, ssm)
     rows = batch * length
     uf, gof = u.reshape(rows, hidden), go.reshape(rows, hidden)
     # grad_B[p, h, c] = sum_r grad_bu[r, p, c] u[r, h];  grad_C[h, p, c] = sum_r go[r, h] xq[r, p, c]
     gbu2, xq2 = gbu.reshape(rows, 2 * ssm), xq.reshape(rows, 2 * ssm)
-    if rows >= MIN_ROWS:
+    if rows >= BLOCK_ROWS:
         gB, gC = rows_product(gbu2, uf, pairs=True), rows_product(gof, xq2)
     else:
         gB = _sum_rows_product(gbu2, uf).reshape(ssm, 2, hidden).permute(0, 2, 1).contiguous()
         gC = _sum_rows_product(gof, xq2)
     gC = gC.reshape(hidden, ssm, 2)
-    if gD is None:
-        gD = (gof * uf).sum(0)
     return gu, gB, gC, gD, ga, gg, gs
 
 

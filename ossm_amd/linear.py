@@ -17,10 +17,11 @@ from torch import Tensor, nn
 from . import _lib
 
 __all__ = ["rows_product", "linear", "linear_weight", "LinearFn", "is_plain",
-           "MIN_ROWS"]
+           "MIN_ROWS", "BLOCK_ROWS"]
 
-# Fewer rows go to the library: 200 rows 9 us there against 12, 1000 rows 60
-# against 14 ([R, 80] x [R, 40] and [R, 256] x [R, 64]).
+BLOCK_ROWS = 16  # the least the kernel takes
+# LinearFn with fewer rows leaves the weight gradient to the library's GEMM: 200 rows
+# 9 us against 12, 1000 rows 60 against 14 ([R, 80] x [R, 40] and [R, 256] x [R, 64]).
 MIN_ROWS = 512
 
 
@@ -40,7 +41,7 @@ def rows_product(a: Tensor, b: Tensor, pairs: bool = False) -> Tensor:
     R, M, N = a.size(0), a.size(1), b.size(1)
     if pairs and M % 2 != 0:
         raise RuntimeError("rows_product: pairs needs an even number of columns in a")
-    if R < MIN_ROWS or M == 0 or N == 0:
+    if R < BLOCK_ROWS or M == 0 or N == 0:
         out = a.t() @ b
         return out.reshape(M // 2, 2, N).transpose(1, 2).contiguous() if pairs else out
     a, b = (t if t.stride(1) == 1 and t.stride(0) >= t.size(1) else t.contiguous() for t in (a, b))

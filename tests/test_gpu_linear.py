@@ -18,9 +18,9 @@ def _bound(a, b):
     return 4 * 2.0 ** -24 * (a.abs().double().t() @ b.abs().double()) + 1e-30
 
 
-# one short block after the rule's floor, a ragged last block, tiles with one
+# one block, a last block of one row, a ragged last block, tiles with one
 # column, exact tiles, columns past a tile, more tiles than CUs / slices
-@pytest.mark.parametrize("shape", [(512, 1, 1), (513, 128, 64), (527, 129, 65), (1000, 4, 130), (4097, 36, 128),
+@pytest.mark.parametrize("shape", [(16, 3, 2), (17, 130, 66), (512, 1, 1), (513, 128, 64), (527, 129, 65), (1000, 4, 130), (4097, 36, 128),
                                    (20000, 256, 3), (640, 2050, 1030)],
                          ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("layout", ["plain", "pairs", "strided", "odd_stride"])
