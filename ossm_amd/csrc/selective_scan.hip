@@ -63,6 +63,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cfloat>
 #include <cstdlib>
 #include <climits>
 #include <initializer_list>
@@ -481,6 +482,54 @@ __device__ __forceinline__ void store_states(float* __restrict__ s, const StateR
 }
 
 // ---- forward ------------------------------------------------------------------
+// Time segments whose carries go through memory (see segment_plan).  mode 0: a
+// segment re-runs the recurrence over the segments it depends on; 1: it only runs
+// its own, from zero, and stores where that ends and its sum of dt (the transition
+// of state n over the segment is exp(A_n sum dt)); 2: it folds the stored ones
+// into its carry.
+struct SegCarry {
+  int mode;
+  float* end;  // [segment][B, D][N]
+  float* dt;   // [segment][B, D]
+};
+
+// h past a segment that ends at `end` from zero, `sdt` its sum of dt.  Infinities go
+// on as they do step by step: a zero state leaves the transition unread, an infinite
+// one stays (their products with an overflowed or underflowed transition would be
+// NaN), and one that overflows here keeps its sign, the earlier growth's.
+__device__ __forceinline__ float fold_segment(float h, float sdt, float A2, float end) {
+  if (h == 0.f) return end;
+  float f = fast_exp2(sdt * A2);
+  if (fabsf(h) == INFINITY) f = fmaxf(f, FLT_MIN);
+  return fabsf(f * h) == INFINITY && fabsf(end) == INFINITY ? f * h : fmaf(f, h, end);
+}
+
+// The carry of one row's states [n0, n0 + NPW) past segments first, first + step, ..
+// (n of them).  A batch of loads is in flight at once: one segment after the other
+// cost a memory latency each, 31 of them longer than the scan.
+template <int NPW>
+__device__ __forceinline__ void fold_segments(float (&h)[NPW], const float (&A2)[NPW], const SegCarry& c, int first,
+                                              int step, int n, size_t n_rows, size_t row, int N, int n0) {
+  constexpr int kBatch = 8;
+  for (int j0 = 0; j0 < n; j0 += kBatch) {
+    float sdt[kBatch], e[kBatch][NPW];
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) {
+      const size_t at = (first + step * min(j0 + k, n - 1)) * n_rows + row;
+      sdt[k] = c.dt[at];
+#pragma unroll
+      for (int q = 0; q < NPW; ++q) e[k][q] = n0 + q < N ? c.end[at * N + n0 + q] : 0.f;
+    }
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) {
+      if (j0 + k < n) {
+#pragma unroll
+        for (int q = 0; q < NPW; ++q) h[q] = fold_segment(h[q], sdt[k], A2[q], e[k][q]);
+      }
+    }
+  }
+}
+
 template <class E>
 struct FwdArgs {
   const E* u;
@@ -503,6 +552,7 @@ struct FwdArgs {
   // [B, D, L] only: per-channel skip D (the extended API): the last pass adds
   // D u to y before raw_out and the gate; null for the reference's scan
   const float* dskip;
+  SegCarry carry;
 };
 
 // (dt_t, u_t) pairs of a [.., L] row tile: s[row * RS2 + 2t].
@@ -722,7 +772,8 @@ __device__ __forceinline__ void reduce_groups(float (&yv)[kFwdTile],
 // GATED kernels multiply by silu(z) in the last pass; VEC: L % 4 == 0 and
 // u/dt/z/out rows 16-byte aligned.  NPW: states per lane (FwdLayout); the
 // [B, L, D] layout (BLD) runs 4.
-template <class E, bool VEC, bool GATED, bool BLD, int NPW>
+// CARRY: segments' carries through memory (SegCarry).
+template <class E, bool VEC, bool GATED, bool BLD, int NPW, bool CARRY>
 __global__ __launch_bounds__(kThreads) void selective_fwd_kernel(FwdArgs<E> a) {
   using LY = FwdLayout<NPW>;
   constexpr int TT = kFwdTile;
@@ -788,7 +839,8 @@ __global__ __launch_bounds__(kThreads) void selective_fwd_kernel(FwdArgs<E> a) {
   // Time split: gridDim.z segments of consecutive tiles; segment s scans
   // tiles [s n / S, (s + 1) n / S) after re-running h alone over the tiles
   // before them (no outputs, the same per-step arithmetic, so the state it
-  // reaches is bitwise the one the earlier segments compute).
+  // reaches is bitwise the one the earlier segments compute), or from the
+  // folded ends of the earlier segments (SegCarry).
   const int n_tiles = (a.L + TT - 1) / TT;
   const int n_seg = static_cast<int>(gridDim.z), seg = static_cast<int>(blockIdx.z);
   const int t_lo = (seg * n_tiles / n_seg) * TT;
@@ -796,9 +848,17 @@ __global__ __launch_bounds__(kThreads) void selective_fwd_kernel(FwdArgs<E> a) {
 
   FwdTile<ROWS> nxt;
   float zn[SEG];  // the gate of the lane's output segment, one tile ahead
-  fwd_prefetch<E, VEC, BLD>(nxt, a, row0, bc0, d0, 0);
-  for (int t0 = 0; t0 < t_lo; t0 += TT) {
-    // h only over the earlier segment's tiles
+  // the tiles h alone runs over: those before the segment, or (mode 1) its own
+  const bool ends = CARRY && a.carry.mode == 1;
+  const int r_lo = CARRY ? t_lo : 0, r_hi = CARRY ? (ends ? t_hi : t_lo) : t_lo;
+  const size_t seg_row = static_cast<size_t>(b) * a.D + dc, n_rows = static_cast<size_t>(gridDim.y) * a.D;
+  if constexpr (CARRY) {
+    if (ends && seg == n_seg - 1) return;  // nothing reads the last one's end
+    if (!ends) fold_segments(h, A2, a.carry, 0, 1, seg, n_rows, seg_row, a.N, n0);
+  }
+  fwd_prefetch<E, VEC, BLD>(nxt, a, row0, bc0, d0, r_lo);
+  float sum_dt = 0.f;
+  for (int t0 = r_lo; t0 < r_hi; t0 += TT) {
     __syncthreads();
     if constexpr (BLD) {
       store_cols_dtu<TT, RS2>(s_dtu, nxt.dt, nxt.u, a.dt_bias, d0, a.D, t0, a.L);
@@ -815,11 +875,21 @@ __global__ __launch_bounds__(kThreads) void selective_fwd_kernel(FwdArgs<E> a) {
       const float2 du = *reinterpret_cast<const float2*>(dturow + 2 * i);
       const float dtv = du.x;
       const float dtu = dtv * du.y;
+      if constexpr (CARRY) sum_dt += dtv;
       float Bv[NPW];
       unpack(bc_vals(BCgrp, i).b, Bv);
 #pragma unroll
       for (int j = 0; j < NPW; ++j) h[j] = fmaf(fast_exp2(dtv * A2[j]), h[j], dtu * Bv[j]);
     }
+  }
+  if (ends) {
+    if (dvalid) {
+      if (g == 0) a.carry.dt[seg * n_rows + seg_row] = sum_dt;
+#pragma unroll
+      for (int q = 0; q < NPW; ++q)
+        if (n0 + q < a.N) a.carry.end[(seg * n_rows + seg_row) * a.N + n0 + q] = h[q];
+    }
+    return;
   }
   if constexpr (GATED && !BLD) load_gate(zn, t_lo);
   for (int t0 = t_lo; t0 < t_hi; t0 += TT) {
@@ -1017,6 +1087,7 @@ struct BwdArgs {
   // dD = sum_t gy u into part_dD [time segments * B, D]
   const float* dskip;
   float* part_dD;
+  SegCarry carry;
 };
 
 struct BwdTile {
@@ -1088,7 +1159,7 @@ __device__ __forceinline__ void adj_prefetch(AdjTile& f, const BwdArgs<E>& a, si
   load_states<kBwdTile>(f.C, a.Cm, bc0, a.ld_bc, t0, a.L, a.N, a.n_base);
 }
 
-template <class E, bool VEC, bool GATED, bool BLD, bool SKIP>
+template <class E, bool VEC, bool GATED, bool BLD, bool SKIP, bool CARRY>
 __global__ __launch_bounds__(kThreads) void selective_bwd_kernel(BwdArgs<E> a) {
   static_assert(!BLD || std::is_same_v<E, float>, "the [B, L, D] layout is fp32");
   static_assert(!(BLD && SKIP), "the skip D is for the [B, D, L] layout");
@@ -1151,10 +1222,19 @@ __global__ __launch_bounds__(kThreads) void selective_bwd_kernel(BwdArgs<E> a) {
   const int n_seg = static_cast<int>(gridDim.z), seg = static_cast<int>(blockIdx.z);
   const int tile_lo = seg * n_tiles / n_seg;
   const int tile_hi = (seg + 1) * n_tiles / n_seg;
-  if (tile_hi < n_tiles) {
+  // the tiles the adjoint alone runs over: those after the segment, or (mode 1) its own
+  const bool ends = CARRY && a.carry.mode == 1;
+  const int r_hi = CARRY ? tile_hi : n_tiles, r_lo = ends ? tile_lo : tile_hi;
+  const size_t seg_row = static_cast<size_t>(b) * a.D + (dvalid ? d : a.D - 1);
+  const size_t n_rows = static_cast<size_t>(a.Bsz) * a.D;
+  if (ends && seg == 0) return;  // nothing reads the first one's
+  if (CARRY && wave_active && !ends)
+    fold_segments(gs, A2, a.carry, n_seg - 1, -1, n_seg - 1 - seg, n_rows, seg_row, a.N, n0);
+  if (r_lo < r_hi) {
     AdjTile p;
-    adj_prefetch<E, VEC, GATED, BLD>(p, a, row0, bc0, d0, n_tiles - 1);
-    for (int tile = n_tiles - 1; tile >= tile_hi; --tile) {
+    float sum_dt = 0.f;
+    adj_prefetch<E, VEC, GATED, BLD>(p, a, row0, bc0, d0, r_hi - 1);
+    for (int tile = r_hi - 1; tile >= r_lo; --tile) {
       const int t0 = tile * TT;
       __syncthreads();
       if constexpr (BLD) {
@@ -1188,7 +1268,7 @@ __global__ __launch_bounds__(kThreads) void selective_bwd_kernel(BwdArgs<E> a) {
         }
       }
       __syncthreads();
-      if (tile > tile_hi) adj_prefetch<E, VEC, GATED, BLD>(p, a, row0, bc0, d0, tile - 1);
+      if (tile > r_lo) adj_prefetch<E, VEC, GATED, BLD>(p, a, row0, bc0, d0, tile - 1);
       if (wave_active) {
         const float* dtrow = s_dt + lane * RS;
         const float* gyrow = s_gy + lane * RS;
@@ -1198,10 +1278,20 @@ __global__ __launch_bounds__(kThreads) void selective_bwd_kernel(BwdArgs<E> a) {
           const float gy = gyrow[i], dtv = dtrow[i];
           const float4 Ct = *reinterpret_cast<const float4*>(Ccol + i * kPassStates);
           const float Cv[4] = {Ct.x, Ct.y, Ct.z, Ct.w};
+          if constexpr (CARRY) sum_dt += dtv;
 #pragma unroll
           for (int j = 0; j < kNpw; ++j) gs[j] = fmaf(gy, Cv[j], gs[j]) * fast_exp2(dtv * A2[j]);
         }
       }
+    }
+    if (ends) {
+      if (dvalid && wave_active) {
+        if (w == 0) a.carry.dt[seg * n_rows + seg_row] = sum_dt;
+#pragma unroll
+        for (int q = 0; q < kNpw; ++q)
+          if (n0 + q < a.N) a.carry.end[(seg * n_rows + seg_row) * a.N + n0 + q] = gs[q];
+      }
+      return;
     }
   }
 
@@ -2280,6 +2370,29 @@ bool cols_vectorizable(int64_t D, const MambaLayout& ml, std::initializer_list<c
   return true;
 }
 
+// Segments of a problem whose few rows leave the device idle: as many as give
+// `want` workgroups per compute unit, each of at least 64 steps, up to 32, their
+// carries through memory (SegCarry: a launch that runs every segment from zero, then
+// the scan).  Per row the path is 2 L / S steps, against 0.87 to 1.0 L where segments
+// re-run the ones before them (time_segments).  0 below three segments and below 512
+// steps, where the second launch eats what the split saves.  The variables that
+// force another path turn it off.
+// fp32, N = 16, gated, forward / backward, us, re-run -> carried:
+//   B, D = 1, 922:  L = 256  16 -> 18 / 28 -> 28,  512  29 -> 22 / 48 -> 35,
+//                   2048  108 -> 40 / 163 -> 70,  8192  419 -> 103 / 618 -> 163
+//   B, D = 27, 80:  L = 256  18 -> 20 / 32 -> 34,  512  33 -> 33 / 55 -> 54,
+//                   2048  119 -> 96 / 190 -> 137
+//   B, D = 16, 512 (forward not split):  1024  74 -> 74 / 177 -> 156
+// The outputs' error against float64 is the re-run segments' or smaller (decay over
+// 2000 steps: 5e-7 here, 4e-6 there, one product of the steps' transitions).
+int segment_plan(int64_t n_wg, int64_t L, int want, int n_cu) {
+  if (L < 512) return 0;
+  for (const char* name : {"OSSM_SEL_SPLIT", "OSSM_SEL_FWD_NPW", "OSSM_SEL_BWD_NPW"})
+    if (std::getenv(name) != nullptr) return 0;
+  const int64_t s = std::min<int64_t>({static_cast<int64_t>(want) * n_cu / std::max<int64_t>(n_wg, 1), L / 64, 32});
+  return s >= 3 ? static_cast<int>(s) : 0;
+}
+
 // Time segments per (batch row, channel tile), 1, 2 or 4: the fewest that
 // give at least `want` workgroups per compute unit, with every segment at
 // least two tiles long.  OSSM_SEL_SPLIT=1|2|4 overrides.  Segment s re-runs
@@ -2351,6 +2464,18 @@ int fwd_states_per_lane(int64_t rows64) {
   return rows64 * kMaxWaves < static_cast<int64_t>(OSSM_SEL_FWD_NPW2_BELOW) * 4 * n_cu ? 2 : 4;
 }
 
+template <class E, bool BLD, int NPW, bool CARRY>
+auto fwd_kernel(bool vec, const void* gate) {
+  return vec ? (gate ? selective_fwd_kernel<E, true, true, BLD, NPW, CARRY> : selective_fwd_kernel<E, true, false, BLD, NPW, CARRY>)
+             : (gate ? selective_fwd_kernel<E, false, true, BLD, NPW, CARRY> : selective_fwd_kernel<E, false, false, BLD, NPW, CARRY>);
+}
+
+template <class E, bool BLD, bool SKIP, bool CARRY>
+auto bwd_kernel(bool vec, const void* gate) {
+  return vec ? (gate ? selective_bwd_kernel<E, true, true, BLD, SKIP, CARRY> : selective_bwd_kernel<E, true, false, BLD, SKIP, CARRY>)
+             : (gate ? selective_bwd_kernel<E, false, true, BLD, SKIP, CARRY> : selective_bwd_kernel<E, false, false, BLD, SKIP, CARRY>);
+}
+
 // E = float: the fp32 API of the reference.  E = bf16_t: the same scan with
 // bf16 rows, B and C in HBM (A, chunk_states and dA stay fp32).  ml: the
 // [B, L, D] layout (fp32 only); null for the reference's [B, D, L].  dskip:
@@ -2410,10 +2535,34 @@ int selective_forward_impl(const E* u, const E* dt, const float* A, const E* Bm,
   }
   // states per lane: 2 (32-channel workgroups) when 64-channel workgroups
   // would leave the SIMDs short of waves, else 4; the [B, L, D] layout runs 4
-  const int npw = ml != nullptr ? 4 : fwd_states_per_lane(((dim + kWave - 1) / kWave) * batch);
+  // and few rows run time segments, 4 states per lane (segment_plan)
+  const int64_t rows64 = batch * ((dim + kWave - 1) / kWave);
+  int n_seg = segment_plan(rows64, length, kFwdWgPerCu, device_cu_count(call.device()));
+  if (n_seg > 0) {
+    // the fp32 sums of several bf16 passes, then the segments' ends and sums of dt
+    const size_t acc_n = n_pass > 1 && !std::is_same_v<E, float> ? static_cast<size_t>(batch * dim * length) : 0;
+    const size_t rows_n = static_cast<size_t>(n_seg) * batch * dim;
+    void* ws = nullptr;
+    if (acquire_workspace(call, (acc_n + rows_n * (dstate + 1)) * sizeof(float), &ws)) {
+      // e.g. under capture, where it may not grow: without the carries' memory
+      (void)hipGetLastError();
+      clear_error();
+      n_seg = 0;
+      if (acc_n > 0) {  // the attempt may have released what held the sums
+        if (int rc = acquire_workspace(call, acc_n * sizeof(float), &ws)) return rc;
+        a.acc = static_cast<float*>(ws);
+      }
+    } else {
+      if (acc_n > 0) a.acc = static_cast<float*>(ws);
+      a.carry.end = static_cast<float*>(ws) + acc_n;
+      a.carry.dt = a.carry.end + rows_n * dstate;
+    }
+  }
+  const bool carried = n_seg > 0;
+  const int npw = ml != nullptr || carried ? 4 : fwd_states_per_lane(rows64);
   const int rows = npw == 4 ? FwdLayout<4>::kRows : FwdLayout<2>::kRows;
   const int64_t n_dtiles = (dim + rows - 1) / rows;
-  const int n_seg = time_segments(n_dtiles * batch, length, kFwdTile, kFwdWgPerCu);
+  if (!carried) n_seg = time_segments(n_dtiles * batch, length, kFwdTile, kFwdWgPerCu);
   const dim3 grid(static_cast<unsigned>(n_dtiles), static_cast<unsigned>(batch),
                   static_cast<unsigned>(n_seg));
   for (int p = 0; p < n_pass; ++p) {
@@ -2424,17 +2573,20 @@ int selective_forward_impl(const E* u, const E* dt, const float* A, const E* Bm,
     K kern;
     if (ml != nullptr) {
       if constexpr (std::is_same_v<E, float>) {
-        kern = a.vec ? (gate ? selective_fwd_kernel<E, true, true, true, 4> : selective_fwd_kernel<E, true, false, true, 4>)
-                     : (gate ? selective_fwd_kernel<E, false, true, true, 4> : selective_fwd_kernel<E, false, false, true, 4>);
+        kern = carried ? fwd_kernel<E, true, 4, true>(a.vec, gate) : fwd_kernel<E, true, 4, false>(a.vec, gate);
       } else {
         return set_error(OSSM_ERR_UNSUPPORTED, std::string(what) + ": the [B, L, D] layout is fp32");
       }
     } else if (npw == 4) {
-      kern = a.vec ? (gate ? selective_fwd_kernel<E, true, true, false, 4> : selective_fwd_kernel<E, true, false, false, 4>)
-                   : (gate ? selective_fwd_kernel<E, false, true, false, 4> : selective_fwd_kernel<E, false, false, false, 4>);
+      kern = carried ? fwd_kernel<E, false, 4, true>(a.vec, gate) : fwd_kernel<E, false, 4, false>(a.vec, gate);
     } else {
-      kern = a.vec ? (gate ? selective_fwd_kernel<E, true, true, false, 2> : selective_fwd_kernel<E, true, false, false, 2>)
-                   : (gate ? selective_fwd_kernel<E, false, true, false, 2> : selective_fwd_kernel<E, false, false, false, 2>);
+      kern = fwd_kernel<E, false, 2, false>(a.vec, gate);
+    }
+    if (carried) {
+      a.carry.mode = 1;
+      hipLaunchKernelGGL(kern, grid, dim3(kThreads), 0, stream, a);
+      if (int rc = launch_check("selective_fwd_kernel (segment ends)")) return rc;
+      a.carry.mode = 2;
     }
     hipLaunchKernelGGL(kern, grid, dim3(kThreads), 0, stream, a);
     if (int rc = launch_check("selective_fwd_kernel")) return rc;
@@ -2474,21 +2626,36 @@ int selective_backward_impl(const E* grad_out, const E* u, const E* dt, const fl
                      std::string(what) + ": a gated scan needs raw_outputs and dgate");
   const int n_pass = static_cast<int>((dstate + kPassStates - 1) / kPassStates);
   // [B, D, L]: 2 states per lane (32-channel workgroups) or 4 (64-channel)
-  const bool npw2 = ml == nullptr && bwd2_offsets_fit(length, dstate, dstate) &&
-                    bwd_states_per_lane(batch * ((dim + kWave - 1) / kWave)) == 2;
-  const int64_t wg_rows = npw2 ? kB2Rows : kWave;
-  const int64_t n_dtiles = (dim + wg_rows - 1) / wg_rows;
+  // few rows: segments with carried adjoints (the 4-states kernel), else one of
+  // the kernels with the segments it re-runs
+  const int64_t rows64 = batch * ((dim + kWave - 1) / kWave);
+  int n_seg = segment_plan(rows64, length, kBwdWgPerCu, device_cu_count(call.device()));
+  bool carried = n_seg > 0, npw2 = false;
+  int64_t n_dtiles = 0, dA_rows = 0;
   const int64_t n_bln = batch * length * dstate;
   const int64_t n_dn = dim * dstate;
   const int64_t n_rows = batch * dim * length;
   const bool staged = !std::is_same_v<E, float> && n_pass > 1;  // fp32 du/ddt between passes
-  const int n_seg = npw2 ? time_segments(n_dtiles * batch, length, kB2Tile, kBwd2WgPerCu)
-                         : time_segments(n_dtiles * batch, length, kBwdTile, kBwdWgPerCu);
-  const int64_t dA_rows = n_seg * batch;  // dA partial rows: (segment, batch row)
-  const size_t part_floats = static_cast<size_t>(2 * n_dtiles * n_bln + dA_rows * n_dn) +
-                            (staged ? 2 * n_rows : 0) + (dskip ? dA_rows * dim : 0);
+  size_t part_floats = 0;
   void* ws = nullptr;
-  if (int rc = acquire_workspace(call, part_floats * sizeof(float), &ws)) return rc;
+  for (;;) {
+    npw2 = !carried && ml == nullptr && bwd2_offsets_fit(length, dstate, dstate) && bwd_states_per_lane(rows64) == 2;
+    const int64_t wg_rows = npw2 ? kB2Rows : kWave;
+    n_dtiles = (dim + wg_rows - 1) / wg_rows;
+    if (!carried)
+      n_seg = npw2 ? time_segments(n_dtiles * batch, length, kB2Tile, kBwd2WgPerCu)
+                   : time_segments(n_dtiles * batch, length, kBwdTile, kBwdWgPerCu);
+    dA_rows = n_seg * batch;  // dA partial rows: (segment, batch row)
+    part_floats = static_cast<size_t>(2 * n_dtiles * n_bln + dA_rows * n_dn) + (staged ? 2 * n_rows : 0) +
+                  (dskip ? dA_rows * dim : 0);
+    const size_t carry_floats = carried ? static_cast<size_t>(dA_rows) * dim * (dstate + 1) : 0;
+    const int rc = acquire_workspace(call, (part_floats + carry_floats) * sizeof(float), &ws);
+    if (rc == OSSM_OK) break;
+    if (!carried) return rc;
+    (void)hipGetLastError();  // e.g. under capture, where it may not grow
+    clear_error();
+    carried = false;
+  }
   float* part_dB = static_cast<float*>(ws);
   float* part_dC = part_dB + n_dtiles * n_bln;
   float* part_dA = part_dC + n_dtiles * n_bln;
@@ -2496,6 +2663,10 @@ int selective_backward_impl(const E* grad_out, const E* u, const E* dt, const fl
   float* part_dD = dskip ? part_dA + dA_rows * n_dn + (staged ? 2 * n_rows : 0) : nullptr;
 
   BwdArgs<E> a{};
+  if (carried) {
+    a.carry.end = static_cast<float*>(ws) + part_floats;
+    a.carry.dt = a.carry.end + static_cast<size_t>(dA_rows) * dim * dstate;
+  }
   a.gout = grad_out;
   a.u = u;
   a.dt = dt;
@@ -2559,17 +2730,20 @@ int selective_backward_impl(const E* grad_out, const E* u, const E* dt, const fl
                    : (gate ? selective_bwd2_kernel<E, false, true, false> : selective_bwd2_kernel<E, false, false, false>);
     } else if (ml != nullptr) {
       if constexpr (std::is_same_v<E, float>) {
-        kern = a.vec ? (gate ? selective_bwd_kernel<E, true, true, true, false> : selective_bwd_kernel<E, true, false, true, false>)
-                     : (gate ? selective_bwd_kernel<E, false, true, true, false> : selective_bwd_kernel<E, false, false, true, false>);
+        kern = carried ? bwd_kernel<E, true, false, true>(a.vec, gate) : bwd_kernel<E, true, false, false>(a.vec, gate);
       } else {
         return set_error(OSSM_ERR_UNSUPPORTED, std::string(what) + ": the [B, L, D] layout is fp32");
       }
     } else if (dskip != nullptr) {
-      kern = a.vec ? (gate ? selective_bwd_kernel<E, true, true, false, true> : selective_bwd_kernel<E, true, false, false, true>)
-                   : (gate ? selective_bwd_kernel<E, false, true, false, true> : selective_bwd_kernel<E, false, false, false, true>);
+      kern = carried ? bwd_kernel<E, false, true, true>(a.vec, gate) : bwd_kernel<E, false, true, false>(a.vec, gate);
     } else {
-      kern = a.vec ? (gate ? selective_bwd_kernel<E, true, true, false, false> : selective_bwd_kernel<E, true, false, false, false>)
-                   : (gate ? selective_bwd_kernel<E, false, true, false, false> : selective_bwd_kernel<E, false, false, false, false>);
+      kern = carried ? bwd_kernel<E, false, false, true>(a.vec, gate) : bwd_kernel<E, false, false, false>(a.vec, gate);
+    }
+    if (carried) {
+      a.carry.mode = 1;
+      hipLaunchKernelGGL(kern, grid, dim3(kThreads), 0, stream, a);
+      if (int rc = launch_check("selective_bwd_kernel (segment ends)")) return rc;
+      a.carry.mode = 2;
     }
     hipLaunchKernelGGL(kern, grid, dim3(kThreads), 0, stream, a);
     if (int rc = launch_check("selective_bwd_kernel")) return rc;

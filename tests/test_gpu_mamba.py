@@ -143,6 +143,16 @@ def _scan_ref64(u, dt_pre, bias, A, Bg, Cg, z):
 @pytest.mark.parametrize("shape", [(2, 70, 20, 5, 2), (1, 45, 36, 17, 3)],
                          ids=lambda s: "x".join(map(str, s)))
 def test_scan_bld_backward_matches_fp64_autograd(M, shape):
+    _scan_bld_backward(M, shape)
+
+
+# few rows: the time segments' adjoints go through memory
+@pytest.mark.parametrize("shape", [(1, 512, 36, 17, 3), (1, 570, 70, 16, 4)], ids=lambda s: "x".join(map(str, s)))
+def test_scan_bld_backward_segment_carries(M, shape):
+    _scan_bld_backward(M, shape)
+
+
+def _scan_bld_backward(M, shape):
     nb, L, D, N, R = shape
     announce(f"mamba scan bwd B={nb} L={L} D={D} N={N}")
     u, xz, dt_pre, bias, A, proj = _scan_inputs(nb, L, D, N, R, 5)

@@ -152,6 +152,48 @@ def test_selective_forward_both_layouts(K, shape, npw, gated, monkeypatch):
     _check_all(out, grads, *args, what=f"fwd npw{npw} {shape}")
 
 
+# few rows, so the time segments hand their carries on through memory: the fewest
+# segments, ragged tiles, channels and states, and several passes over the states
+SEGMENT_SHAPES = [(1, 1, 512, 1), (1, 70, 533, 16), (2, 40, 2070, 5), (1, 130, 700, 40)]
+
+
+@pytest.mark.parametrize("gated", [True, False], ids=["gate", "nogate"])
+@pytest.mark.parametrize("shape", SEGMENT_SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_selective_segment_carries(K, shape, gated):
+    import torch
+
+    args = selective_inputs(*shape, seed=sum(shape), gated=gated)
+    announce(f"selective segments {shape} gated={gated}")
+    out, chunks, raw, grads = _run(K, *args)
+    _check_all(out, grads, *args, what=f"{shape}")
+    dev = [None if x is None else to_dev(x) for x in args[:6]]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        cap, cap_chunks, _ = K.selective_scan_cuda(*dev)
+    for _ in range(2):
+        graph.replay()
+        torch.cuda.synchronize()
+        # the captured call may have had no memory for the carries
+        assert_close(to_np(cap), to_np(out), RTOL, ATOL, "captured out")
+        assert_close(to_np(cap_chunks), to_np(chunks), RTOL, ATOL, "captured chunk_states")
+
+
+def test_selective_segment_carries_of_infinite_states(K, monkeypatch):
+    """An infinite and an overflowing state cross the segments as they cross steps."""
+    u, dt, A, Bm, Cm, z, g = selective_inputs(1, 4, 640, 16, seed=9, gated=False)
+    u[0, 0, 3], u[0, 1, 350] = np.inf, -np.inf
+    A[2] = 40.0  # grows past the range
+    u[0, 3], A[3] = 0.0, 500.0  # stays zero under transitions that overflow
+    announce("selective segments, infinite states")
+    got, chunks, _ = K.selective_scan_cuda(*[to_dev(x) for x in (u, dt, A, Bm, Cm)], None)
+    monkeypatch.setenv("OSSM_SEL_FWD_NPW", "4")  # the same lanes, segments re-run
+    ref, ref_chunks, _ = K.selective_scan_cuda(*[to_dev(x) for x in (u, dt, A, Bm, Cm)], None)
+    np.testing.assert_allclose(to_np(chunks), to_np(ref_chunks), rtol=RTOL, atol=ATOL)
+    # (row 2's y, a sum of states near the range's end, overflows by their last bits)
+    rows = [0, 1, 3]
+    np.testing.assert_allclose(to_np(got)[:, rows], to_np(ref)[:, rows], rtol=RTOL, atol=ATOL)
+
+
 def test_selective_checkpoints_are_states(K):
     """chunk_states rows hold h after steps 32c+15 and 32c+31 (the final state
     past the end): checked against a brute-force recurrence."""

@@ -137,6 +137,11 @@ def test_selective_bf16_forward_both_layouts(K, shape, npw, monkeypatch):
     _bf16_case(K, shape, True)
 
 
+@pytest.mark.parametrize("shape", [(1, 70, 533, 5), (2, 40, 1025, 24)], ids=lambda s: "x".join(map(str, s)))
+def test_selective_bf16_segment_carries(K, shape):
+    _bf16_case(K, shape, True)
+
+
 def _bf16_case(K, shape, gated):
     import torch
 

@@ -120,6 +120,13 @@ def test_selective_skip_both_layouts(K, shape, npw, monkeypatch):
     check_skip(run_skip(K, *args), args, f"{shape} npw={npw}")
 
 
+@pytest.mark.parametrize("shape", [(1, 70, 533, 5), (2, 40, 1025, 24)], ids=lambda s: "x".join(map(str, s)))
+def test_selective_skip_segment_carries(K, shape):
+    args = skip_inputs(*shape, seed=sum(shape), gated=True)
+    announce(f"selective skip segments {shape}")
+    check_skip(run_skip(K, *args), args, f"{shape}")
+
+
 @pytest.mark.parametrize("npw", [2, 4])
 def test_selective_skip_zero_d_is_the_plain_scan(K, npw, monkeypatch):
     """D = 0: the skip entry points return the plain ones' outputs and
