@@ -6,8 +6,8 @@
 //   LinOSS (linoss.py:209-215):    dt = sigmoid(steps), a = relu(A), g = 0
 // A few hundred values: the time is launches.  As torch operations the D-LinOSS
 // form takes 21 forward launches and about 40 backward, each a host call of about
-// 5 us: a [8, 1030, 100] layer forward 134 us against 39 here (28 of them the
-// layer's own kernel), a [32, 4096, 128] training step 935 against 825.
+// 5 us: with them a [8, 1030, 100] layer forward took 134 us and now takes 32 (25 of
+// them the layer's own kernel); a [32, 4096, 128] training step took 110 us more.
 // The D-LinOSS values are the float operations' own, rounding by rounding (a is
 // a difference of nearly equal terms there, and the layer's unfused form, which
 // runs them, has to agree with the fused one).  The LinOSS values are formed in
