@@ -518,13 +518,13 @@ __device__ __forceinline__ void fold_segments(float (&h)[NPW], const float (&A2)
       const size_t at = (first + step * min(j0 + k, n - 1)) * n_rows + row;
       sdt[k] = c.dt[at];
 #pragma unroll
-      for (int q = 0; q < NPW; ++q) e[k][q] = n0 + q < N ? c.end[at * N + n0 + q] : 0.f;
+      for (int q = 0; q < NPW; ++q) e[k][q] = c.end[at * N + min(n0 + q, N - 1)];
     }
 #pragma unroll
     for (int k = 0; k < kBatch; ++k) {
       if (j0 + k < n) {
 #pragma unroll
-        for (int q = 0; q < NPW; ++q) h[q] = fold_segment(h[q], sdt[k], A2[q], e[k][q]);
+        for (int q = 0; q < NPW; ++q) h[q] = fold_segment(h[q], sdt[k], A2[q], n0 + q < N ? e[k][q] : 0.f);
       }
     }
   }
@@ -2370,27 +2370,32 @@ bool cols_vectorizable(int64_t D, const MambaLayout& ml, std::initializer_list<c
   return true;
 }
 
-// Segments of a problem whose few rows leave the device idle: as many as give
-// `want` workgroups per compute unit, each of at least 64 steps, up to 32, their
-// carries through memory (SegCarry: a launch that runs every segment from zero, then
-// the scan).  Per row the path is 2 L / S steps, against 0.87 to 1.0 L where segments
-// re-run the ones before them (time_segments).  0 below three segments and below 512
-// steps, where the second launch eats what the split saves.  The variables that
-// force another path turn it off.
+// Segments of a problem whose few rows (batch row, 64 channels) leave the device idle,
+// their carries through memory (SegCarry: a launch that runs every segment from zero,
+// then the scan): 2 L / S steps per row, against 0.87 to 1.0 L where segments re-run
+// the ones before them (time_segments).  As many as give the forward one workgroup per
+// compute unit at 64 steps or two at 128 (two run 1.75 times slower each: 32 segments
+// of 64 steps took 47 us where 17 take 37), and the backward two; up to 32.  0 below
+// `least` segments and below 512 steps, where the second launch and the fold eat what
+// the split saves.  The variables that force another path turn it off.
 // fp32, N = 16, gated, forward / backward, us, re-run -> carried:
-//   B, D = 1, 922:  L = 256  16 -> 18 / 28 -> 28,  512  29 -> 22 / 48 -> 35,
-//                   2048  108 -> 40 / 163 -> 70,  8192  419 -> 103 / 618 -> 163
-//   B, D = 27, 80:  L = 256  18 -> 20 / 32 -> 34,  512  33 -> 33 / 55 -> 54,
-//                   2048  119 -> 96 / 190 -> 137
-//   B, D = 16, 512 (forward not split):  1024  74 -> 74 / 177 -> 156
+//   B, D = 1, 922:  L = 256  16 -> 18 / 28 -> 28,  512  29 -> 21 / 48 -> 38,
+//                   2048  107 -> 37 / 161 -> 69,  8192  415 -> 91 / 611 -> 159
+//   B, D = 27, 80:  L = 256  18 -> 20 / 32 -> 34,  1024  62 -> 48 / 97 -> 79,
+//                   8192  456 -> 234 / 717 -> 495
+//   B, D = 12, 512 (5 segments, hence the forward's least):  700  53 -> 56 / 92 -> 94,
+//                   2048  139 -> 120 / 234 -> 248
+//   B, D = 16, 512 (4): 512  38 -> 48 / 91 -> 88,  2048  137 -> 146 / 354 -> 305
 // The outputs' error against float64 is the re-run segments' or smaller (decay over
 // 2000 steps: 5e-7 here, 4e-6 there, one product of the steps' transitions).
-int segment_plan(int64_t n_wg, int64_t L, int want, int n_cu) {
+int segment_plan(int64_t rows64, int64_t L, bool backward, int least, int n_cu) {
   if (L < 512) return 0;
   for (const char* name : {"OSSM_SEL_SPLIT", "OSSM_SEL_FWD_NPW", "OSSM_SEL_BWD_NPW"})
     if (std::getenv(name) != nullptr) return 0;
-  const int64_t s = std::min<int64_t>({static_cast<int64_t>(want) * n_cu / std::max<int64_t>(n_wg, 1), L / 64, 32});
-  return s >= 3 ? static_cast<int>(s) : 0;
+  const int64_t per = n_cu / std::max<int64_t>(rows64, 1), per2 = 2 * n_cu / std::max<int64_t>(rows64, 1);
+  const int64_t s = std::min<int64_t>(
+      backward ? std::min(per2, (L + 63) / 64) : std::max(std::min(per, (L + 63) / 64), std::min(per2, L / 128)), 32);
+  return s >= least ? static_cast<int>(s) : 0;
 }
 
 // Time segments per (batch row, channel tile), 1, 2 or 4: the fewest that
@@ -2537,7 +2542,7 @@ int selective_forward_impl(const E* u, const E* dt, const float* A, const E* Bm,
   // would leave the SIMDs short of waves, else 4; the [B, L, D] layout runs 4
   // and few rows run time segments, 4 states per lane (segment_plan)
   const int64_t rows64 = batch * ((dim + kWave - 1) / kWave);
-  int n_seg = segment_plan(rows64, length, kFwdWgPerCu, device_cu_count(call.device()));
+  int n_seg = segment_plan(rows64, length, false, length < 1024 ? 8 : 5, device_cu_count(call.device()));
   if (n_seg > 0) {
     // the fp32 sums of several bf16 passes, then the segments' ends and sums of dt
     const size_t acc_n = n_pass > 1 && !std::is_same_v<E, float> ? static_cast<size_t>(batch * dim * length) : 0;
@@ -2629,7 +2634,11 @@ int selective_backward_impl(const E* grad_out, const E* u, const E* dt, const fl
   // few rows: segments with carried adjoints (the 4-states kernel), else one of
   // the kernels with the segments it re-runs
   const int64_t rows64 = batch * ((dim + kWave - 1) / kWave);
-  int n_seg = segment_plan(rows64, length, kBwdWgPerCu, device_cu_count(call.device()));
+  // (where the 2-states kernel runs its four in one round of the device, five or fewer
+  // carried ones are no faster: 234 -> 248 us at B, D, L = 12, 512, 2048)
+  const int n_cu = device_cu_count(call.device());
+  const bool one_round = ml == nullptr && 4 * batch * ((dim + kB2Rows - 1) / kB2Rows) <= int64_t(kBwd2WgPerCu) * n_cu;
+  int n_seg = segment_plan(rows64, length, true, one_round ? 6 : 3, n_cu);
   bool carried = n_seg > 0, npw2 = false;
   int64_t n_dtiles = 0, dA_rows = 0;
   const int64_t n_bln = batch * length * dstate;
