@@ -727,7 +727,9 @@ int chunks64(int64_t L, int64_t nc) {
 // grow; a full device) the call runs as one chunk, which needs only the sums.
 template <class Sums>
 int plan64(StreamCall& call, int64_t L, int64_t nc, bool varying, Sums sums, Plan64* pl, double** part) {
-  int n = chunks64(L, nc);
+  // a captured call without sums takes no workspace, so that its graph may replay
+  // beside the capture stream's own work
+  int n = call.capturing() && sums(1) == 0 ? 1 : chunks64(L, nc);
   for (;;) {
     const size_t rows = n > 1 ? static_cast<size_t>(n) * nc : 0;
     const size_t n_sums = (sums(n) + 1) & ~size_t(1);  // 16-byte aligned double2 behind them

@@ -2543,9 +2543,12 @@ int selective_forward_impl(const E* u, const E* dt, const float* A, const E* Bm,
   // and few rows run time segments, 4 states per lane (segment_plan)
   const int64_t rows64 = batch * ((dim + kWave - 1) / kWave);
   int n_seg = segment_plan(rows64, length, false, length < 1024 ? 8 : 5, device_cu_count(call.device()));
+  const size_t acc_n = n_pass > 1 && !std::is_same_v<E, float> ? static_cast<size_t>(batch * dim * length) : 0;
+  // a captured call that needs no workspace otherwise takes none here, so that its
+  // graph may replay beside the capture stream's own work
+  if (call.capturing() && acc_n == 0) n_seg = 0;
   if (n_seg > 0) {
     // the fp32 sums of several bf16 passes, then the segments' ends and sums of dt
-    const size_t acc_n = n_pass > 1 && !std::is_same_v<E, float> ? static_cast<size_t>(batch * dim * length) : 0;
     const size_t rows_n = static_cast<size_t>(n_seg) * batch * dim;
     void* ws = nullptr;
     if (acquire_workspace(call, (acc_n + rows_n * (dstate + 1)) * sizeof(float), &ws)) {

@@ -173,7 +173,7 @@ def test_selective_segment_carries(K, shape, gated):
     for _ in range(2):
         graph.replay()
         torch.cuda.synchronize()
-        # the captured call may have had no memory for the carries
+        # a captured forward takes no workspace: its segments are re-run
         assert_close(to_np(cap), to_np(out), RTOL, ATOL, "captured out")
         assert_close(to_np(cap_chunks), to_np(chunks), RTOL, ATOL, "captured chunk_states")
 
