@@ -946,22 +946,27 @@ __global__ __launch_bounds__(kLayerThreads) void dlinoss_layer_bwd_kernel(
   }
 }
 
-// grad_D[h] = the workgroups' sums: 16 columns by 16 row lanes, in order, in double.
-__global__ __launch_bounds__(256) void layer_grad_d_kernel(const float* __restrict__ part, float* __restrict__ out,
-                                                           int rows, int H) {
-  __shared__ double s_p[16][16];
-  const int cl = threadIdx.x & 15, rl = threadIdx.x >> 4, h = blockIdx.x * 16 + cl;
+// grad_D[h] = the workgroups' sums, in a fixed order, in double: 8 columns (32-byte
+// runs) by 128 row lanes.  Bound by load latency: 16 columns by 16 lanes, 8 workgroups
+// of 256 rows a lane, took 16 us for [4096, 128]; this 9.
+constexpr int kGdCols = 8, kGdLanes = 128;
+
+__global__ __launch_bounds__(kGdCols * kGdLanes) void layer_grad_d_kernel(const float* __restrict__ part,
+                                                                          float* __restrict__ out, int rows, int H) {
+  __shared__ double s_p[kGdLanes][kGdCols];
+  const int cl = threadIdx.x % kGdCols, rl = threadIdx.x / kGdCols, h = blockIdx.x * kGdCols + cl;
   double s = 0.0;
   if (h < H) {
 #pragma unroll 8
-    for (int r = rl; r < rows; r += 16) s += part[static_cast<size_t>(r) * H + h];
+    for (int r = rl; r < rows; r += kGdLanes) s += part[static_cast<size_t>(r) * H + h];
   }
   s_p[rl][cl] = s;
-  __syncthreads();
-  if (rl != 0 || h >= H) return;
 #pragma unroll
-  for (int v = 1; v < 16; ++v) s += s_p[v][cl];
-  out[h] = static_cast<float>(s);
+  for (int n = kGdLanes / 2; n > 0; n /= 2) {
+    __syncthreads();
+    if (rl < n) s_p[rl][cl] = s += s_p[rl + n][cl];
+  }
+  if (rl == 0 && h < H) out[h] = static_cast<float>(s);
 }
 
 int launch_split_weights(const SplitW& g0, const SplitW& g1, const SplitW& g2, int n, int H, int P,
@@ -1072,8 +1077,8 @@ int launch_layer_bwd(LayerBwdArgs args, float* ga, float* gg, float* gs, float* 
                      static_cast<unsigned long long*>(payload), sync);
   if (int rc = launch_check("dlinoss_layer_bwd_kernel")) return rc;
   if (grad_d != nullptr) {
-    hipLaunchKernelGGL(layer_grad_d_kernel, dim3(static_cast<unsigned>((args.H + 15) / 16)), dim3(256), 0, stream,
-                       args.part_d, grad_d, static_cast<int>(n_wg), args.H);
+    hipLaunchKernelGGL(layer_grad_d_kernel, dim3(static_cast<unsigned>((args.H + kGdCols - 1) / kGdCols)),
+                       dim3(kGdCols * kGdLanes), 0, stream, args.part_d, grad_d, static_cast<int>(n_wg), args.H);
     if (int rc = launch_check("layer_grad_d_kernel")) return rc;
   }
   if (args.P == 0) return OSSM_OK;
