@@ -13,7 +13,8 @@
 //   2. scan64_{fwd,bwd}_kernel: each (chunk, channel) folds the aggregates of
 //      the chunks before it (after it, in reverse) into its carry, with the
 //      chunk transition M^CL formed once per lane by binary powering (or the
-//      stored products), and walks its steps again from that carry, writing the
+//      stored products; a carry that is not finite is walked step by step
+//      instead), and walks its steps again from that carry, writing the
 //      outputs.  Consecutive lanes own consecutive channels, so every load and
 //      store of a wave is one contiguous run.
 // Bound by HBM: a forward reads bu twice (the second time largely from the
@@ -427,6 +428,11 @@ struct Plan64 {
   RMatD* tr;
 };
 
+// Whether every component is finite (x - x is 0, or NaN for infinities and NaN).
+__device__ __forceinline__ bool st_finite(St s) {
+  return (s.x - s.x) + (s.y - s.y) + (s.z - s.z) + (s.w - s.w) == 0.0;
+}
+
 template <class M>
 __global__ __launch_bounds__(kWave) void chunk64_fwd_kernel(typename M::Params prm,
                                                             const double2* __restrict__ in, Plan64 pl) {
@@ -471,6 +477,17 @@ __global__ __launch_bounds__(kWave) void scan64_fwd_kernel(typename M::Params pr
 #pragma unroll 8
       for (int j = 0; j < c; ++j)
         s = st_add(st_apply(MC, s), load_st(pl.agg + 2 * (static_cast<size_t>(j) * pl.nc + ch)));
+    }
+    // A chunk's transition may overflow where no state does (times zero: NaN), and an
+    // infinite state goes on step by step in its own way: walk the steps before the
+    // chunk instead, which takes what one lane per sequence took.
+    if (!st_finite(s)) {
+      s = st_zero();
+#pragma unroll 4
+      for (int t = 0; t < t0; ++t) {
+        if constexpr (M::kVarying) k = M::coef(prm, t, ch, m);
+        s = M::step(k, s, M::load_in(in, static_cast<size_t>(t) * pl.nc + ch));
+      }
     }
   }
 #pragma unroll 8
@@ -530,6 +547,14 @@ __global__ __launch_bounds__(kWave) void scan64_bwd_kernel(
 #pragma unroll 8
       for (int j = pl.n_chunks - 1; j > c; --j)
         y = st_add(st_apply(MC, y), load_st(pl.agg + 2 * (static_cast<size_t>(j) * pl.nc + ch)));
+    }
+    if (!st_finite(y)) {  // as in scan64_fwd_kernel
+      y = st_zero();
+#pragma unroll 4
+      for (int t = pl.L - 1; t >= t1; --t) {
+        if constexpr (M::kVarying) k = M::coef(prm, t, ch, m);
+        y = M::rev(k, M::mu(y, M::load_in(gout, static_cast<size_t>(t) * pl.nc + ch)));
+      }
     }
   }
   double acc[M::kSums];

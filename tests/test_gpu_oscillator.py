@@ -183,6 +183,61 @@ def test_complex128_scans_chunk_edges(K, shape):
         np.testing.assert_allclose(to_np(got), r, rtol=1e-10, atol=1e-12 * max(1.0, float(np.abs(r).max())))
 
 
+def _unstable_inputs(rng, L):
+    """Four channels of an L-step scan whose transition grows about 1e6 times a step
+    (so that a chunk's power of it overflows), but for the second, a stable one:
+    never driven; stable, with a NaN at step 2000; driven in the last 3 steps; driven
+    from step 100, so that it overflows on the way."""
+    x = rng.normal(size=(L, 1, 4)) + 1j * rng.normal(size=(L, 1, 4))
+    x[:, :, 0] = 0
+    x[2000, 0, 1] = np.nan
+    x[:L - 3, :, 2] = 0
+    x[:100, :, 3] = 0
+    return x
+
+
+def _same_values(got, want, what):
+    """rtol 1e-10, and NaN and infinities in the same places."""
+    view = lambda z: np.ascontiguousarray(z).view(np.float64)  # noqa: E731
+    np.testing.assert_allclose(view(got), view(want), rtol=1e-10, atol=1e-12, err_msg=what)
+
+
+@pytest.mark.parametrize("variant", VARIANTS)
+def test_dlinoss_complex128_chunks_keep_zeros_and_infinities(K, variant):
+    """A chunk's transition may overflow where no state does: chunked scans give what
+    walking the steps one by one gives."""
+    L = 4096
+    rng = np.random.default_rng(17)
+    a = np.full(4, {"imex1": 1e6, "imex2": 1e6, "im": -0.999999, "ex": 1e12}[variant])
+    g, dt = np.zeros(4), np.ones(4)
+    a[1], dt[1], g[1] = 0.3, 0.25, 0.5
+    bu, go = _unstable_inputs(rng, L), _unstable_inputs(rng, L)[::-1].copy()
+    announce(f"complex128 unstable chunks dlinoss {variant}")
+    with np.errstate(all="ignore"):
+        ref = oracle.dlinoss_forward(variant, a, g, dt, bu)
+        st = _fwd(K, variant, a, g, dt, bu)
+        _same_values(to_np(st), ref, "states")
+        rgb = oracle.dlinoss_backward(variant, a, g, dt, bu, ref, go)[3]
+        gb = _bwd(K, variant, a, g, dt, bu, to_dev(ref), go)[3]
+        _same_values(to_np(gb), rgb, "grad_bu")
+
+
+def test_linoss_complex128_chunks_keep_zeros_and_infinities(K):
+    """As above: M = diag(1e6, 0.5), driven in its second component or late."""
+    L = 4096
+    rng = np.random.default_rng(18)
+    ms = [np.full(4, v, np.complex128) for v in (1e6, 0, 0, 0.5)]
+    ms[0][1] = 0.9
+    b = np.stack([_unstable_inputs(rng, L), rng.normal(size=(L, 1, 4)) + 0j], -1)
+    go = np.stack([_unstable_inputs(rng, L)[::-1], rng.normal(size=(L, 1, 4)) + 0j], -1)
+    announce("complex128 unstable chunks linoss")
+    with np.errstate(all="ignore"):
+        ref = oracle.linoss_forward(*ms, b)
+        _same_values(to_np(K.linoss_scan(*[to_dev(m) for m in ms], to_dev(b))), ref, "states")
+        gb = K.linoss_scan_backward(*[to_dev(m) for m in ms], to_dev(ref), to_dev(go))[1]
+        _same_values(to_np(gb), oracle.linoss_backward(*ms, ref, go)[1], "grad_b")
+
+
 def test_complex128_forward_captured_without_workspace(K):
     """The complex128 forward allocated nothing before it was chunked, so a
     capture on a fresh stream, whose workspace may not grow, still goes

@@ -275,6 +275,32 @@ def test_sdlinoss_complex128_chunk_edges(K, shape, tag):
         assert_close(to_np(got), ref, RTOL64, ATOL64 * max(1.0, float(np.abs(ref).max())), name)
 
 
+@pytest.mark.parametrize("tag", ["m", "full"])
+@pytest.mark.parametrize("variant", VARIANTS)
+def test_sdlinoss_complex128_chunks_keep_zeros_and_infinities(K, variant, tag):
+    """Transitions that grow 1e6 times a step (S at its clamp, or a large A) overflow
+    over a chunk where a channel that is not driven, or late, stays finite."""
+    from tests.test_gpu_oscillator import _same_values, _unstable_inputs
+
+    L = 4096
+    rng = np.random.default_rng(19)
+    A = np.full(4, {"imex1": 0.3, "imex2": -1.0, "im": -1.0, "ex": 1e12}[variant])
+    G = np.full(4, -1.0 if variant == "imex1" else 0.0)
+    S = np.ones(4)
+    A[1], G[1], S[1] = 0.3, 0.5, 0.25
+    if tag == "full":
+        A, G, S = (np.broadcast_to(x, (L, 1, 4)).copy() for x in (A, G, S))
+    bu, go = _unstable_inputs(rng, L), _unstable_inputs(rng, L)[::-1].copy()
+    announce(f"sdlinoss c128 unstable chunks {variant} {tag}")
+    with np.errstate(all="ignore"):
+        ref = oracle.sdlinoss_forward(variant, A, G, S, bu)
+        args = [to_dev(x) for x in (A, G, S, bu)]
+        st = getattr(K, f"sdlinoss_{variant}_forward")(*args)
+        _same_values(to_np(st), ref, "states")
+        gb = getattr(K, f"sdlinoss_{variant}_backward")(*args, to_dev(ref), to_dev(go))[3]
+        _same_values(to_np(gb), oracle.sdlinoss_backward(variant, A, G, S, bu, ref, go)[3], "grad_bu")
+
+
 def test_sdlinoss_complex128_golden_and_edges(K):
     """The reference kernel vectors in fp64 (bound set by their fp32
     arithmetic), one-step and single-channel shapes, and empty inputs."""
