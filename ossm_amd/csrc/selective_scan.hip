@@ -63,7 +63,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <cfloat>
 #include <cstdlib>
 #include <climits>
 #include <initializer_list>
@@ -486,22 +485,30 @@ __device__ __forceinline__ void store_states(float* __restrict__ s, const StateR
 // segment re-runs the recurrence over the segments it depends on; 1: it only runs
 // its own, from zero, and stores where that ends and its sum of dt (the transition
 // of state n over the segment is exp(A_n sum dt)); 2: it folds the stored ones
-// into its carry.
+// into its carry, and does as in mode 0 where that leaves the range.
 struct SegCarry {
   int mode;
   float* end;  // [segment][B, D][N]
   float* dt;   // [segment][B, D]
 };
 
-// h past a segment that ends at `end` from zero, `sdt` its sum of dt.  Infinities go
-// on as they do step by step: a zero state leaves the transition unread, an infinite
-// one stays (their products with an overflowed or underflowed transition would be
-// NaN), and one that overflows here keeps its sign, the earlier growth's.
+// h past a segment that ends at `end` from zero, `sdt` its sum of dt: the
+// transition exp(A sdt) in two halves, since it may leave the range where its product
+// with the state does not (1e-20 under e^100).  A zero state leaves it unread.  What
+// still comes out infinite or NaN is walked step by step (left_range).
 __device__ __forceinline__ float fold_segment(float h, float sdt, float A2, float end) {
   if (h == 0.f) return end;
-  float f = fast_exp2(sdt * A2);
-  if (fabsf(h) == INFINITY) f = fmaxf(f, FLT_MIN);
-  return fabsf(f * h) == INFINITY && fabsf(end) == INFINITY ? f * h : fmaf(f, h, end);
+  const float f = fast_exp2(0.5f * sdt * A2);
+  return fmaf(f * h, f, end);
+}
+
+// Whether any state of the workgroup is infinite or NaN.  Every thread calls it.
+template <int NPW>
+__device__ __forceinline__ bool left_range(const float (&h)[NPW]) {
+  float s = 0.f;
+#pragma unroll
+  for (int q = 0; q < NPW; ++q) s += h[q] - h[q];
+  return __syncthreads_or(s != 0.f);
 }
 
 // The carry of one row's states [n0, n0 + NPW) past segments first, first + step, ..
@@ -850,11 +857,19 @@ __global__ __launch_bounds__(kThreads) void selective_fwd_kernel(FwdArgs<E> a) {
   float zn[SEG];  // the gate of the lane's output segment, one tile ahead
   // the tiles h alone runs over: those before the segment, or (mode 1) its own
   const bool ends = CARRY && a.carry.mode == 1;
-  const int r_lo = CARRY ? t_lo : 0, r_hi = CARRY ? (ends ? t_hi : t_lo) : t_lo;
+  int r_lo = CARRY ? t_lo : 0;
+  const int r_hi = ends ? t_hi : t_lo;
   const size_t seg_row = static_cast<size_t>(b) * a.D + dc, n_rows = static_cast<size_t>(gridDim.y) * a.D;
   if constexpr (CARRY) {
     if (ends && seg == n_seg - 1) return;  // nothing reads the last one's end
-    if (!ends) fold_segments(h, A2, a.carry, 0, 1, seg, n_rows, seg_row, a.N, n0);
+    if (!ends) {
+      fold_segments(h, A2, a.carry, 0, 1, seg, n_rows, seg_row, a.N, n0);
+      if (left_range(h)) {
+#pragma unroll
+        for (int j = 0; j < NPW; ++j) h[j] = 0.f;
+        r_lo = 0;
+      }
+    }
   }
   fwd_prefetch<E, VEC, BLD>(nxt, a, row0, bc0, d0, r_lo);
   float sum_dt = 0.f;
@@ -1224,12 +1239,20 @@ __global__ __launch_bounds__(kThreads) void selective_bwd_kernel(BwdArgs<E> a) {
   const int tile_hi = (seg + 1) * n_tiles / n_seg;
   // the tiles the adjoint alone runs over: those after the segment, or (mode 1) its own
   const bool ends = CARRY && a.carry.mode == 1;
-  const int r_hi = CARRY ? tile_hi : n_tiles, r_lo = ends ? tile_lo : tile_hi;
+  int r_hi = CARRY ? tile_hi : n_tiles;
+  const int r_lo = ends ? tile_lo : tile_hi;
   const size_t seg_row = static_cast<size_t>(b) * a.D + (dvalid ? d : a.D - 1);
   const size_t n_rows = static_cast<size_t>(a.Bsz) * a.D;
   if (ends && seg == 0) return;  // nothing reads the first one's
-  if (CARRY && wave_active && !ends)
-    fold_segments(gs, A2, a.carry, n_seg - 1, -1, n_seg - 1 - seg, n_rows, seg_row, a.N, n0);
+  if (CARRY && !ends) {
+    if (wave_active)
+      fold_segments(gs, A2, a.carry, n_seg - 1, -1, n_seg - 1 - seg, n_rows, seg_row, a.N, n0);
+    if (left_range(gs)) {
+#pragma unroll
+      for (int j = 0; j < kNpw; ++j) gs[j] = 0.f;
+      r_hi = n_tiles;
+    }
+  }
   if (r_lo < r_hi) {
     AdjTile p;
     float sum_dt = 0.f;

@@ -194,6 +194,27 @@ def test_selective_segment_carries_of_infinite_states(K, monkeypatch):
     np.testing.assert_allclose(to_np(got)[:, rows], to_np(ref)[:, rows], rtol=RTOL, atol=ATOL)
 
 
+def test_selective_segment_carries_past_the_range_of_a_transition(K):
+    """exp(A sum dt) of a segment overflows (row 0) or underflows (row 1) where the
+    state it carries on stays in range; each way, against the fp64 oracle."""
+    L = 640
+    dt = np.full((1, 2, L), 1e-3, np.float32)
+    dt[:, :, 192:256] = 100.0 / 64  # one segment: e^100 and e^-100
+    A = np.array([[1.0], [-1.0]], np.float32)
+    Bm = Cm = np.ones((1, L, 1), np.float32)
+    u, g = np.zeros((2, 1, 2, L), np.float32)
+    u[0, 0, 5], u[0, 1, 5] = 1e-17, 1e33
+    g[0, 0, L - 5], g[0, 1, L - 5] = 1e-17, 1e33
+    announce("selective segments past a transition's range")
+    dev = [to_dev(x) for x in (u, dt, A, Bm, Cm)]
+    out, chunks, raw = K.selective_scan_cuda(*dev, None)
+    du = K.selective_scan_cuda_backward(to_dev(g), *dev, None, chunks, raw, 16)[0]
+    f64 = [x.astype(np.float64) for x in (u, dt, A, Bm, Cm)]
+    # 64 steps' rounded exponents on each side: below 1e-4
+    np.testing.assert_allclose(to_np(out), oracle.selective_forward(*f64), rtol=1e-4)
+    np.testing.assert_allclose(to_np(du), oracle.selective_backward(g.astype(np.float64), *f64)[0], rtol=1e-4)
+
+
 def test_selective_checkpoints_are_states(K):
     """chunk_states rows hold h after steps 32c+15 and 32c+31 (the final state
     past the end): checked against a brute-force recurrence."""
