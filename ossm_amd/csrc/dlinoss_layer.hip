@@ -71,13 +71,17 @@ constexpr int kBwdGroups = kLayerMax / 32 / kLayerWaves;
 // the compiler then keeps them in flight instead of waiting for each.
 constexpr int kAhead = 4;
 
-__device__ __forceinline__ floatx16 mfma32(float a, float b, floatx16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-}
-
 __device__ __forceinline__ int round32(int n) { return (n + 31) & ~31; }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+
+// A weight matrix of the split projections (see split_weights_kernel).
+struct SplitW {
+  const float* w;
+  uint4* out;
+  int w_is_c;  // C [H, P, 2], else B [P, H, 2]
+  int in_form;
+};
 
 struct LayerArgs {
   const float* u;   // [B, L, H]
@@ -88,11 +92,10 @@ struct LayerArgs {
   const float* g;
   const float* dt;
   const float* lo;  // [3, P]: what a, g, dt leave of their double values; may be null
-  const uint4* w_in;   // SPLIT: split weights of the in- and out-projection (SplitW)
-  const uint4* w_out;
   float* y;         // [B, L, H]
   float4* carries;  // [B, n_chunks, P]: state entering each chunk (for the backward); may be null
   int Bsz, L, H, P, n_chunks;
+  SplitW w_in, w_out;  // SPLIT: the in- and out-projection's weights
 };
 
 // Oscillator p's coefficients; with lo, from its parameters in double.
@@ -221,13 +224,6 @@ __device__ __forceinline__ void stage_store(const RowStage<SK>& r, float* __rest
 // [l]; columns and k outside the tensor hold zeros, so the loops need no masks.
 // "in" form: column p, k = h, components re and im (NC = 2); "out" form: column
 // h, k = 2 p + component (NC = 1).
-struct SplitW {
-  const float* w;
-  uint4* out;
-  int w_is_c;  // C [H, P, 2], else B [P, H, 2]
-  int in_form;
-};
-
 __device__ __forceinline__ float weight_at(const SplitW& g, int H, int P, int h, int p, int c) {
   if (h >= H || p >= P) return 0.f;
   return g.w[(g.w_is_c ? static_cast<size_t>(h) * P + p : static_cast<size_t>(p) * H + h) * 2 + c];
@@ -266,11 +262,34 @@ __global__ __launch_bounds__(kSplitThreads) void split_weights_kernel(SplitW g0,
   dst[2 * kWave] = __builtin_bit_cast(uint4, f.t2);
 }
 
+// acc[c] = A (32 rows, fp32 in LDS; row: the lane's) times the weights of column
+// group cg, in fp32 and as they lie in memory: for sums that left the range of the
+// split ones.  K: the padded number of k.
+template <int NC>
+__device__ __forceinline__ void exact_project(const float* row, const SplitW& g, int H, int P, int cg, int K,
+                                              floatx16 (&acc)[NC]) {
+  int lane = threadIdx.x & (kWave - 1);
+  asm volatile("" : "+v"(lane));  // keeps this path's values out of the registers of the others
+  const int half = lane >> 5, col = cg * 32 + (lane & 31);
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[c][r] = 0.f;
+#pragma unroll 2
+  for (int k2 = 0; k2 < K; k2 += 2) {
+    const int k = k2 + half;
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+      acc[c] = mfma32(row[k], NC == 2 ? weight_at(g, H, P, k, col, c) : weight_at(g, H, P, col, k / 2, k & 1),
+                        acc[c]);
+  }
+}
+
 // acc[c] += A (32 rows, fp32 in LDS; arow: the lane's row from its first k) times
 // the split weights of one column group over S k-steps.  Weights AH steps ahead.
 template <int NC, int AH>
-__device__ __forceinline__ void split_project(const float* arow, const uint4* __restrict__ w, int S,
-                                              floatx16 (&acc)[NC]) {
+__device__ __forceinline__ void split_sums(const float* arow, const uint4* __restrict__ w, int S,
+                                           floatx16 (&acc)[NC]) {
   constexpr int kStep = NC * 3 * kWave;
   w += threadIdx.x & (kWave - 1);
   uint4 wb[AH][NC][3];
@@ -304,6 +323,15 @@ __device__ __forceinline__ void split_project(const float* arow, const uint4* __
       __builtin_amdgcn_sched_barrier(0);
     }
   }
+}
+
+// acc[c] (zero) += A (row: the lane's, in LDS) times the weights of column group cg.
+template <int NC, int AH>
+__device__ __forceinline__ void split_project(const float* row, const SplitW& g, int H, int P, int cg, int S,
+                                              floatx16 (&acc)[NC]) {
+  const int half = (threadIdx.x & (kWave - 1)) >> 5;
+  split_sums<NC, AH>(row + 8 * half, g.out + static_cast<size_t>(cg) * S * (NC * 3 * kWave), S, acc);
+  if (any_nonfinite(acc)) exact_project<NC>(row, g, H, P, cg, 16 * S, acc);
 }
 
 // SMALL: Hp, Pp <= 128 (one oscillator group per wave, four row groups per
@@ -372,8 +400,7 @@ void dlinoss_layer_fwd_kernel(
       for (int r = 0; r < 16; ++r) acc_re[i][r] = acc_im[i][r] = 0.f;
       if constexpr (SPLIT) {
         floatx16 acc[2] = {acc_re[i], acc_im[i]};
-        const int S = Hp / 16;
-        split_project<2, SMALL ? 1 : 2>(sU + m * HS + 8 * half, A.w_in + static_cast<size_t>(pg) * S * 6 * kWave, S, acc);
+        split_project<2, SMALL ? 1 : 2>(sU + m * HS, A.w_in, A.H, A.P, pg, Hp / 16, acc);
         acc_re[i] = acc[0];
         acc_im[i] = acc[1];
         continue;
@@ -496,8 +523,7 @@ void dlinoss_layer_fwd_kernel(
         uv[r] = A.u[row0 + static_cast<size_t>(min(acc_row(r, lane), nt - 1)) * A.H + min(h, A.H - 1)];
       if constexpr (SPLIT) {
         floatx16 one[1] = {acc};
-        const int S = Pp / 8;
-        split_project<1, SMALL ? 1 : 2>(sX + m * XS + 8 * kk, A.w_out + static_cast<size_t>(hg) * S * 3 * kWave, S, one);
+        split_project<1, SMALL ? 1 : 2>(sX + m * XS, A.w_out, A.H, A.P, hg, Pp / 8, one);
         acc = one[0];
       } else {
       float4 cb[AH];
@@ -566,9 +592,6 @@ struct LayerBwdArgs {
   const float* g;
   const float* dt;
   const float* lo;       // as LayerArgs::lo
-  const uint4* w_gx;     // SPLIT: split weights of the g_x, bu and grad_u projections
-  const uint4* w_bu;
-  const uint4* w_gu;
   const float4* carries; // [B, n_chunks, P] from the forward
   float* grad_u;         // [B, L, H]
   float2* grad_bu;       // [B, L, P] (re, im)
@@ -577,6 +600,7 @@ struct LayerBwdArgs {
   float* part_d;         // [workgroup][H]: sums of gy u over the chunk's steps, or null
   ZeroFill zero;         // grad a, g, dt, cleared by the first workgroup
   int Bsz, L, H, P, n_chunks;
+  SplitW w_gx, w_bu, w_gu;  // SPLIT: the weights of the g_x, bu and grad_u projections
 };
 
 // Weights of the g_x projection for oscillator p and h = h0 .. h0 + 3:
@@ -675,8 +699,7 @@ __global__ __launch_bounds__(kLayerThreads) void dlinoss_layer_bwd_kernel(
       for (int r = 0; r < 16; ++r) acc_re[r] = acc_im[r] = 0.f;
       if constexpr (SPLIT) {
         floatx16 acc[2] = {acc_re, acc_im};
-        const int S = Hp / 16;
-        split_project<2, 2>(sA + m * HS + 8 * half, A.w_gx + static_cast<size_t>(pg) * S * 6 * kWave, S, acc);
+        split_project<2, 2>(sA + m * HS, A.w_gx, A.H, A.P, pg, Hp / 16, acc);
         acc_re = acc[0];
         acc_im = acc[1];
       } else {
@@ -768,8 +791,7 @@ __global__ __launch_bounds__(kLayerThreads) void dlinoss_layer_bwd_kernel(
       for (int r = 0; r < 16; ++r) acc_re[i][r] = acc_im[i][r] = 0.f;
       if constexpr (SPLIT) {
         floatx16 acc[2] = {acc_re[i], acc_im[i]};
-        const int S = Hp / 16;
-        split_project<2, 2>(sA + m * HS + 8 * half, A.w_bu + static_cast<size_t>(pg) * S * 6 * kWave, S, acc);
+        split_project<2, 2>(sA + m * HS, A.w_bu, A.H, A.P, pg, Hp / 16, acc);
         acc_re[i] = acc[0];
         acc_im[i] = acc[1];
         continue;
@@ -906,8 +928,7 @@ __global__ __launch_bounds__(kLayerThreads) void dlinoss_layer_bwd_kernel(
         gyv[r] = A.gy[row0 + static_cast<size_t>(min(acc_row(r, lane), nt - 1)) * A.H + min(h, A.H - 1)];
       if constexpr (SPLIT) {
         floatx16 one[1] = {acc};
-        const int S = Pp / 8;
-        split_project<1, 2>(sG + m * XS + 8 * kk, A.w_gu + static_cast<size_t>(hg) * S * 3 * kWave, S, one);
+        split_project<1, 2>(sG + m * XS, A.w_gu, A.H, A.P, hg, Pp / 8, one);
         acc = one[0];
       } else {
       float4 cb[kAhead];
@@ -1052,12 +1073,10 @@ int launch_layer_bwd(LayerBwdArgs args, float* ga, float* gg, float* gs, float* 
   args.part_d = grad_d != nullptr ? args.partials + n_part : nullptr;
   if (split) {
     auto* w = reinterpret_cast<uint4*>(static_cast<char*>(ws) + part_bytes);
-    args.w_gx = w;
-    args.w_bu = w + w_uint4;
-    args.w_gu = w + 2 * w_uint4;
-    if (int rc = launch_split_weights({args.Cw, w, 1, 1}, {args.Bw, w + w_uint4, 0, 1},
-                                      {args.Bw, w + 2 * w_uint4, 0, 0}, 3, args.H, args.P, stream))
-      return rc;
+    args.w_gx = {args.Cw, w, 1, 1};
+    args.w_bu = {args.Bw, w + w_uint4, 0, 1};
+    args.w_gu = {args.Bw, w + 2 * w_uint4, 0, 0};
+    if (int rc = launch_split_weights(args.w_gx, args.w_bu, args.w_gu, 3, args.H, args.P, stream)) return rc;
   }
   args.zero = ZeroFill{{ga, gg, gs}, {args.P, args.P, args.P}};
   const bool pad = args.H % 32 != 0 || args.P % 32 != 0;
@@ -1116,10 +1135,9 @@ int launch_layer(LayerArgs args, hipStream_t stream) {
       split = false;
     } else {
       auto* w = static_cast<uint4*>(ws);
-      args.w_in = w;
-      args.w_out = w + n;
-      if (int rc = launch_split_weights({args.Bw, w, 0, 1}, {args.Cw, w + n, 1, 0}, {}, 2, args.H, args.P, stream))
-        return rc;
+      args.w_in = {args.Bw, w, 0, 1};
+      args.w_out = {args.Cw, w + n, 1, 0};
+      if (int rc = launch_split_weights(args.w_in, args.w_out, {}, 2, args.H, args.P, stream)) return rc;
     }
   }
   const bool pad = args.H % 32 != 0 || args.P % 32 != 0;
@@ -1173,7 +1191,7 @@ int ossm_dlinoss_layer_forward_wide(int variant, const float* inputs, const floa
     return set_error(OSSM_ERR_UNSUPPORTED, std::string(what) + ": size exceeds 32-bit indexing");
   if (!inputs || !D || !outputs || (ssm > 0 && (!B || !C || !a_diag || !g_diag || !step)))
     return set_error(OSSM_ERR_INVALID_ARGUMENT, std::string(what) + ": null pointer");
-  LayerArgs args{inputs, B, C, D, a_diag, g_diag, step, params_lo, nullptr, nullptr, outputs, static_cast<float4*>(carries),
+  LayerArgs args{inputs, B, C, D, a_diag, g_diag, step, params_lo, outputs, static_cast<float4*>(carries),
                  static_cast<int>(batch), static_cast<int>(length), static_cast<int>(hidden),
                  static_cast<int>(ssm), static_cast<int>(n_chunks)};
   hipStream_t stream = static_cast<hipStream_t>(stream_v);
@@ -1232,7 +1250,7 @@ int ossm_dlinoss_layer_backward_wide(int variant, const float* inputs, const flo
   if (!inputs || !grad_output || !D || !grad_inputs ||
       (ssm > 0 && (!B || !C || !a_diag || !g_diag || !step || !carries || !grad_bu || !x_conj)))
     return set_error(OSSM_ERR_INVALID_ARGUMENT, std::string(what) + ": null pointer");
-  LayerBwdArgs args{inputs, grad_output, B, C, D, a_diag, g_diag, step, params_lo, nullptr, nullptr, nullptr,
+  LayerBwdArgs args{inputs, grad_output, B, C, D, a_diag, g_diag, step, params_lo,
                     static_cast<const float4*>(carries), grad_inputs,
                     static_cast<float2*>(grad_bu), static_cast<float2*>(x_conj), nullptr, nullptr,
                     ZeroFill{}, static_cast<int>(batch), static_cast<int>(length),

@@ -74,6 +74,40 @@ __device__ __forceinline__ unsigned clamp_col(int c0, int j, int n) {
   return static_cast<unsigned>(min(c0 + j / V * V, n - V) + j % V);
 }
 
+// A wave's tile in fp32, for sums that left the range of the split products
+// (split_mfma.hpp).
+__device__ __forceinline__ void exact_tile(const RowsProduct& g, int slice, int m0, int n0, floatx16 (&acc)[4][2]) {
+  int lane = threadIdx.x & (kWave - 1);
+  asm volatile("" : "+v"(lane));  // keeps this path's values out of the main loop's registers
+  const int half = lane >> 5, l32 = lane & 31;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  const long long n_blocks = (g.R + kBlockRows - 1) / kBlockRows;
+  for (long long blk = static_cast<long long>(slice) * kRpWaves + wave_id(); blk < n_blocks;
+       blk += static_cast<long long>(g.slices) * kRpWaves) {
+#pragma unroll 1
+    for (int i = 0; i < 8; ++i) {
+      const long long row = blk * kBlockRows + 8 * half + i;
+      const bool in = row < g.R;
+      const float* pa = g.a + min(row, g.R - 1) * g.lda;
+      const float* pb = g.b + min(row, g.R - 1) * g.ldb;
+      float va[4], vb[2];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) va[j] = in ? pa[clamp_col<1>(m0 + 4 * l32, j, g.M)] : 0.f;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) vb[j] = in ? pb[clamp_col<1>(n0 + 2 * l32, j, g.N)] : 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int k = 0; k < 2; ++k) acc[j][k] = mfma32(va[j], vb[k], acc[j][k]);
+    }
+  }
+}
+
 // VA, VB: columns of a and b loaded at once.
 template <int VA, int VB>
 __global__ __launch_bounds__(kRpThreads, 1) __attribute__((amdgpu_waves_per_eu(2, 2)))
@@ -169,6 +203,9 @@ void rows_product_kernel(RowsProduct g) {
     term(t0, t1);
     term(t0, t0);
   }
+
+  if (any_nonfinite(acc[0]) || any_nonfinite(acc[1]) || any_nonfinite(acc[2]) || any_nonfinite(acc[3]))
+    exact_tile(g, slice, m0, n0, acc);
 
   // The workgroup's tile.  Waves 4-7 hand theirs to waves 0-3 through LDS, then
   // all waves add those four, 16 elements per thread (three halving rounds

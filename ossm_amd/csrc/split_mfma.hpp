@@ -7,8 +7,13 @@
 // the 2^-24 of the product's own fp32 rounding.  v_mfma_f32_32x32x16_bf16 has 16 times the
 // fp32 MFMA's rate (32 cycles for 16 k against 64 for 2), so six of them are 2.7x
 // as fast as the fp32 instruction, and one accumulator rounding covers 16
-// products instead of 2.  An infinite operand gives NaN (inf - inf in the
-// split) where fp32 gives an infinity or NaN.
+// products instead of 2.
+//
+// Range: the 24 bits hold for |x| from about 2^-109 (1.5e-33) on; below it the lower
+// terms run into bf16's smallest values, 2^-133, whose halves are x's error.  An
+// infinite operand, or one past bf16's largest value (3.39e38), which rounds to
+// infinity, makes every sum it enters NaN (inf - inf in the split): a wave whose
+// sums are not all finite (any_nonfinite) forms them again in fp32.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -51,6 +56,25 @@ __device__ __forceinline__ SplitFrag split8(const float (&x)[8]) {
 
 __device__ __forceinline__ floatx16 mfma_bf16(bf16x8 a, bf16x8 b, floatx16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// Whether any sum that the wave holds is infinite or NaN (wave-uniform): their sum
+// then is too (as where it overflows).
+template <int N>
+__device__ __forceinline__ bool any_nonfinite(const floatx16 (&c)[N]) {
+  float s[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r & 3] += c[i][r];
+  s[0] = (s[0] + s[1]) + (s[2] + s[3]);
+  return __any(s[0] - s[0] != 0.f);
+}
+
+// c += a b over 2 k in fp32: lane l gives row (column) l % 32 at k = l / 32; the sums
+// lie as the bf16 instruction's do.
+__device__ __forceinline__ floatx16 mfma32(float a, float b, floatx16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
 
 // c += a b over 16 k, smallest terms first

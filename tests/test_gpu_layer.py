@@ -309,6 +309,45 @@ def test_layer_backward_recompute_path(layers, monkeypatch):
     no_device_errors()
 
 
+@pytest.mark.parametrize("shape", [(16, 513, 128, 128), (64, 2050, 20, 30)], ids=lambda s: "x".join(map(str, s)))
+def test_layer_split_infinities_and_largest_values(layers, shape):
+    """Split projections give fp32's infinities and NaN, and values where an operand
+    lies past bfloat16's largest; against the fp32 projections, which the first two
+    batch rows alone take."""
+    nb, L, H, P = shape
+    announce(f"layer split infinities {shape}")
+    args = [to_dev(x) for x in _layer_inputs(nb, L, H, P, 51, "imex1")]
+    u, B, C, D = args[:4]
+    go = torch.randn_like(u)
+    t = 40
+    B[0, :, 1], C[:, 0, 1] = 0.0, 0.0  # oscillator 0 is real: no inf - inf
+    B[0, :, 0], C[:, 0, 0] = B[0, :, 0].abs() + 0.1, C[:, 0, 0].abs() + 0.1
+    B[:, 3] *= 2.0 ** -40
+    C[3] *= 2.0 ** -40
+    D[3] = 2.0 ** -40
+    u[1, t, 3] = go[1, t, 3] = torch.finfo(torch.float32).max
+    u[0, t], go[0, t] = 3e38, 3e38  # oscillator 0's sums overflow, the others' do not
+    B[1:] *= 1e-3
+    C[:, 1:] *= 1e-3
+    D[:] = D.clamp(-1, 1)
+
+    def run(rows):
+        leaves = [u[:rows].clone().requires_grad_(), *args[1:]]
+        y = layers.DlinossLayerFn.apply("imex1", *leaves)
+        return y[:2], torch.autograd.grad(y, leaves[0], go[:rows])[0][:2]
+
+    for x, r in zip(run(nb), run(2)):
+        assert bool(torch.isinf(r[0, t]).all()) and bool(torch.isfinite(r[1]).all())
+        x, r = to_np(x), to_np(r)
+        finite = np.isfinite(r)
+        np.testing.assert_array_equal(x[~finite], r[~finite])
+        # each step's outputs to 1e-4 of that step's largest: it falls from 1e26 and more
+        scale = np.where(finite, np.abs(r), 0).max(-1, keepdims=True)
+        err = np.abs(np.where(finite, x, 0) - np.where(finite, r, 0))
+        assert (err <= 1e-4 * scale).all(), float((err / np.maximum(scale, 1e-30)).max())
+    no_device_errors()
+
+
 # at and above the sizes where the projections run as split bf16 products:
 # exact tiles, ragged H and P (weights zero-padded by the split), unaligned rows
 # (P or H not a multiple of 4), a short last chunk, grad_D in the kernel (padded H a

@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 def _bound(a, b):
     """|error| of a float32 product sum_r a b, split terms dropped at 2^-25 and
     summed in runs of 16: a few 2^-24 of sum |a b| covers both."""
-    return 4 * 2.0 ** -24 * (a.abs().double().t() @ b.abs().double()) + 1e-30
+    return 4 * 2.0 ** -24 * (a.abs().double().t() @ b.abs().double())
 
 
 # one block, a last block of one row, a ragged last block, tiles with one
@@ -62,6 +62,29 @@ def test_rows_product_wide_range_and_special_values():
     got = rows_product(a, b)
     bad = ~torch.isfinite(got)
     assert bool(bad[2].all()) and bool(bad[4].all()) and not bool(bad[[0, 1, 3, 5, 6, 7]].any())
+
+
+def test_rows_product_infinities_and_largest_values():
+    """Infinite and overflowing sums are infinities of float32's sign, and values past
+    bfloat16's largest, which rounds to infinity, are values (several row counts: a
+    wave's only block, its last one, one of many)."""
+    need_gpu()
+    from ossm_amd.linear import rows_product
+
+    for R in (16, 640, 70000):
+        announce(f"rows_product infinities R={R}")
+        a, b = torch.randn(R, 130, device="cuda"), torch.randn(R, 67, device="cuda")
+        a[R - 3, 4], b[7, 66] = float("inf"), -float("inf")
+        a[R // 2, 129] = torch.finfo(torch.float32).max
+        b[R // 2] *= 2.0 ** -20
+        a[9, 64], b[9, 3] = 1e30, 1e30
+        # the sum of (inf, -inf) and of NaN with anything are NaN both ways
+        got, want = rows_product(a, b), (a.double().t() @ b.double()).float()
+        assert torch.equal(torch.isfinite(got), torch.isfinite(want))
+        bad = ~torch.isfinite(want)
+        assert torch.equal(got[bad].nan_to_num(0.0), want[bad].nan_to_num(0.0))
+        bound = torch.where(bad, 0.0, _bound(a, b))
+        assert bool(((got.double() - want.double()).abs()[~bad] <= bound[~bad]).all())
 
 
 @pytest.mark.parametrize("bias", [True, False])
