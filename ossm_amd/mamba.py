@@ -355,7 +355,8 @@ class MambaMixer(nn.Module):
         params = (self.conv1d.weight, self.conv1d.bias, self.x_proj.weight, self.dt_proj.weight,
                   self.dt_proj.bias, self.A_log)
         if is_plain(self.x_proj) and self.x_proj.bias is None and xz.numel() > 0 and _all_float(xz, params):
-            return linear(self.out_proj, MixerCoreFn.apply(xz, *params))
+            y = MixerCoreFn.apply(xz, *params)
+            return linear(self.out_proj, y.to(self.out_proj.weight.dtype))
         x, z = _ColumnSplit.apply(xz, Di)                 # views, row stride 2 * d_inner
         x_conv = mamba_conv_silu(x, self.conv1d.weight.float(),
                                  None if self.conv1d.bias is None else self.conv1d.bias.float())

@@ -304,3 +304,34 @@ def test_mixer_core_matches_separate_functions(M, shape, monkeypatch):
         g, r = to_np(g), to_np(r)
         np.testing.assert_allclose(g, r, rtol=1e-4, atol=1e-5 * max(1.0, float(np.abs(r).max())))
     no_device_errors()
+
+
+def _both_ways(M, run, monkeypatch):
+    """run() through the mixer's fused middle and through the separate Functions."""
+    got = run()
+    with monkeypatch.context() as m:
+        m.setattr(M, "_all_float", lambda *a: False)
+        return got, run()
+
+
+def _mixer_grads(mixer, x, go):
+    y = mixer(x)
+    return [y, *torch.autograd.grad(y, [x, *mixer.parameters()], go)]
+
+
+def test_mixer_core_with_projections_in_bfloat16(M, monkeypatch):
+    """The usual mixed-precision layout: the outer projections in bfloat16, the state
+    space's parameters in float32."""
+    torch.manual_seed(3)
+    mixer = M.MambaMixer(16, d_state=4, d_conv=4, expand=2, dt_rank=3).cuda()
+    mixer.in_proj.bfloat16()
+    mixer.out_proj.bfloat16()
+    x = torch.randn(2, 50, 16, device="cuda", dtype=torch.bfloat16, requires_grad=True)
+    go = torch.randn(2, 50, 16, device="cuda", dtype=torch.bfloat16)
+    announce("mixer core, bfloat16 projections")
+    got, ref = _both_ways(M, lambda: _mixer_grads(mixer, x, go), monkeypatch)
+    for g, r in zip(got, ref):  # the same kernels; sums of float32 rounded to 8 bits
+        assert g.dtype == r.dtype
+        g, r = to_np(g.float()), to_np(r.float())
+        np.testing.assert_allclose(g, r, rtol=2e-2, atol=1e-2 * max(1.0, float(np.abs(r).max())))
+    no_device_errors()
