@@ -253,7 +253,7 @@ class MixerCoreFn(torch.autograd.Function):
                                                    u.data_ptr(), Bz, L, Di, w.size(1), st))
             proj = F.linear(u, xproj_w)
             dt = F.linear(proj[..., :R], dt_w)  # its bias goes into the softplus
-            A = -torch.exp(A_log)
+            A = -torch.exp(A_log.contiguous())
             y, raw = torch.empty_like(u), torch.empty_like(u)
             ck = torch.empty((Bz, Di, int(lib.ossm_selective_num_chunks(L)), 2 * N), dtype=torch.float32,
                              device=dev)

@@ -335,3 +335,19 @@ def test_mixer_core_with_projections_in_bfloat16(M, monkeypatch):
         g, r = to_np(g.float()), to_np(r.float())
         np.testing.assert_allclose(g, r, rtol=2e-2, atol=1e-2 * max(1.0, float(np.abs(r).max())))
     no_device_errors()
+
+
+def test_mixer_core_reads_strided_parameters(M, monkeypatch):
+    """Parameters that are views with other strides (here transposes)."""
+    torch.manual_seed(4)
+    mixer = M.MambaMixer(16, d_state=4, d_conv=4, expand=2, dt_rank=3).cuda()
+    for owner, name in ((mixer, "A_log"), (mixer.x_proj, "weight"), (mixer.dt_proj, "weight")):
+        p = getattr(owner, name).detach()
+        setattr(owner, name, torch.nn.Parameter((p + 0.1 * torch.randn_like(p)).t().contiguous().t()))
+    x = torch.randn(2, 50, 16, device="cuda", requires_grad=True)
+    announce("mixer core, strided parameters")
+    got, ref = _both_ways(M, lambda: _mixer_grads(mixer, x, torch.ones_like(x)), monkeypatch)
+    for g, r in zip(got, ref):
+        g, r = to_np(g), to_np(r)
+        np.testing.assert_allclose(g, r, rtol=1e-4, atol=1e-5 * max(1.0, float(np.abs(r).max())))
+    no_device_errors()
