@@ -202,6 +202,15 @@ def _all_float(xz: Tensor, params) -> bool:
                                   and t.device == xz.device) for t in (xz, *params)))
 
 
+def _core_shapes(Di: int, R: int, N: int, xz: Tensor, conv_w: Tensor, conv_b: Optional[Tensor],
+                 xproj_w: Tensor, dt_w: Tensor, dt_b: Optional[Tensor], A_log: Tensor) -> bool:
+    """Whether a mixer of d_inner ``Di``, dt_rank ``R`` and d_state ``N`` has these shapes."""
+    return (xz.dim() == 3 and xz.size(2) == 2 * Di
+            and conv_w.dim() > 1 and conv_w.size(0) == Di and conv_w.numel() == Di * conv_w.size(-1)
+            and (conv_b is None or conv_b.shape == (Di,)) and xproj_w.shape == (R + 2 * N, Di)
+            and dt_w.shape == (Di, R) and dt_b is not None and dt_b.shape == (Di,) and A_log.shape == (Di, N))
+
+
 class _ColumnSplit(torch.autograd.Function):
     """``xz[..., :d], xz[..., d:]`` as views, whose backward writes the gradient
     of ``xz`` in one pass (torch.cat of the two); slicing the tensor directly
@@ -240,6 +249,14 @@ class MixerCoreFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, xz: Tensor, conv_w: Tensor, conv_b: Optional[Tensor], xproj_w: Tensor,
                 dt_w: Tensor, dt_b: Tensor, A_log: Tensor) -> Tensor:  # type: ignore[override]
+        params = (conv_w, conv_b, xproj_w, dt_w, dt_b, A_log)
+        if dt_w.dim() != 2 or A_log.dim() != 2 or \
+                not _core_shapes(*dt_w.shape, A_log.size(1), xz, *params):
+            raise RuntimeError("mixer: inconsistent shapes xz, conv weight, conv bias, x_proj, dt_proj, dt bias, "
+                               f"A_log: {[t if t is None else tuple(t.shape) for t in (xz, *params)]}")
+        if not xz.is_cuda or any(t is not None and (t.dtype != torch.float32 or t.device != xz.device)
+                                 for t in (xz, *params)):
+            raise RuntimeError("mixer: every tensor must be a float32 GPU tensor, on one device")
         Di, R, N = dt_w.size(0), dt_w.size(1), A_log.size(1)
         lib = _lib.load()
         xz = xz.contiguous()
@@ -354,7 +371,9 @@ class MambaMixer(nn.Module):
         xz = linear(self.in_proj, inputs).float()
         params = (self.conv1d.weight, self.conv1d.bias, self.x_proj.weight, self.dt_proj.weight,
                   self.dt_proj.bias, self.A_log)
-        if is_plain(self.x_proj) and self.x_proj.bias is None and xz.numel() > 0 and _all_float(xz, params):
+        # other shapes (replaced parameters) take the separate steps, which refuse what does not fit
+        if is_plain(self.x_proj) and self.x_proj.bias is None and xz.numel() > 0 \
+                and _all_float(xz, params) and _core_shapes(Di, R, N, xz, *params):
             y = MixerCoreFn.apply(xz, *params)
             return linear(self.out_proj, y.to(self.out_proj.weight.dtype))
         x, z = _ColumnSplit.apply(xz, Di)                 # views, row stride 2 * d_inner

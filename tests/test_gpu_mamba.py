@@ -351,3 +351,40 @@ def test_mixer_core_reads_strided_parameters(M, monkeypatch):
         g, r = to_np(g), to_np(r)
         np.testing.assert_allclose(g, r, rtol=1e-4, atol=1e-5 * max(1.0, float(np.abs(r).max())))
     no_device_errors()
+
+
+def test_mixer_with_replaced_parameters(M):
+    """Parameters replaced by ones of other sizes are refused, as by the separate
+    steps, and ones that fit each other but for d_state too."""
+    torch.manual_seed(6)
+    x = torch.randn(2, 20, 16, device="cuda")
+    P = lambda *s: torch.nn.Parameter(0.1 * torch.randn(*s, device="cuda"))  # noqa: E731
+    announce("mixer, replaced parameters")
+    for owner, name, value in (("", "A_log", P(32, 5)), ("", "A_log", P(31, 4)), ("x_proj", "weight", P(13, 32)),
+                               ("dt_proj", "weight", P(33, 3)), ("dt_proj", "bias", P(31)),
+                               ("conv1d", "bias", P(30)), ("in_proj", "weight", P(66, 16))):
+        mixer = M.MambaMixer(16, d_state=4, d_conv=4, expand=2, dt_rank=3).cuda()
+        setattr(getattr(mixer, owner) if owner else mixer, name, value)
+        with pytest.raises(RuntimeError):
+            mixer(x)
+    mixer.in_proj.weight, mixer.A_log, mixer.x_proj.weight = P(64, 16), P(32, 5), P(13, 32)
+    with pytest.raises(RuntimeError, match="inconsistent shapes"):
+        mixer(x)
+    no_device_errors()
+
+
+# few rows: carried segments that write dz, dB and dC in place; d_inner and R + 2N
+# odd, several passes over the states
+@pytest.mark.parametrize("shape", [(1, 533, 16, 16, 2), (1, 600, 33, 17, 1)], ids=lambda s: "x".join(map(str, s)))
+def test_mixer_core_with_segment_carries(M, shape, monkeypatch):
+    nb, L, d_model, N, expand = shape
+    torch.manual_seed(L)
+    mixer = M.MambaMixer(d_model, d_state=N, d_conv=4, expand=expand, dt_rank=3).cuda()
+    x = torch.randn(nb, L, d_model, device="cuda", requires_grad=True)
+    go = torch.randn(nb, L, d_model, device="cuda")
+    announce(f"mixer core, segments {shape}")
+    got, ref = _both_ways(M, lambda: _mixer_grads(mixer, x, go), monkeypatch)
+    for g, r in zip(got, ref):
+        g, r = to_np(g), to_np(r)
+        np.testing.assert_allclose(g, r, rtol=1e-4, atol=1e-5 * max(1.0, float(np.abs(r).max())))
+    no_device_errors()

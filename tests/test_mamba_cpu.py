@@ -95,3 +95,24 @@ def test_mixer_entries_reject_what_the_kernels_cannot_read():
         mamba_conv_silu(x, torch.zeros(8, 1, 4))
     with pytest.raises(RuntimeError, match="float32 GPU tensor"):
         selective_scan_mamba(x, x, torch.zeros(8, 2), torch.zeros(1, 4, 2), torch.zeros(1, 4, 2))
+
+
+def _core_args(Di=6, R=2, N=4, L=5):
+    z = torch.zeros
+    return [z(2, L, 2 * Di), z(Di, 1, 3), z(Di), z(R + 2 * N, Di), z(Di, R), z(Di), z(Di, N)]
+
+
+@pytest.mark.parametrize("which, shape", [(0, (2, 5, 10)), (0, (10, 12)), (1, (5, 1, 3)), (1, (6, 2, 3)), (2, (5,)),
+                                          (3, (11, 6)), (3, (10, 5)), (4, (7, 2)), (4, (12,)), (5, (7,)), (6, (6, 5)),
+                                          (6, (7, 4)), (6, (24,))])
+def test_mixer_core_refuses_shapes_that_do_not_fit(which, shape):
+    """Before any pointer is taken: each tensor in turn of another size than the
+    others imply, then tensors that the kernels cannot read."""
+    from ossm_amd.mamba import MixerCoreFn
+
+    args = _core_args()
+    args[which] = torch.zeros(shape)
+    with pytest.raises(RuntimeError, match="inconsistent shapes"):
+        MixerCoreFn.apply(*args)
+    with pytest.raises(RuntimeError, match="float32 GPU tensor"):
+        MixerCoreFn.apply(*_core_args())
