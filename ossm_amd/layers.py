@@ -77,6 +77,12 @@ class LayerParamsFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, damped: bool, A_diag: Tensor, G_diag: Optional[Tensor],
                 steps: Tensor):  # type: ignore[override]
+        params = (A_diag, G_diag, steps) if damped else (A_diag, steps)
+        if any(t is None or t.dim() != 1 or t.shape != A_diag.shape for t in params):
+            raise RuntimeError("oscillator parameters must be vectors of one length, got "
+                               f"{[t if t is None else tuple(t.shape) for t in params]}")
+        if any(t.dtype != torch.float32 or not t.is_cuda or t.device != A_diag.device for t in params):
+            raise RuntimeError("oscillator parameters must be float32 GPU tensors, on one device")
         A, G, s = (None if t is None else t.contiguous() for t in (A_diag, G_diag, steps))
         out = torch.empty((6, A.numel()), dtype=torch.float32, device=A.device)
         _lib.run(_lib.load().ossm_layer_params_forward, A, int(damped), A.data_ptr(), _lib.ptr(G),
@@ -113,11 +119,14 @@ class LayerParamsFn(torch.autograd.Function):
 
 
 def fused_layer_supported(inputs: Tensor, params, hidden: int, ssm: int) -> bool:
-    """Whether a layer of this size runs as the fused kernel on ``inputs`` as it is:
-    float32 throughout on one GPU, no autocast, nothing empty."""
+    """Whether a LinOSS layer with ``params`` (A_diag, B, C, D, steps) runs as the fused
+    kernel on ``inputs`` as it is: float32 throughout on one GPU, no autocast, nothing
+    empty, nothing that broadcasts."""
     return (inputs.is_cuda and inputs.dtype == torch.float32 and inputs.numel() > 0
             and 0 < hidden <= _LAYER_MAX and 0 < ssm <= _LAYER_MAX
             and all(t.dtype == torch.float32 and t.device == inputs.device for t in params)
+            and all(t.shape == want for t, want in
+                    zip(params, ((ssm,), (ssm, hidden, 2), (hidden, ssm, 2), (hidden,), (ssm,))))
             and not torch.is_autocast_enabled("cuda"))
 
 
@@ -403,8 +412,11 @@ class DampedLinOSSLayer(nn.Module):
                   (self.A_diag, self.G_diag, self.steps, self.B, self.C, self.D)]
         Bw, Cw, Dw = params[3:]
         if u.is_cuda and self.hidden_dim <= _LAYER_MAX and self.ssm_size <= _LAYER_MAX:
-            a, g, dt, lo = LayerParamsFn.apply(True, *params[:3])
-            y = DlinossLayerFn.apply(self.variant, u, Bw, Cw, Dw, a, g, dt, lo)
+            if all(t.shape == (self.ssm_size,) for t in params[:3]):
+                a, g, dt, _ = LayerParamsFn.apply(True, *params[:3])
+            else:  # replaced parameters may broadcast
+                a, g, dt = project_parameters(*params[:3])
+            y = DlinossLayerFn.apply(self.variant, u, Bw, Cw, Dw, a, g, dt)
         else:
             a, g, dt = project_parameters(*params[:3])
             y = unfused_layer_forward(self.variant, u, Bw, Cw, Dw, a, g, dt)

@@ -101,3 +101,33 @@ def test_linoss_layer_fused_matches_composition(disc, shape, monkeypatch):
     for x, r in zip(got, ref):
         x, r = x.detach().cpu().numpy(), r.detach().cpu().numpy()
         np.testing.assert_allclose(x, r, rtol=1e-4, atol=1e-4 * max(1.0, float(np.abs(r).max())))
+
+
+@pytest.mark.parametrize("disc", ["IM", "IMEX"])
+def test_layers_with_parameters_that_broadcast(disc):
+    """Replaced parameters of one element are shared by all oscillators (channels), as
+    by the torch operations; other sizes are refused."""
+    need_gpu()
+    from ossm_amd import layers, linoss
+
+    announce(f"layers, broadcast parameters {disc}")
+    torch.manual_seed(3)
+    P = lambda v: torch.nn.Parameter(v.detach().clone())  # noqa: E731
+    u = torch.randn(2, 40, 6, device="cuda")
+    for make, shared in ((lambda: layers.DampedLinOSSLayer(7, 6), ("A_diag",)),
+                         (lambda: linoss.LinOSSLayer(7, 6, disc), ("D", "steps") if disc == "IM" else ("D",))):
+        torch.manual_seed(4)
+        layer = make().cuda()
+        for name in shared:
+            p = getattr(layer, name)
+            setattr(layer, name, P(p[:1].expand_as(p)))
+        want = torch.autograd.grad(layer(u).square().sum(), [getattr(layer, n) for n in shared])
+        for name in shared:
+            setattr(layer, name, P(getattr(layer, name)[:1]))
+        got = torch.autograd.grad(layer(u).square().sum(), [getattr(layer, n) for n in shared])
+        for g, w in zip(got, want):
+            np.testing.assert_allclose(g.cpu().numpy(), w.sum(0, keepdim=True).cpu().numpy(), rtol=1e-4, atol=1e-4)
+        layer = make().cuda()
+        layer.steps = torch.nn.Parameter(torch.zeros(9, device="cuda"))
+        with pytest.raises(RuntimeError):
+            layer(u)

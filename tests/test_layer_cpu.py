@@ -174,3 +174,19 @@ def test_weight_gradient_row_sum_split(rows):
     got = _sum_rows_product(a, b)
     assert got.shape == (12, 7)
     assert torch.allclose(got, a.t() @ b, rtol=1e-12, atol=1e-12)
+
+
+@pytest.mark.parametrize("damped", [True, False])
+def test_layer_params_refuse_sizes_that_do_not_fit(damped):
+    """Before any pointer is taken: parameters of other lengths or not vectors, then
+    host tensors."""
+    from ossm_amd.layers import LayerParamsFn
+
+    z = torch.zeros
+    G = z(5) if damped else None
+    for A, g, s in ((z(5), G, z(1)), (z(5), G, z(4)), (z(1), G, z(5)), (z(5, 1), G, z(5)), (z(()), G, z(())),
+                    *([(z(5), z(6), z(5)), (z(5), None, z(5))] if damped else [])):
+        with pytest.raises(RuntimeError, match="vectors of one length"):
+            LayerParamsFn.apply(damped, A, g, s)
+    with pytest.raises(RuntimeError, match="float32 GPU tensors"):
+        LayerParamsFn.apply(damped, z(5), G, z(5))
