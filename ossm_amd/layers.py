@@ -118,12 +118,18 @@ class LayerParamsFn(torch.autograd.Function):
         return (None, *[out[i] if n else None for i, n in enumerate(ctx.needs_input_grad[1:])])
 
 
+def _layer_sizes_fit(batch: int, length: int, hidden: int, ssm: int) -> bool:
+    """The fused layer kernels' size limits (those ossm_dlinoss_layer_* refuse above)."""
+    return (hidden <= _LAYER_MAX and ssm <= _LAYER_MAX and batch * ssm <= (2 ** 31 - 1) // 8
+            and batch * -(-length // _CHUNK) < 2 ** 31)
+
+
 def fused_layer_supported(inputs: Tensor, params, hidden: int, ssm: int) -> bool:
     """Whether a LinOSS layer with ``params`` (A_diag, B, C, D, steps) runs as the fused
     kernel on ``inputs`` as it is: float32 throughout on one GPU, no autocast, nothing
     empty, nothing that broadcasts."""
-    return (inputs.is_cuda and inputs.dtype == torch.float32 and inputs.numel() > 0
-            and 0 < hidden <= _LAYER_MAX and 0 < ssm <= _LAYER_MAX
+    return (inputs.is_cuda and inputs.dtype == torch.float32 and inputs.numel() > 0 and ssm > 0
+            and _layer_sizes_fit(inputs.size(0), inputs.size(1), hidden, ssm)
             and all(t.dtype == torch.float32 and t.device == inputs.device for t in params)
             and all(t.shape == want for t, want in
                     zip(params, ((ssm,), (ssm, hidden, 2), (hidden, ssm, 2), (hidden,), (ssm,))))

@@ -190,3 +190,23 @@ def test_layer_params_refuse_sizes_that_do_not_fit(damped):
             LayerParamsFn.apply(damped, A, g, s)
     with pytest.raises(RuntimeError, match="float32 GPU tensors"):
         LayerParamsFn.apply(damped, z(5), G, z(5))
+
+
+def test_layer_size_limits_are_the_librarys():
+    """What ``_layer_sizes_fit`` lets through the library takes, and what it does not
+    the library refuses, each side of every line (host checks: null pointers)."""
+    from ossm_amd import _lib, layers
+
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("libossm_scan.so not built (python -m ossm_amd.build)")
+    lib, m = _lib.load(), 2 ** 31 - 1
+    for batch, length, hidden, ssm in ((m // 8, 1, 1, 1), (m // 8 + 1, 1, 1, 1), (m // 64, 9, 5, 8), (m // 64 + 1, 9, 5, 8),
+                                       (1, m, 1, 1), (2 ** 10, 2 ** 26 - 32, 3, 2), (2 ** 10, 2 ** 26, 3, 2),
+                                       (1, 1, 256, 256), (1, 1, 257, 1), (1, 1, 1, 257)):
+        sizes = (batch, length, hidden, ssm)
+        rcs = {lib.ossm_dlinoss_layer_forward_wide(0, *[None] * 10, *sizes, None),
+               lib.ossm_dlinoss_layer_backward_wide(0, *[None] * 17, *sizes, None)}
+        if ssm > 0 and layers._layer_sizes_fit(*sizes):
+            assert 3 not in rcs, sizes  # a null pointer is what is wrong
+        else:
+            assert 3 in rcs, sizes
