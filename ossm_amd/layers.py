@@ -284,13 +284,16 @@ def unfused_layer_forward(variant: str, inputs: Tensor, B: Tensor, C: Tensor, D:
 
 class DlinossLayerFn(torch.autograd.Function):
     """Fused forward and backward (``dlinoss_layer_backward``); shapes whose
-    backward does not fit recompute through ``unfused_layer_forward``."""
+    backward does not fit, and backwards that are differentiated again, go
+    through ``unfused(variant, inputs, B, C, D, a_diag, g_diag, step)``, the same
+    layer as separate differentiable steps."""
 
     @staticmethod
     def forward(ctx, variant: str, inputs: Tensor, B: Tensor, C: Tensor, D: Tensor,
-                a_diag: Tensor, g_diag: Tensor, step: Tensor,
-                lo: Optional[Tensor] = None) -> Tensor:  # type: ignore[override]
+                a_diag: Tensor, g_diag: Tensor, step: Tensor, lo: Optional[Tensor] = None,
+                unfused=unfused_layer_forward) -> Tensor:  # type: ignore[override]
         ctx.variant = variant
+        ctx.unfused = unfused
         batch, length, hidden = inputs.shape
         ssm = B.size(0)
         carries = None
@@ -305,17 +308,18 @@ class DlinossLayerFn(torch.autograd.Function):
     def backward(ctx, grad_out: Tensor):  # type: ignore[override]
         *saved, carries, lo = ctx.saved_tensors
         needs = ctx.needs_input_grad[1:8]
-        tail = (None,) * (len(ctx.needs_input_grad) - 8)  # lo, where it was passed
-        if ctx.fused_bwd:
+        tail = (None,) * (len(ctx.needs_input_grad) - 8)  # lo and unfused, where they were passed
+        again = torch.is_grad_enabled()  # create_graph
+        if ctx.fused_bwd and not again:
             grads = dlinoss_layer_backward(ctx.variant, *saved[:1], grad_out, *saved[1:], carries, lo)
             return (None, *[gr if n else None for gr, n in zip(grads, needs)], *tail)
         with torch.enable_grad():
-            leaves = [t.detach().requires_grad_(bool(n)) for t, n in zip(saved, needs)]
-            y = unfused_layer_forward(ctx.variant, *leaves)
-            wanted = [t for t in leaves if t.requires_grad]
-            got = iter(torch.autograd.grad(y, wanted, grad_out)) if wanted else iter(())
-        grads = [next(got) if t.requires_grad else None for t in leaves]
-        return (None, *grads, *tail)
+            args = saved if again else [t.detach().requires_grad_(bool(n)) for t, n in zip(saved, needs)]
+            wanted = [t for t, n in zip(args, needs) if n]
+            y = ctx.unfused(ctx.variant, *args)
+            got = iter(torch.autograd.grad(y, wanted, grad_out, create_graph=again, allow_unused=True)
+                       if wanted else ())
+        return (None, *[next(got) if n else None for n in needs], *tail)
 
 
 class DampedLinOSSLayer(nn.Module):

@@ -49,6 +49,36 @@ def linoss_transition(a_diag: Tensor, step: Tensor, discretization: str):
     return m11, -step * a_diag, step, 1.0 - dt2a, step, step * step
 
 
+def _unfused(discretization: str, ssm: int, inputs: Tensor, B: Tensor, C: Tensor, D: Tensor,
+             a_diag: Tensor, step: Tensor) -> Tensor:
+    """The layer as separate steps, from its projected parameters."""
+    batch, length, hidden = inputs.shape
+    flat = inputs.reshape(batch * length, hidden)
+    # bu = u B^T as two real GEMMs, as the reference forms it (linoss.py:222-227)
+    bu = torch.complex(flat @ B[..., 0].t(), flat @ B[..., 1].t())
+    bu = bu.reshape(batch, length, ssm)
+    if length == 0:
+        x = bu.new_zeros(batch, 0, ssm)
+    else:
+        cd = bu.dtype
+        m11, m12, m21, m22, f1, f2 = linoss_transition(a_diag, step, discretization)
+        a_matrix = torch.stack((torch.stack((m11, m12), -1), torch.stack((m21, m22), -1)), -2).to(cd)
+        bu_seq = bu.permute(1, 0, 2)  # [L, B, P]
+        b_seq = torch.stack((bu_seq * f1.to(cd), bu_seq * f2.to(cd)), -1).contiguous()
+        states = run_associative_scan(a_matrix, b_seq)  # [L, B, P, 2]
+        x = states[..., 1].permute(1, 0, 2)  # [B, L, P]
+    x = x.reshape(batch * length, ssm)
+    y = x.real @ C[..., 0].t() - x.imag @ C[..., 1].t()
+    return y.reshape(batch, length, hidden) + inputs * D
+
+
+# the D-LinOSS recurrence that a discretisation is with g = 0, and the layer of it as
+# DlinossLayerFn differentiates it where its kernels do not
+_VARIANTS = {"IM": "im", "IMEX": "imex2"}
+_UNFUSED = {v: (lambda _, u, B, C, D, a, g, dt, d=d: _unfused(d, B.size(0), u, B, C, D, a, dt))
+            for d, v in _VARIANTS.items()}
+
+
 class LinOSSLayer(nn.Module):
     """Single LinOSS state-space layer (reference LinOSSLayer, linoss.py:172-315)."""
 
@@ -79,7 +109,7 @@ class LinOSSLayer(nn.Module):
     def forward(self, inputs: Tensor) -> Tensor:
         if inputs.dim() != 3:
             raise ValueError("LinOSSLayer expects input of shape (batch, length, hidden_dim).")
-        batch, length, hidden = inputs.shape
+        hidden = inputs.size(-1)
         if hidden != self.hidden_dim:
             raise ValueError(f"Expected hidden_dim={self.hidden_dim}, received {hidden}.")
         dtype, device = inputs.dtype, inputs.device
@@ -88,25 +118,7 @@ class LinOSSLayer(nn.Module):
                                  self.ssm_size):
             # IM and IMEX are the undamped (g = 0) D-LinOSS im and imex2 recurrences
             a, g, dt, lo = LayerParamsFn.apply(False, self.A_diag, None, self.steps)
-            return DlinossLayerFn.apply("im" if self.discretization == "IM" else "imex2", inputs,
-                                        self.B, self.C, self.D, a, g, dt, lo)
-        a_diag = cast(torch.relu(self.A_diag))
-        step = cast(torch.sigmoid(self.steps))
-        flat = inputs.reshape(batch * length, hidden)
-        # bu = u B^T as two real GEMMs, as the reference forms it (linoss.py:222-227)
-        bu = torch.complex(flat @ cast(self.B[..., 0]).t(), flat @ cast(self.B[..., 1]).t())
-        bu = bu.reshape(batch, length, self.ssm_size)
-        if length == 0:
-            x = bu.new_zeros(batch, 0, self.ssm_size)
-        else:
-            cd = bu.dtype
-            m11, m12, m21, m22, f1, f2 = linoss_transition(a_diag, step, self.discretization)
-            a_matrix = torch.stack((torch.stack((m11, m12), -1), torch.stack((m21, m22), -1)),
-                                   -2).to(cd)
-            bu_seq = bu.permute(1, 0, 2)  # [L, B, P]
-            b_seq = torch.stack((bu_seq * f1.to(cd), bu_seq * f2.to(cd)), -1).contiguous()
-            states = run_associative_scan(a_matrix, b_seq)  # [L, B, P, 2]
-            x = states[..., 1].permute(1, 0, 2)  # [B, L, P]
-        x = x.reshape(batch * length, self.ssm_size)
-        y = x.real @ cast(self.C[..., 0]).t() - x.imag @ cast(self.C[..., 1]).t()
-        return y.reshape(batch, length, hidden) + inputs * cast(self.D)
+            variant = _VARIANTS[self.discretization]
+            return DlinossLayerFn.apply(variant, inputs, self.B, self.C, self.D, a, g, dt, lo, _UNFUSED[variant])
+        return _unfused(self.discretization, self.ssm_size, inputs, cast(self.B), cast(self.C), cast(self.D),
+                        cast(torch.relu(self.A_diag)), cast(torch.sigmoid(self.steps)))

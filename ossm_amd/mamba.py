@@ -236,6 +236,17 @@ class _ColumnSplit(torch.autograd.Function):
         return torch.cat([gx, gz], dim=-1), None
 
 
+def _mixer_core(xz: Tensor, conv_w: Tensor, conv_b: Optional[Tensor], xproj_w: Tensor, dt_w: Tensor,
+                dt_b: Tensor, A_log: Tensor) -> Tensor:
+    """``MixerCoreFn`` as separate steps."""
+    R, N = dt_w.size(1), A_log.size(1)
+    x, z = _ColumnSplit.apply(xz, dt_w.size(0))
+    u = mamba_conv_silu(x, conv_w, conv_b)
+    proj = linear_weight(u, xproj_w)
+    dt = linear_weight(proj[..., :R], dt_w)
+    return selective_scan_mamba(u, dt, -torch.exp(A_log), proj[..., R:R + N], proj[..., R + N:], gate=z, dt_bias=dt_b)
+
+
 class MixerCoreFn(torch.autograd.Function):
     """The mixer between its in and out projections, ``xz`` [B, L, 2 Di] to
     ``y`` [B, L, Di]: conv + SiLU, x_proj, dt_proj, the gated scan.  Its backward
@@ -259,7 +270,7 @@ class MixerCoreFn(torch.autograd.Function):
             raise RuntimeError("mixer: every tensor must be a float32 GPU tensor, on one device")
         Di, R, N = dt_w.size(0), dt_w.size(1), A_log.size(1)
         lib = _lib.load()
-        xz = xz.contiguous()
+        given, xz = xz, xz.contiguous()
         Bz, L, ld = xz.shape
         w = conv_w.reshape(Di, -1).contiguous()
         dev, st = xz.device, _lib.stream_of(xz)
@@ -278,12 +289,20 @@ class MixerCoreFn(torch.autograd.Function):
             _lib.check(lib.ossm_selective_mamba_forward(
                 u.data_ptr(), Di, dt.data_ptr(), Di, dtb.data_ptr(), A.data_ptr(), pp, pp + 4 * N,
                 R + 2 * N, z, ld, y.data_ptr(), raw.data_ptr(), ck.data_ptr(), Bz, Di, L, N, st))
-        ctx.save_for_backward(xz, u, proj, dt, A, ck, raw, conv_w, conv_b, xproj_w, dt_w, dt_b)
+        ctx.save_for_backward(given, u, proj, dt, A, ck, raw, conv_w, conv_b, xproj_w, dt_w, dt_b,
+                              A_log)
         return y
 
     @staticmethod
     def backward(ctx, gy: Tensor):  # type: ignore[override]
-        xz, u, proj, dt, A, ck, raw, conv_w, conv_b, xproj_w, dt_w, dt_b = ctx.saved_tensors
+        xz, u, proj, dt, A, ck, raw, conv_w, conv_b, xproj_w, dt_w, dt_b, A_log = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            # create_graph: differentiable again, as separate steps
+            inputs = (xz, conv_w, conv_b, xproj_w, dt_w, dt_b, A_log)
+            wanted = [t for t, n in zip(inputs, ctx.needs_input_grad) if n]
+            got = iter(torch.autograd.grad(_mixer_core(*inputs), wanted, gy, create_graph=True, allow_unused=True))
+            return tuple(next(got) if n else None for n in ctx.needs_input_grad)
+        xz = xz.contiguous()
         Di, R, N = dt_w.size(0), dt_w.size(1), A.size(1)
         Bz, L, ld = xz.shape
         rows, ldp = Bz * L, R + 2 * N

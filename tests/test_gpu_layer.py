@@ -348,6 +348,28 @@ def test_layer_split_infinities_and_largest_values(layers, shape):
     no_device_errors()
 
 
+@pytest.mark.parametrize("variant", VARIANTS)
+def test_layer_second_derivatives(layers, variant):
+    """create_graph: the gradients carry the graph that the unfused layer's do."""
+    announce(f"layer create_graph {variant}")
+    args = _layer_inputs(2, 40, 12, 9, 57, variant)
+    go = to_dev(np.random.default_rng(58).normal(size=args[0].shape).astype(np.float32))
+
+    def second(fn):
+        leaves = [to_dev(x).requires_grad_() for x in args]
+        first = torch.autograd.grad(fn(variant, *leaves), leaves, go, create_graph=True)
+        assert all(g.requires_grad for g in first[:4])  # of u, B, C, D
+        return torch.autograd.grad(sum(g.square().sum() for g in first if g.requires_grad), leaves,
+                                   allow_unused=True)
+
+    got, want = second(layers.DlinossLayerFn.apply), second(layers.unfused_layer_forward)
+    for x, r, name in zip(got, want, ("u", "B", "C", "D", "a", "g", "step")):
+        assert (x is None) == (r is None), name
+        if r is not None:
+            np.testing.assert_allclose(to_np(x), to_np(r), rtol=1e-3, atol=1e-4 * max(1.0, float(r.abs().max())),
+                                       err_msg=name)
+
+
 # at and above the sizes where the projections run as split bf16 products:
 # exact tiles, ragged H and P (weights zero-padded by the split), unaligned rows
 # (P or H not a multiple of 4), a short last chunk, grad_D in the kernel (padded H a

@@ -116,3 +116,29 @@ def test_linoss_matrix_scan_fn_complex_matrix(linoss):
     np.testing.assert_allclose(tb.grad.cpu().numpy(), rb.grad.numpy(), rtol=1e-4, atol=1e-4)
     one = torch.tensor(b[:1], dtype=torch.complex64, device="cuda")
     assert torch.equal(bridge.run_associative_scan(tM.detach(), one), one)
+
+
+@pytest.mark.parametrize("disc", ["IM", "IMEX"])
+def test_linoss_layer_second_derivatives(linoss, disc, monkeypatch):
+    """create_graph through the fused layer gives the composition's second
+    derivatives (those through the products and the parameter maps; the scan's own
+    backward has no graph in either)."""
+    torch.manual_seed(7)
+    layer = linoss.LinOSSLayer(9, 12, disc).cuda()
+    u = torch.randn(2, 40, 12, device="cuda", requires_grad=True)
+    go = torch.randn(2, 40, 12, device="cuda")
+    announce(f"linoss layer create_graph {disc}")
+
+    def second():
+        wrt = [u, *layer.parameters()]
+        first = torch.autograd.grad(layer(u), wrt, go, create_graph=True)
+        return torch.autograd.grad(sum(g.square().sum() for g in first if g.requires_grad), wrt,
+                                   allow_unused=True)
+
+    got = second()
+    monkeypatch.setattr(linoss, "fused_layer_supported", lambda *a: False)
+    for x, r in zip(got, second()):
+        assert (x is None) == (r is None)
+        if r is not None:
+            np.testing.assert_allclose(x.cpu().numpy(), r.cpu().numpy(), rtol=1e-3,
+                                       atol=1e-4 * max(1.0, float(r.abs().max())))

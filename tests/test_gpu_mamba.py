@@ -353,6 +353,29 @@ def test_mixer_core_reads_strided_parameters(M, monkeypatch):
     no_device_errors()
 
 
+def test_mixer_core_second_derivatives(M, monkeypatch):
+    """create_graph: what the separate Functions' gradients carry (the terms through
+    the projections and A_log; conv and scan have no graph of their own)."""
+    torch.manual_seed(5)
+    mixer = M.MambaMixer(8, d_state=4, d_conv=4, expand=2, dt_rank=3).cuda()
+    x = torch.randn(2, 300, 8, device="cuda", requires_grad=True)
+    go = torch.randn(2, 300, 8, device="cuda")
+    announce("mixer core create_graph")
+
+    def second():
+        wrt = [x, *mixer.parameters()]
+        first = torch.autograd.grad(mixer(x), wrt, go, create_graph=True)
+        return torch.autograd.grad(sum(g.square().sum() for g in first if g.requires_grad), wrt,
+                                   allow_unused=True)
+
+    got, ref = _both_ways(M, second, monkeypatch)
+    for g, r in zip(got, ref):
+        assert (g is None) == (r is None)
+        if r is not None:
+            g, r = to_np(g), to_np(r)
+            np.testing.assert_allclose(g, r, rtol=1e-3, atol=1e-4 * max(1.0, float(np.abs(r).max())))
+
+
 def test_mixer_with_replaced_parameters(M):
     """Parameters replaced by ones of other sizes are refused, as by the separate
     steps, and ones that fit each other but for d_state too."""
