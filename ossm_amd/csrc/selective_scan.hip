@@ -480,6 +480,17 @@ __device__ __forceinline__ void store_states(float* __restrict__ s, const StateR
   }
 }
 
+// First tile of time segment `seg` of n_seg (the last's end at seg = n_seg).  Unsigned:
+// 32 segments of the longest rows' 2^26 tiles are past an int.
+constexpr __host__ __device__ int segment_tile(int seg, int n_tiles, int n_seg) {
+  return static_cast<int>(static_cast<unsigned>(seg) * static_cast<unsigned>(n_tiles) / static_cast<unsigned>(n_seg));
+}
+constexpr int kMaxSegments = 32;
+constexpr int kMaxTiles = (INT_MAX / 2 + 15) / 16;  // of 16 steps, at the largest length (check_selective)
+static_assert(segment_tile(kMaxSegments, kMaxTiles, kMaxSegments) == kMaxTiles &&
+              segment_tile(kMaxSegments - 1, kMaxTiles, kMaxSegments) == kMaxTiles / kMaxSegments * (kMaxSegments - 1) &&
+              segment_tile(1, 10, 3) == 3 && segment_tile(2, 10, 3) == 6);
+
 // ---- forward ------------------------------------------------------------------
 // Time segments whose carries go through memory (see segment_plan).  mode 0: a
 // segment re-runs the recurrence over the segments it depends on; 1: it only runs
@@ -850,8 +861,8 @@ __global__ __launch_bounds__(kThreads) void selective_fwd_kernel(FwdArgs<E> a) {
   // folded ends of the earlier segments (SegCarry).
   const int n_tiles = (a.L + TT - 1) / TT;
   const int n_seg = static_cast<int>(gridDim.z), seg = static_cast<int>(blockIdx.z);
-  const int t_lo = (seg * n_tiles / n_seg) * TT;
-  const int t_hi = min(a.L, ((seg + 1) * n_tiles / n_seg) * TT);
+  const int t_lo = segment_tile(seg, n_tiles, n_seg) * TT;
+  const int t_hi = min(a.L, segment_tile(seg + 1, n_tiles, n_seg) * TT);
 
   FwdTile<ROWS> nxt;
   float zn[SEG];  // the gate of the lane's output segment, one tile ahead
@@ -1235,8 +1246,8 @@ __global__ __launch_bounds__(kThreads) void selective_bwd_kernel(BwdArgs<E> a) {
   // per-step arithmetic (so the carry is bitwise the one the later segments
   // reach).
   const int n_seg = static_cast<int>(gridDim.z), seg = static_cast<int>(blockIdx.z);
-  const int tile_lo = seg * n_tiles / n_seg;
-  const int tile_hi = (seg + 1) * n_tiles / n_seg;
+  const int tile_lo = segment_tile(seg, n_tiles, n_seg);
+  const int tile_hi = segment_tile(seg + 1, n_tiles, n_seg);
   // the tiles the adjoint alone runs over: those after the segment, or (mode 1) its own
   const bool ends = CARRY && a.carry.mode == 1;
   int r_hi = CARRY ? tile_hi : n_tiles;
@@ -1927,8 +1938,8 @@ void selective_bwd2_kernel(BwdArgs<E> a) {
   // time split as in selective_bwd_kernel: segment s runs tiles
   // [s n / S, (s + 1) n / S) after an adjoint-only pass over the later tiles
   const int n_seg = static_cast<int>(gridDim.z), seg = static_cast<int>(blockIdx.z);
-  const int tile_lo = seg * n_tiles / n_seg;
-  const int tile_hi = (seg + 1) * n_tiles / n_seg;
+  const int tile_lo = segment_tile(seg, n_tiles, n_seg);
+  const int tile_hi = segment_tile(seg + 1, n_tiles, n_seg);
   if (tile_hi < n_tiles) {
     AdjTile2 p;
     adj2_prefetch<E, VEC, GATED>(p, a, g, roff, cs, n_tiles - 1);
@@ -2417,7 +2428,8 @@ int segment_plan(int64_t rows64, int64_t L, bool backward, int least, int n_cu) 
     if (std::getenv(name) != nullptr) return 0;
   const int64_t per = n_cu / std::max<int64_t>(rows64, 1), per2 = 2 * n_cu / std::max<int64_t>(rows64, 1);
   const int64_t s = std::min<int64_t>(
-      backward ? std::min(per2, (L + 63) / 64) : std::max(std::min(per, (L + 63) / 64), std::min(per2, L / 128)), 32);
+      backward ? std::min(per2, (L + 63) / 64) : std::max(std::min(per, (L + 63) / 64), std::min(per2, L / 128)),
+      kMaxSegments);
   return s >= least ? static_cast<int>(s) : 0;
 }
 
