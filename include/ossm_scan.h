@@ -59,7 +59,7 @@ enum {
 enum { OSSM_DLINOSS_IMEX1 = 0, OSSM_DLINOSS_IMEX2 = 1, OSSM_DLINOSS_IM = 2, OSSM_DLINOSS_EX = 3 };
 
 /* Library ABI version (bumped on any change of the entry points or their
-   behaviour; currently 16). */
+   behaviour; currently 17). */
 int ossm_abi_version(void);
 
 /* Message of the last failing call on this host thread ("" if none). */

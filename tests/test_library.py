@@ -59,7 +59,7 @@ def test_library_exports_every_declared_symbol():
     assert not missing, missing
     # every declared symbol has a ctypes signature in the binding
     assert set(_declared_functions()) == set(_lib.EXPORTED)
-    assert _lib.load().ossm_abi_version() == 16
+    assert _lib.load().ossm_abi_version() == 17
 
 
 def test_selective_skip_entry_points_refuse_a_null_d():
