@@ -513,13 +513,20 @@ __device__ __forceinline__ float fold_segment(float h, float sdt, float A2, floa
   return fmaf(f * h, f, end);
 }
 
-// Whether any state of the workgroup is infinite or NaN.  Every thread calls it.
+// Whether any state of the workgroup is infinite or NaN.  Every thread calls it, once.
 template <int NPW>
 __device__ __forceinline__ bool left_range(const float (&h)[NPW]) {
+  __shared__ int s_left[kMaxWaves];  // a word per wave and one barrier (__syncthreads_or: 0.5 us more)
   float s = 0.f;
 #pragma unroll
   for (int q = 0; q < NPW; ++q) s += h[q] - h[q];
-  return __syncthreads_or(s != 0.f);
+  const bool any = __any(s != 0.f);
+  if ((threadIdx.x & (kWave - 1)) == 0) s_left[threadIdx.x / kWave] = any;
+  __syncthreads();
+  int left = 0;
+#pragma unroll
+  for (int w = 0; w < kMaxWaves; ++w) left |= s_left[w];
+  return left != 0;
 }
 
 // The carry of one row's states [n0, n0 + NPW) past segments first, first + step, ..
@@ -1185,8 +1192,11 @@ __device__ __forceinline__ void adj_prefetch(AdjTile& f, const BwdArgs<E>& a, si
   load_states<kBwdTile>(f.C, a.Cm, bc0, a.ld_bc, t0, a.L, a.N, a.n_base);
 }
 
+// SKIP and CARRY together want 259 registers: held to 256, two waves per SIMD (2
+// spilled; bf16 [16, 512, 2048], N = 16, 463 -> 321 us).
 template <class E, bool VEC, bool GATED, bool BLD, bool SKIP, bool CARRY>
-__global__ __launch_bounds__(kThreads) void selective_bwd_kernel(BwdArgs<E> a) {
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SKIP && CARRY ? 2 : 1)))
+void selective_bwd_kernel(BwdArgs<E> a) {
   static_assert(!BLD || std::is_same_v<E, float>, "the [B, L, D] layout is fp32");
   static_assert(!(BLD && SKIP), "the skip D is for the [B, D, L] layout");
   constexpr int TT = kBwdTile;
@@ -2413,13 +2423,21 @@ bool cols_vectorizable(int64_t D, const MambaLayout& ml, std::initializer_list<c
 // `least` segments and below 512 steps, where the second launch and the fold eat what
 // the split saves.  The variables that force another path turn it off.
 // fp32, N = 16, gated, forward / backward, us, re-run -> carried:
-//   B, D = 1, 922:  L = 256  16 -> 18 / 28 -> 28,  512  29 -> 21 / 48 -> 38,
-//                   2048  107 -> 37 / 161 -> 69,  8192  415 -> 91 / 611 -> 159
-//   B, D = 27, 80:  L = 256  18 -> 20 / 32 -> 34,  1024  62 -> 48 / 97 -> 79,
-//                   8192  456 -> 234 / 717 -> 495
+//   B, D = 1, 922:  L = 256  16 -> 18 / 28 -> 28,  512  29 -> 21 / 48 -> 39,
+//                   2048  107 -> 38 / 161 -> 68,  8192  415 -> 92 / 611 -> 160
+//   B, D = 27, 80:  L = 256  18 -> 20 / 32 -> 34,  600  38 -> 37 / 61 -> 59,
+//                   2048  117 -> 71 / 183 -> 132
 //   B, D = 12, 512 (5 segments, hence the forward's least):  700  53 -> 56 / 92 -> 94,
 //                   2048  139 -> 120 / 234 -> 248
-//   B, D = 16, 512 (4): 512  38 -> 48 / 91 -> 88,  2048  137 -> 146 / 354 -> 305
+//   B, D = 16, 512 (4): 512  38 -> 48 / 91 -> 88,  2048  137 -> 146 / 328 -> 293
+// Backward against the 2-states kernel, fp32 / bf16 with skip, where it does and does
+// not pay (N = 4 and 12 leave waves idle as 8 and 24 do):
+//   B, D, L = 8, 512, 600 (8)    N = 8  56 -> 57 / 66 -> 60,  16  60 -> 63 / 69 -> 68
+//             10, 512, 600 (6)   N = 8  62 -> 67 / 68 -> 74,  16  73 -> 73 / 79 -> 79
+//             10, 512, 2048 (6)  N = 8  188 -> 189 / 205 -> 191,  16  223 -> 201 / 238 -> 206
+//             16, 512, 2048 (4)  N = 8  247 -> 277 / 265 -> 302,  16  328 -> 293 / 335 -> 325,
+//                                24  666 -> 622 / 646 -> 666
+//             20, 512, 2048 (3)  N = 16  389 -> 379 / 408 -> 418
 // The outputs' error against float64 is the re-run segments' or smaller (decay over
 // 2000 steps: 5e-7 here, 4e-6 there, one product of the steps' transitions).
 int segment_plan(int64_t rows64, int64_t L, bool backward, int least, int n_cu) {
@@ -2672,11 +2690,19 @@ int selective_backward_impl(const E* grad_out, const E* u, const E* dt, const fl
   // few rows: segments with carried adjoints (the 4-states kernel), else one of
   // the kernels with the segments it re-runs
   const int64_t rows64 = batch * ((dim + kWave - 1) / kWave);
-  // (where the 2-states kernel runs its four in one round of the device, five or fewer
-  // carried ones are no faster: 234 -> 248 us at B, D, L = 12, 512, 2048)
   const int n_cu = device_cu_count(call.device());
-  const bool one_round = ml == nullptr && 4 * batch * ((dim + kB2Rows - 1) / kB2Rows) <= int64_t(kBwd2WgPerCu) * n_cu;
-  int n_seg = segment_plan(rows64, length, true, one_round ? 6 : 3, n_cu);
+  // fewest segments that pay against the kernel that re-runs them (segment_plan): three
+  // where that is this one ([B, L, D]); against the 2-states kernel six, but only from
+  // 1024 steps on where two workgroups per compute unit leave no room for nine; and
+  // where that kernel takes more than a round of the device four, if every pass fills
+  // the four waves
+  int least = 3;
+  if (ml == nullptr) {
+    const bool one_round = 4 * batch * ((dim + kB2Rows - 1) / kB2Rows) <= int64_t(kBwd2WgPerCu) * n_cu;
+    const bool pays = one_round ? length >= 1024 || 9 * rows64 <= 2 * n_cu : (dstate + kNpw - 1) / kNpw % kMaxWaves == 0;
+    least = pays ? (one_round ? 6 : 4) : kMaxSegments + 1;
+  }
+  int n_seg = segment_plan(rows64, length, true, least, n_cu);
   bool carried = n_seg > 0, npw2 = false;
   int64_t n_dtiles = 0, dA_rows = 0;
   const int64_t n_bln = batch * length * dstate;
