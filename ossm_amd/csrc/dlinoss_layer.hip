@@ -275,7 +275,6 @@ __device__ __forceinline__ void exact_project(const float* row, const SplitW& g,
   for (int c = 0; c < NC; ++c)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[c][r] = 0.f;
-#pragma unroll 2
   for (int k2 = 0; k2 < K; k2 += 2) {
     const int k = k2 + half;
 #pragma unroll

@@ -21,8 +21,9 @@
 // last-level cache) and writes the states, 64 B per state-step of complex128
 // D-LinOSS against the 48 it cannot do without; the backward 96 against 80.
 // Chunk count and measured figures: chunks64.
-// With one chunk (short sequences, or under stream capture when the
-// workspace would have to grow) step 2 alone is the plain sequential scan.
+// With one chunk (short sequences, channels enough to fill the device, or under
+// stream capture when the workspace would have to grow) step 2 alone is the plain
+// sequential scan.
 //
 // Selective D-LinOSS: recurrence and chain rule of the complex64 kernels
 // (sdlinoss_<v>.cpp forward kernels, backward kernels sdlinoss_imex1.cpp:186-220,
@@ -141,6 +142,17 @@ __device__ __forceinline__ void store_st(double2* p, St s) {
 // pass stores the product of the chunk's transitions).  Time sums: kSums
 // doubles per (chunk, channel), part[(chunk nc + ch) kSums + i].
 
+// Where a scan is cut into chunks (Model::kFwd, kBwd): from `min_len` steps on, and
+// where 2048 waves give each sequence at least `min_chunks`, or `min_chunks_big` once
+// the call moves `big` bytes.  Below, the second launch, the fold and the second
+// read of the inputs cost more than the idle units; the bytes matter because the
+// second read comes from the last-level cache (256 MB) up to there, as do all of a
+// repeated call's.
+struct Chunking {
+  int64_t min_len, min_chunks, big, min_chunks_big;
+};
+constexpr int64_t kMb = 1 << 20;
+
 // Selective D-LinOSS.
 // Where parameter p's gradient goes (mode[p]): 0 = per element at
 // out[t * nc + ch] (full shape); 1 = summed over time; 2 = per element, to be
@@ -154,6 +166,7 @@ template <int V>
 struct Sdl64 {
   static constexpr bool kVarying = true;
   static constexpr int kSums = 3;
+  static constexpr Chunking kFwd{64, 10, 256 * kMb, 5}, kBwd{40, 4, 0, 4}, kBwdConstant{40, 3, 0, 3};
   using Params = Params64;
   using Mat = RMatD;
   using Grads = Grads64;
@@ -262,6 +275,7 @@ struct NoGrads64 {};
 struct Lin64 {
   static constexpr bool kVarying = false;
   static constexpr int kSums = 8;  // grad_m's (re, im) of m11, m12, m21, m22
+  static constexpr Chunking kFwd{100, 10, 256 * kMb, 5}, kBwd{100, 12, 300 * kMb, 8};
   using Params = Lin64Params;
   using Mat = CMatD;
   using Grads = NoGrads64;
@@ -323,6 +337,7 @@ struct Dl64 {
   //   im:    G00, G01, G11, F0 + G10, F1       imex2: G00, G01, G10, G11, F0, F1
   static constexpr int kSums =
       (V == OSSM_DLINOSS_IMEX1 || V == OSSM_DLINOSS_EX) ? 3 : (V == OSSM_DLINOSS_IM ? 5 : 6);
+  static constexpr Chunking kFwd{128, 10, 256 * kMb, 5}, kBwd{100, 8, 300 * kMb, 4};
   using Params = DlParams64;
   using Mat = RMatD;
   using Grads = NoGrads64;
@@ -731,30 +746,39 @@ namespace {
 // of the inputs costs more than the waves hide.  Swept over factors 0.7 to 2.8
 // of sqrt(L) and 2048 to 8192 waves at seven shapes: within 7 % of the best at
 // each.  One lane per sequence against this plan, D-LinOSS imex2 forward /
-// backward, us, [L, B, P]: [256, 2, 64] 22.7 / 65.7 -> 9.4 / 11.7;
-// [2048, 8, 128] 360 / 820 -> 33 / 41 (4.1 TB/s of the backward's 80 B per
-// state-step); [512, 64, 256] 217 / 362 -> 102 / 152; [4096, 32, 128]
-// 1256 / 2584 -> 239 / 328; [16384, 4, 128] 4896 / 10137 -> 128 / 151.  At
-// [4096, 32, 128]: LinOSS 1646 / 4452 -> 335 / 453, selective D-LinOSS with
-// per-step parameters 2022 / 3663 -> 436 / 595.
-int chunks64(int64_t L, int64_t nc) {
-  const int64_t groups = (nc + kWave - 1) / kWave;
-  const int64_t n =
-      std::min<int64_t>(2048 / groups, static_cast<int64_t>(std::sqrt(static_cast<double>(L))));
-  if (n < 2) return 1;
+// backward, us, [L, B, P]: [2048, 8, 128] 360 / 820 -> 31 / 38 (4.4 TB/s of the
+// backward's 80 B per state-step); [512, 64, 256] 217 / 362 -> 104 / 112;
+// [4096, 32, 128] 1256 / 2584 -> 234 / 267; [16384, 4, 128] 4896 / 10137 -> 121 / 130.
+// One chunk -> the plan at the lines drawn, groups of 64 channels (their chunks):
+//   forward, L = 100  1 group      D-LinOSS 10 -> 12  LinOSS 12 -> 12  selective 22 -> 13
+//            L = 300  256 (8)               47 -> 50         113 -> 80          169 -> 111
+//            L = 1500 400 (5)              558 -> 498        703 -> 663         955 -> 941
+//                     512 (4)              561 -> 601        744 -> 806         983 -> 1160
+//                     1024 (2)             967 -> 1120      1281 -> 1534       1402 -> 2234
+//   backward, L = 49  1 group               17 -> 19          15 -> 17           25 -> 21
+//            L = 144  256 (8)               43 -> 41          42 -> 54           97 -> 61
+//            L = 1500 340 (6)              718 -> 463        708 -> 734        1564 -> 1006
+//                     512 (4)              764 -> 683        875 -> 1053       1640 -> 1494
+//                     680 (3)              876 -> 885       1198 -> 1410       1771 -> 1960
+//            (680, parameters constant over time)                             1460 -> 1269
+int chunks64(int64_t L, int64_t nc, const Chunking& c, int64_t bytes) {
+  const int64_t groups = (nc + kWave - 1) / kWave, cap = 2048 / groups;
+  const int64_t n = std::min<int64_t>(cap, static_cast<int64_t>(std::sqrt(static_cast<double>(L))));
+  if (n < 2 || L < c.min_len || cap < (bytes >= c.big ? c.min_chunks_big : c.min_chunks)) return 1;
   const int64_t cl = (L + n - 1) / n;
   return static_cast<int>((L + cl - 1) / cl);
 }
 
-// The chunk plan and the workspace it lives in: `sums(n_chunks)` doubles for
-// the caller's partial sums, then the aggregates and (varying) the transition
+// The chunk plan of a call that moves `bytes` bytes and the workspace it lives in:
+// `sums(n_chunks)` doubles for the caller's partial sums, then the aggregates and (varying) the transition
 // products.  When the workspace cannot be had (under stream capture it may not
 // grow; a full device) the call runs as one chunk, which needs only the sums.
 template <class Sums>
-int plan64(StreamCall& call, int64_t L, int64_t nc, bool varying, Sums sums, Plan64* pl, double** part) {
+int plan64(StreamCall& call, int64_t L, int64_t nc, bool varying, const Chunking& cut, int64_t bytes, Sums sums,
+           Plan64* pl, double** part) {
   // a captured call without sums takes no workspace, so that its graph may replay
   // beside the capture stream's own work
-  int n = call.capturing() && sums(1) == 0 ? 1 : chunks64(L, nc);
+  int n = call.capturing() && sums(1) == 0 ? 1 : chunks64(L, nc, cut, bytes);
   for (;;) {
     const size_t rows = n > 1 ? static_cast<size_t>(n) * nc : 0;
     const size_t n_sums = (sums(n) + 1) & ~size_t(1);  // 16-byte aligned double2 behind them
@@ -781,14 +805,17 @@ int plan64(StreamCall& call, int64_t L, int64_t nc, bool varying, Sums sums, Pla
   }
 }
 
+// step_bytes: read and written per state-step, once each
 template <class M>
 int run_forward64(const typename M::Params& prm, const void* in, void* states, int64_t L, int64_t nc,
-                  hipStream_t stream) {
+                  int64_t step_bytes, hipStream_t stream) {
   StreamCall call(stream);
   if (call.status()) return call.status();
   Plan64 pl{};
   double* part = nullptr;
-  if (int rc = plan64(call, L, nc, M::kVarying, [](int) { return size_t(0); }, &pl, &part)) return rc;
+  if (int rc = plan64(call, L, nc, M::kVarying, M::kFwd, L * nc * step_bytes, [](int) { return size_t(0); }, &pl,
+                      &part))
+    return rc;
   const unsigned groups = static_cast<unsigned>((nc + kWave - 1) / kWave);
   const auto* src = static_cast<const double2*>(in);
   if (pl.n_chunks > 1) {
@@ -848,16 +875,18 @@ int ossm_sdlinoss_forward_f64(int variant, const double* A, int64_t a_len, int64
   if (int rc = check64(variant, shapes, length, batch, ssm, "sdlinoss_forward_f64")) return rc;
   if (!bu || !states) return set_error(OSSM_ERR_INVALID_ARGUMENT, "sdlinoss_forward_f64: null pointer");
   const Params64 prm = params64(shapes, length, batch, ssm);
+  int64_t step_bytes = 48;  // bu and the states, and each parameter that is full size
+  for (const Shape64& s : shapes) step_bytes += s.la == length && s.ba == batch ? 8 : 0;
   hipStream_t stream = static_cast<hipStream_t>(stream_v);
   switch (variant) {
     case OSSM_DLINOSS_IMEX1:
-      return run_forward64<Sdl64<OSSM_DLINOSS_IMEX1>>(prm, bu, states, length, batch * ssm, stream);
+      return run_forward64<Sdl64<OSSM_DLINOSS_IMEX1>>(prm, bu, states, length, batch * ssm, step_bytes, stream);
     case OSSM_DLINOSS_IMEX2:
-      return run_forward64<Sdl64<OSSM_DLINOSS_IMEX2>>(prm, bu, states, length, batch * ssm, stream);
+      return run_forward64<Sdl64<OSSM_DLINOSS_IMEX2>>(prm, bu, states, length, batch * ssm, step_bytes, stream);
     case OSSM_DLINOSS_IM:
-      return run_forward64<Sdl64<OSSM_DLINOSS_IM>>(prm, bu, states, length, batch * ssm, stream);
+      return run_forward64<Sdl64<OSSM_DLINOSS_IM>>(prm, bu, states, length, batch * ssm, step_bytes, stream);
     default:
-      return run_forward64<Sdl64<OSSM_DLINOSS_EX>>(prm, bu, states, length, batch * ssm, stream);
+      return run_forward64<Sdl64<OSSM_DLINOSS_EX>>(prm, bu, states, length, batch * ssm, step_bytes, stream);
   }
 }
 
@@ -910,7 +939,9 @@ int ossm_sdlinoss_backward_f64(int variant, const double* A, int64_t a_len, int6
   };
   Plan64 pl{};
   double* ws = nullptr;
-  if (int rc = plan64(call, length, nc, true,
+  using Any = Sdl64<OSSM_DLINOSS_IMEX1>;
+  const bool constant = rt[0] && rt[1] && rt[2];  // over time: no gradient per step
+  if (int rc = plan64(call, length, nc, true, constant ? Any::kBwdConstant : Any::kBwd, 0,
                       [&](int n) { return rows_of(0, n) + rows_of(1, n) + rows_of(2, n); }, &pl, &ws))
     return rc;
   for (int p = 0; p < 3; ++p) {
@@ -959,7 +990,7 @@ int ossm_linoss_forward_f64(const void* m11, const void* m12, const void* m21, c
   const Lin64Params mp{{static_cast<const double2*>(m11), static_cast<const double2*>(m12),
                         static_cast<const double2*>(m21), static_cast<const double2*>(m22)},
                        static_cast<int>(ssm)};
-  return run_forward64<Lin64>(mp, b_seq, states, length, batch * ssm, static_cast<hipStream_t>(stream_v));
+  return run_forward64<Lin64>(mp, b_seq, states, length, batch * ssm, 64, static_cast<hipStream_t>(stream_v));
 }
 
 int ossm_linoss_backward_f64(const void* m11, const void* m12, const void* m21, const void* m22,
@@ -992,7 +1023,7 @@ int ossm_linoss_backward_f64(const void* m11, const void* m12, const void* m21, 
   const int64_t nc = batch * ssm;
   Plan64 pl{};
   double* part = nullptr;
-  if (int rc = plan64(call, length, nc, false,
+  if (int rc = plan64(call, length, nc, false, Lin64::kBwd, length * nc * 96,
                       [&](int n) { return static_cast<size_t>(n) * nc * Lin64::kSums; }, &pl, &part))
     return rc;
   if (int rc = run_backward64<Lin64>(mp, nullptr, states, grad_output, grad_b, NoGrads64{}, part, pl, stream))
@@ -1018,10 +1049,10 @@ int ossm_dlinoss_forward_f64(int variant, const double* a_diag, const double* g_
   const int64_t nc = batch * ssm;
   hipStream_t stream = static_cast<hipStream_t>(stream_v);
   switch (variant) {
-    case OSSM_DLINOSS_IMEX1: return run_forward64<Dl64<OSSM_DLINOSS_IMEX1>>(prm, bu, states, length, nc, stream);
-    case OSSM_DLINOSS_IMEX2: return run_forward64<Dl64<OSSM_DLINOSS_IMEX2>>(prm, bu, states, length, nc, stream);
-    case OSSM_DLINOSS_IM: return run_forward64<Dl64<OSSM_DLINOSS_IM>>(prm, bu, states, length, nc, stream);
-    default: return run_forward64<Dl64<OSSM_DLINOSS_EX>>(prm, bu, states, length, nc, stream);
+    case OSSM_DLINOSS_IMEX1: return run_forward64<Dl64<OSSM_DLINOSS_IMEX1>>(prm, bu, states, length, nc, 48, stream);
+    case OSSM_DLINOSS_IMEX2: return run_forward64<Dl64<OSSM_DLINOSS_IMEX2>>(prm, bu, states, length, nc, 48, stream);
+    case OSSM_DLINOSS_IM: return run_forward64<Dl64<OSSM_DLINOSS_IM>>(prm, bu, states, length, nc, 48, stream);
+    default: return run_forward64<Dl64<OSSM_DLINOSS_EX>>(prm, bu, states, length, nc, 48, stream);
   }
 }
 
@@ -1059,8 +1090,8 @@ int ossm_dlinoss_backward_f64(int variant, const double* a_diag, const double* g
   const int64_t nc = batch * ssm;
   Plan64 pl{};
   double* part = nullptr;
-  if (int rc = plan64(call, length, nc, false, [&](int n) { return static_cast<size_t>(n) * nc * 6; }, &pl,
-                      &part))
+  if (int rc = plan64(call, length, nc, false, Dl64<OSSM_DLINOSS_IMEX1>::kBwd, length * nc * 80,
+                      [&](int n) { return static_cast<size_t>(n) * nc * 6; }, &pl, &part))
     return rc;
   const int64_t rows = int64_t(pl.n_chunks) * batch;  // of P oscillators' sums each
   if (rows > INT_MAX) return set_error(OSSM_ERR_UNSUPPORTED, "dlinoss_backward_f64: size exceeds 32-bit indexing");

@@ -183,6 +183,14 @@ def test_complex128_scans_chunk_edges(K, shape):
         np.testing.assert_allclose(to_np(got), r, rtol=1e-10, atol=1e-12 * max(1.0, float(np.abs(r).max())))
 
 
+# the fewest steps that are cut into chunks, a short last chunk, and the fewest chunks
+# (2048 waves shared by the channels) of each scan and direction
+@pytest.mark.parametrize("shape", [(99, 1, 1), (100, 2, 5), (127, 1, 3), (128, 1, 70), (131, 3, 43), (128, 4, 3264),
+                                   (150, 4, 4096)], ids=lambda s: "x".join(map(str, s)))
+def test_complex128_scans_cut_into_chunks(K, shape):
+    test_complex128_scans_chunk_edges(K, shape)
+
+
 def _unstable_inputs(rng, L):
     """Four channels of an L-step scan whose transition grows about 1e6 times a step
     (so that a chunk's power of it overflows), but for the second, a stable one:

@@ -275,6 +275,14 @@ def test_sdlinoss_complex128_chunk_edges(K, shape, tag):
         assert_close(to_np(got), ref, RTOL64, ATOL64 * max(1.0, float(np.abs(ref).max())), name)
 
 
+@pytest.mark.parametrize("tag", ["full", "bcast_t", "bcast_b", "m", "lm", "bm"])
+@pytest.mark.parametrize("shape", [(39, 2, 3), (40, 1, 1), (63, 3, 43), (64, 2, 65), (75, 1, 5)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_sdlinoss_complex128_cut_into_chunks(K, shape, tag):
+    """The fewest steps that are cut into chunks, and short last chunks."""
+    test_sdlinoss_complex128_chunk_edges(K, shape, tag)
+
+
 @pytest.mark.parametrize("tag", ["m", "full"])
 @pytest.mark.parametrize("variant", VARIANTS)
 def test_sdlinoss_complex128_chunks_keep_zeros_and_infinities(K, variant, tag):
