@@ -77,12 +77,15 @@ class LayerParamsFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, damped: bool, A_diag: Tensor, G_diag: Optional[Tensor],
                 steps: Tensor):  # type: ignore[override]
-        params = (A_diag, G_diag, steps) if damped else (A_diag, steps)
-        if any(t is None or t.dim() != 1 or t.shape != A_diag.shape for t in params):
-            raise RuntimeError("oscillator parameters must be vectors of one length, got "
-                               f"{[t if t is None else tuple(t.shape) for t in params]}")
-        if any(t.dtype != torch.float32 or not t.is_cuda or t.device != A_diag.device for t in params):
-            raise RuntimeError("oscillator parameters must be float32 GPU tensors, on one device")
+        shape, index = A_diag.shape, A_diag.get_device()
+        rest = (G_diag, steps) if damped else (steps,)
+        for t in rest:
+            if t is None or len(shape) != 1 or t.shape != shape:
+                raise RuntimeError("oscillator parameters must be vectors of one length, got "
+                                   f"{[x if x is None else tuple(x.shape) for x in (A_diag, *rest)]}")
+        for t in (A_diag, *rest):
+            if t.dtype is not torch.float32 or index < 0 or t.get_device() != index:
+                raise RuntimeError("oscillator parameters must be float32 GPU tensors, on one device")
         A, G, s = (None if t is None else t.contiguous() for t in (A_diag, G_diag, steps))
         out = torch.empty((6, A.numel()), dtype=torch.float32, device=A.device)
         _lib.run(_lib.load().ossm_layer_params_forward, A, int(damped), A.data_ptr(), _lib.ptr(G),
@@ -130,9 +133,9 @@ def fused_layer_supported(inputs: Tensor, params, hidden: int, ssm: int) -> bool
     empty, nothing that broadcasts."""
     return (inputs.is_cuda and inputs.dtype == torch.float32 and inputs.numel() > 0 and ssm > 0
             and _layer_sizes_fit(inputs.size(0), inputs.size(1), hidden, ssm)
-            and all(t.dtype == torch.float32 and t.device == inputs.device for t in params)
-            and all(t.shape == want for t, want in
-                    zip(params, ((ssm,), (ssm, hidden, 2), (hidden, ssm, 2), (hidden,), (ssm,))))
+            and all(t.dtype is torch.float32 and t.device == inputs.device for t in params)
+            and params[0].shape == params[4].shape == (ssm,) and params[3].shape == (hidden,)
+            and params[1].shape == (ssm, hidden, 2) and params[2].shape == (hidden, ssm, 2)
             and not torch.is_autocast_enabled("cuda"))
 
 
@@ -144,21 +147,26 @@ def _check_layer_args(inputs: Tensor, B: Tensor, C: Tensor, D: Tensor, a: Tensor
     if B.dim() != 3 or B.size(1) != hidden or B.size(2) != 2:
         raise RuntimeError(f"B must have shape (ssm_size, {hidden}, 2), got {tuple(B.shape)}")
     ssm = B.size(0)
-    if tuple(C.shape) != (hidden, ssm, 2):
+    if C.shape != (hidden, ssm, 2):
         raise RuntimeError(f"C must have shape ({hidden}, {ssm}, 2), got {tuple(C.shape)}")
-    if tuple(D.shape) != (hidden,):
+    if D.shape != (hidden,):
         raise RuntimeError(f"D must have shape ({hidden},), got {tuple(D.shape)}")
     for name, t in (("a_diag", a), ("g_diag", g), ("step", step)):
-        if tuple(t.shape) != (ssm,):
+        if t.shape != (ssm,):
             raise RuntimeError(f"{name} must have shape ({ssm},), got {tuple(t.shape)}")
     return batch, length, hidden, ssm
 
 
 def _check_on_gpu(tensors, hidden: int, ssm: int) -> None:
-    if any(t.dtype != torch.float32 for t in tensors):
-        raise RuntimeError("the fused D-LinOSS layer computes in float32; got "
-                           + ", ".join(str(t.dtype) for t in tensors))
-    if not all(t.is_cuda for t in tensors) or len({t.device for t in tensors}) != 1:
+    index = tensors[0].get_device()
+    one = index >= 0
+    for t in tensors:
+        if t.dtype is not torch.float32:
+            raise RuntimeError("the fused D-LinOSS layer computes in float32; got "
+                               + ", ".join(str(x.dtype) for x in tensors))
+        if t.get_device() != index:
+            one = False
+    if not one:
         raise RuntimeError("the fused D-LinOSS layer needs every tensor on one GPU")
     if hidden > _LAYER_MAX or ssm > _LAYER_MAX:
         raise RuntimeError(f"the fused D-LinOSS layer supports hidden_dim and ssm_size up to "
@@ -422,7 +430,7 @@ class DampedLinOSSLayer(nn.Module):
                   (self.A_diag, self.G_diag, self.steps, self.B, self.C, self.D)]
         Bw, Cw, Dw = params[3:]
         if u.is_cuda and self.hidden_dim <= _LAYER_MAX and self.ssm_size <= _LAYER_MAX:
-            if all(t.shape == (self.ssm_size,) for t in params[:3]):
+            if params[0].shape == params[1].shape == params[2].shape == (self.ssm_size,):
                 a, g, dt, _ = LayerParamsFn.apply(True, *params[:3])
             else:  # replaced parameters may broadcast
                 a, g, dt = project_parameters(*params[:3])

@@ -265,9 +265,10 @@ class MixerCoreFn(torch.autograd.Function):
                 not _core_shapes(*dt_w.shape, A_log.size(1), xz, *params):
             raise RuntimeError("mixer: inconsistent shapes xz, conv weight, conv bias, x_proj, dt_proj, dt bias, "
                                f"A_log: {[t if t is None else tuple(t.shape) for t in (xz, *params)]}")
-        if not xz.is_cuda or any(t is not None and (t.dtype != torch.float32 or t.device != xz.device)
-                                 for t in (xz, *params)):
-            raise RuntimeError("mixer: every tensor must be a float32 GPU tensor, on one device")
+        index = xz.get_device()
+        for t in (xz, *params):
+            if t is not None and (t.dtype is not torch.float32 or index < 0 or t.get_device() != index):
+                raise RuntimeError("mixer: every tensor must be a float32 GPU tensor, on one device")
         Di, R, N = dt_w.size(0), dt_w.size(1), A_log.size(1)
         lib = _lib.load()
         given, xz = xz, xz.contiguous()
@@ -390,9 +391,9 @@ class MambaMixer(nn.Module):
         xz = linear(self.in_proj, inputs).float()
         params = (self.conv1d.weight, self.conv1d.bias, self.x_proj.weight, self.dt_proj.weight,
                   self.dt_proj.bias, self.A_log)
-        # other shapes (replaced parameters) take the separate steps, which refuse what does not fit
-        if is_plain(self.x_proj) and self.x_proj.bias is None and xz.numel() > 0 \
-                and _all_float(xz, params) and _core_shapes(Di, R, N, xz, *params):
+        # replaced parameters that do not have the mixer's sizes take the separate steps
+        if is_plain(self.x_proj) and self.x_proj.bias is None and xz.numel() > 0 and _all_float(xz, params) \
+                and params[3].shape == (Di, R) and params[5].shape == (Di, N) and params[0].size(0) == Di:
             y = MixerCoreFn.apply(xz, *params)
             return linear(self.out_proj, y.to(self.out_proj.weight.dtype))
         x, z = _ColumnSplit.apply(xz, Di)                 # views, row stride 2 * d_inner
