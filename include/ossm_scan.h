@@ -34,8 +34,8 @@
  * before enqueuing anything (run it once eagerly on the stream first), as
  * does OSSM_SCAN_ORDER=dispatch (host-chosen tags for every launch).
  * Buffers a graph captured are never freed.  Replays use the capture
- * stream's scratch: replay the graph on that stream, or ordered with
- * everything else that uses it.
+ * stream's scratch and workspace: replay the graph on that stream, or
+ * ordered with everything else there that calls the library.
  */
 #ifndef OSSM_SCAN_H
 #define OSSM_SCAN_H

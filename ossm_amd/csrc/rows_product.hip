@@ -13,11 +13,11 @@
 // (bitwise repeatable).
 //
 // Bound: the matrix cores and the splitting together, 48 instructions of 32
-// cycles and 264 VALU per 16 rows and tile (two waves per SIMD of just these,
-// without loads: 1.45 PFLOP/s of bf16; this kernel 0.9 at [131072, 256, 128], its
-// loads one block ahead).  Against the library's fp32 GEMM on the same operands, us
+// cycles and 264 VALU per 16 rows and tile (0.9 PFLOP/s of bf16 at [131072, 256, 128],
+// loads one block ahead; an 8192^3 bf16 product of the library reaches 1.2).  Against
+// the library's fp32 GEMM on the same operands, us
 // (and its relative error against float64): [51200, 256, 64] 164 -> 24
-// (2.5e-6 -> 2.8e-7); [51200, 128, 4] 71 -> 18; [131072, 256, 128] 345 -> 59
+// (2.5e-6 -> 2.8e-7); [51200, 128, 4] 71 -> 18; [131072, 256, 128] 345 -> 58
 // (4e-6 -> 4.3e-7; as 32 batched slices 75, 1.1e-6); [32768, 3072, 768]
 // 2388 -> 1340; [1000, 256, 64] 60 -> 14.
 

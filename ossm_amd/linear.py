@@ -19,9 +19,13 @@ from . import _lib
 __all__ = ["rows_product", "linear", "linear_weight", "LinearFn", "is_plain",
            "MIN_ROWS", "BLOCK_ROWS"]
 
-BLOCK_ROWS = 16  # the least the kernel takes
-# LinearFn with fewer rows leaves the weight gradient to the library's GEMM: 200 rows
-# 9 us against 12, 1000 rows 60 against 14 ([R, 80] x [R, 40] and [R, 256] x [R, 64]).
+# The least the kernel takes, and where the layers' and the mixer's own backwards, which
+# have no operation of torch's to fall back on but transposed products and copies, take
+# it: training steps of [rows, 64] at 16 to 400 rows, LinOSS layer 162 us against 196 to
+# 292 with those, mixer 519 against 526 to 528.
+BLOCK_ROWS = 16
+# LinearFn leaves fewer rows to torch: the weight gradient alone then takes 9 us against
+# 12 at 200 rows, 60 against 14 at 1000 ([R, 80] x [R, 40] and [R, 256] x [R, 64]).
 MIN_ROWS = 512
 
 
